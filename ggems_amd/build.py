@@ -59,8 +59,15 @@ def build_host():
 
 
 def extract_data():
+    """The physics blob, or None where there is neither a GGEMS source tree nor a
+    blob of an earlier build: the libraries do not need it to build, and the
+    engine ABI (whose caller brings the tables) does not need it to run."""
     sys.path.insert(0, os.path.join(HERE, "data"))
     import extract_physics_data
+    if not extract_physics_data.available():
+        print("no GGEMS source tree (GGEMS_SOURCE_DIR): building without the physics data, which GGEMS's material "
+              "and cross-section classes read", file=sys.stderr)
+        return None
     return extract_physics_data.main()
 
 

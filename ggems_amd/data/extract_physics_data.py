@@ -155,9 +155,22 @@ def write_blob(arrays, path):
     os.replace(tmp, path)
 
 
+def _root(ggems_root=None):
+    return ggems_root or os.environ.get("GGEMS_SOURCE_DIR", "/root/reference")
+
+
+def _is_tree(root):
+    return os.path.isdir(os.path.join(root, "include", "GGEMS"))
+
+
+def available(ggems_root=None):
+    """whether main() can give a blob: a source tree to read, or the blob of an earlier build"""
+    return _is_tree(_root(ggems_root)) or os.path.exists(BLOB)
+
+
 def main(ggems_root=None):
-    ggems_root = ggems_root or os.environ.get("GGEMS_SOURCE_DIR", "/root/reference")
-    if not os.path.isdir(os.path.join(ggems_root, "include", "GGEMS")):
+    ggems_root = _root(ggems_root)
+    if not _is_tree(ggems_root):
         if os.path.exists(BLOB):
             print("GGEMS source tree not found; keeping existing", BLOB)
             return BLOB
