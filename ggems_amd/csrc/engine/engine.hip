@@ -1464,32 +1464,52 @@ __global__ __launch_bounds__(kDoseBlock) void dose_kernel(DoseParams D) {
 // ---------------------------------------------------------------------------
 // ray-traced primary transmission (DRR)
 // ---------------------------------------------------------------------------
-// One thread per detector pixel: the segment from the focal point to the
-// pixel centre crosses every voxel solid; the exact length inside each
-// voxel (a 3D DDA in FP64) is added to the voxel's global material in LDS.
-// The transmission is then sum_b w_b exp(-sum_m sigma_tot(m, b) L_m) over
-// the energy bins b the source spectrum reaches, sigma_tot being the
-// left-bin total of the activated processes the transport uses for its
-// distances (GGEMSPhotonNavigator.hh:57-93).
-constexpr int kDrrBlock = 128;
+// kDrrSegs threads per detector pixel: the segment from the focal point to
+// the pixel centre crosses every voxel solid, and each thread walks its
+// eighth of the way through it (a 3D DDA in FP64).  The exact length inside
+// each material goes to LDS, where the pixel's threads sum their parts; they
+// then share the energy bins b the source spectrum reaches and sum
+// w_b exp(-sum_m sigma_tot(m, b) L_m), sigma_tot being the left-bin total of
+// the activated processes the transport uses for its distances
+// (GGEMSPhotonNavigator.hh:57-93).
+//
+// One thread per pixel was bound by the chain of its steps: each waited for
+// the label it had just addressed, and 32 materials' sums per thread left
+// room for 10 waves on a compute unit.  The walk does not depend on the
+// labels, so kDrrBatch steps are made ahead and their labels requested
+// together; lengths are summed over runs of one material; and eight threads
+// share the chain.  A block holds 8 x 4 pixels, whose rays read the same
+// label bricks at a time.  What bounds it now is the FP64 issue of the walk.
+// A 512 x 384 panel behind 512 x 512 x 256 voxels: 800 us before, 229 us; a
+// 256 x 256 panel behind 96 x 96 x 64 voxels: 88 us before, 33 us, and the
+// spectrum table that a second kernel made for each such image (46 us) is now
+// made once, with the source.
+constexpr int kDrrSegs = 8, kDrrTileX = 8, kDrrTileY = 4, kDrrTile = kDrrTileX * kDrrTileY;
+constexpr int kDrrBlock = kDrrSegs * kDrrTile;
+constexpr int kDrrBatch = 8;
 constexpr int kDrrMaxMat = 32;
+constexpr int kNoAllocMaxBins = 1024;  // ggh_drr_noalloc's documented limit
 
 struct DrrParams {
   const DevSolid* solids;
   int32_t n_solids;
   int32_t box;
   Mat34 src_m, box_m;
-  const float4* sig;
-  int32_t nbins, n_mat;
-  const int32_t* w_bin;
+  int32_t n_mat;
+  // the spectrum's bins of nonzero weight: their weights, and sigma_tot [bin][material]
   const float* w;
+  const double* mu;
   int32_t n_w;
-  const uint32_t* n_w_dev;  // weight count on the device (the allocation-free entry point), else null
   int32_t only;  // the one voxel solid present (an acquisition projection over several phantoms), or -1
   float* image;
 };
 
-__device__ void drr_voxel_solid(const DevSolid& s, f3 gs, f3 ge, double* L) {
+// dynamic LDS of a block: a length per material and thread, a partial transmission per thread
+size_t drr_lds_bytes(int n_mat) { return (size_t)(n_mat + 1) * kDrrBlock * sizeof(double); }
+
+// this thread's part `seg` of the way from gs to ge through a voxel solid;
+// L[m * kDrrBlock] += the length inside global material m
+__device__ void drr_voxel_solid(const DevSolid& s, f3 gs, f3 ge, int seg, double* L) {
   const VoxGeom& G = s.vox;
   const f3 ls = g2l_pos(s.m, gs), le = g2l_pos(s.m, ge);
   const double o[3] = {ls.x, ls.y, ls.z};
@@ -1498,150 +1518,121 @@ __device__ void drr_voxel_solid(const DevSolid& s, f3 gs, f3 ge, double* L) {
   const double hi[3] = {s.border.hi.x, s.border.hi.y, s.border.hi.z};
   const double vs[3] = {G.vs.x, G.vs.y, G.vs.z};
   const int n[3] = {G.nx, G.ny, G.nz};
+  double rd[3];  // one division an axis: a quotient each for its planes took most of a short walk's time
   double t0 = 0.0, t1 = 1.0;
   for (int a = 0; a < 3; ++a) {
+    rd[a] = 1.0 / d[a];
     if (fabs(d[a]) < 1e-300) {
       if (o[a] < lo[a] || o[a] > hi[a]) return;
     } else {
-      const double ta = (lo[a] - o[a]) / d[a], tb = (hi[a] - o[a]) / d[a];
+      const double ta = (lo[a] - o[a]) * rd[a], tb = (hi[a] - o[a]) * rd[a];
       t0 = fmax(t0, fmin(ta, tb));
       t1 = fmin(t1, fmax(ta, tb));
     }
   }
   if (!(t0 < t1)) return;
   const double len = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+  // the same expression for a part's end and the next one's start
+  const double part = (t1 - t0) * (1.0 / kDrrSegs);
+  const double ta = t0 + part * seg, tb = seg + 1 == kDrrSegs ? t1 : t0 + part * (seg + 1);
+  if (!(ta < tb)) return;
   int i[3], step[3];
   double tmax[3], tdel[3];
-  const double tm = 0.5 * (t0 + fmin(t1, t0 + 1e-9));
+  const double tm = ta + 0.5 * fmin(tb - ta, 1e-9);
   for (int a = 0; a < 3; ++a) {
     const double p = o[a] + d[a] * tm;
     int k = (int)floor((p - lo[a]) / vs[a]);
     i[a] = k < 0 ? 0 : (k >= n[a] ? n[a] - 1 : k);
-    if (d[a] > 0.0) {
-      step[a] = 1;
-      tmax[a] = (lo[a] + (i[a] + 1) * vs[a] - o[a]) / d[a];
-      tdel[a] = vs[a] / d[a];
-    } else if (d[a] < 0.0) {
-      step[a] = -1;
-      tmax[a] = (lo[a] + i[a] * vs[a] - o[a]) / d[a];
-      tdel[a] = -vs[a] / d[a];
-    } else {
-      step[a] = 0;
-      tmax[a] = INFINITY;
-      tdel[a] = INFINITY;
-    }
+    const bool along = fabs(d[a]) >= 1e-300;
+    step[a] = !along ? 0 : (d[a] > 0.0 ? 1 : -1);
+    tmax[a] = along ? (lo[a] + (i[a] + (d[a] > 0.0 ? 1 : 0)) * vs[a] - o[a]) * rd[a] : INFINITY;
+    tdel[a] = along ? vs[a] * fabs(rd[a]) : 0.0;
   }
-  double t = t0;
+  double t = ta;       // end of the last step made
+  double from = ta;    // start of the run of material `cur`, summed up to `upto`
+  double upto = ta;
+  int cur = -1;
+  bool more = true;
   const int max_iter = n[0] + n[1] + n[2] + 3;
-  for (int it = 0; it < max_iter; ++it) {
-    const int a = tmax[0] < tmax[1] ? (tmax[0] < tmax[2] ? 0 : 2) : (tmax[1] < tmax[2] ? 1 : 2);
-    const double tn = fmin(tmax[a], t1);
-    if (tn > t) {
-      const int gm = G.mat_offset + G.labels[i[0] + i[1] * G.nx + i[2] * G.nxy];
-      L[gm] += (tn - t) * len;
+  for (int it = 0; it < max_iter && more; it += kDrrBatch) {
+    uint32_t off[kDrrBatch];
+    double end[kDrrBatch];
+#pragma unroll
+    for (int b = 0; b < kDrrBatch; ++b) {
+      // a finished walk repeats its last voxel with no length
+      off[b] = brick_offset(G.nbx, G.nbxy, i[0], i[1], i[2]);
+      const bool x = (tmax[0] < tmax[1]) & (tmax[0] < tmax[2]);
+      const bool y = !x & (tmax[1] < tmax[2]);
+      const bool z = !x & !y;
+      const double tn = x ? tmax[0] : (y ? tmax[1] : tmax[2]);
+      t = more ? fmax(t, fmin(tn, tb)) : t;
+      end[b] = t;
+      const int j0 = i[0] + (x ? step[0] : 0), j1 = i[1] + (y ? step[1] : 0), j2 = i[2] + (z ? step[2] : 0);
+      more &= (tn < tb) & ((uint32_t)j0 < (uint32_t)n[0]) & ((uint32_t)j1 < (uint32_t)n[1]) &
+              ((uint32_t)j2 < (uint32_t)n[2]);
+      i[0] = more ? j0 : i[0];
+      i[1] = more ? j1 : i[1];
+      i[2] = more ? j2 : i[2];
+      tmax[0] += x ? tdel[0] : 0.0;
+      tmax[1] += y ? tdel[1] : 0.0;
+      tmax[2] += z ? tdel[2] : 0.0;
     }
-    if (tn >= t1) break;
-    t = tn;
-    i[a] += step[a];
-    if (i[a] < 0 || i[a] >= n[a]) break;
-    tmax[a] += tdel[a];
+    int label[kDrrBatch];
+#pragma unroll
+    for (int b = 0; b < kDrrBatch; ++b) label[b] = G.bricks[off[b]];
+#pragma unroll
+    for (int b = 0; b < kDrrBatch; ++b) {
+      if (label[b] != cur) {
+        if (cur >= 0) L[(G.mat_offset + cur) * kDrrBlock] += (upto - from) * len;
+        cur = label[b];
+        from = upto;
+      }
+      upto = end[b];
+    }
   }
+  if (cur >= 0) L[(G.mat_offset + cur) * kDrrBlock] += (upto - from) * len;
 }
 
 __global__ __launch_bounds__(kDrrBlock) void drr_kernel(DrrParams D) {
-  __shared__ double sL[kDrrBlock * kDrrMaxMat];
-  double* L = sL + threadIdx.x * kDrrMaxMat;
-  for (int m = 0; m < kDrrMaxMat; ++m) L[m] = 0.0;
+  extern __shared__ double s_len[];  // [n_mat][kDrrBlock], then [kDrrBlock] partial transmissions
+  const int tid = threadIdx.x, pixel = tid % kDrrTile, seg = tid / kDrrTile;
+  double* L = s_len + tid;
+  for (int m = 0; m < D.n_mat; ++m) L[m * kDrrBlock] = 0.0;
   const DevSolid& box = D.solids[D.box];
-  const int npx = box.ne[0] * box.ne[1];
-  const int px = blockIdx.x * kDrrBlock + threadIdx.x;
-  if (px >= npx) return;
-  const int ix = px % box.ne[0], iy = px / box.ne[0];
-  const float esx = box.box_size.x / (float)box.ne[0], esy = box.box_size.y / (float)box.ne[1];
-  const f3 pc = mk(box.border.lo.x + ((float)ix + 0.5f) * esx, box.border.lo.y + ((float)iy + 0.5f) * esy,
-                   0.5f * (box.border.lo.z + box.border.hi.z));
-  const f3 ge = l2g_pos(D.box_m, pc);
-  const f3 gs = l2g_pos(D.src_m, mk(0.0f, 0.0f, 0.0f));
-  for (int k = 0; k < D.n_solids; ++k)
-    if (D.solids[k].type == kVoxel && (D.only < 0 || k == D.only)) drr_voxel_solid(D.solids[k], gs, ge, L);
-  double t = 0.0;
-  const int n_w = D.n_w_dev ? (int)*D.n_w_dev : D.n_w;
-  for (int j = 0; j < n_w; ++j) {
-    const int b = D.w_bin[j];
-    double mu = 0.0;
-    for (int m = 0; m < D.n_mat; ++m) {
-      const float4 sg = D.sig[m * D.nbins + b];
-      mu += ((double)sg.x + (double)sg.y + (double)sg.z) * L[m];
-    }
-    t += (double)D.w[j] * exp(-mu);
-  }
-  D.image[px] = (float)t;
-}
-
-// ---------------------------------------------------------------------------
-// the ray tracer without allocations (ggh_drr_noalloc): the spectrum weights
-// are built on the device into a file-scope staging array instead of buffers
-// allocated per call.  Layout in 32-bit words: [0] the weight count, [64 ..
-// 64 + kNoAllocMaxBins) the energy bins, then the FP32 weights.  Every call
-// on one GPU shares the array.
-// ---------------------------------------------------------------------------
-constexpr int kNoAllocMaxBins = 1024;
-constexpr int kScratchBins = 64, kScratchWeights = kScratchBins + kNoAllocMaxBins;
-constexpr int kScratchWords = kScratchWeights + kNoAllocMaxBins;
-static __device__ __align__(256) uint32_t scratch[kScratchWords];
-
-// BinarySearch over the whole energy grid (GGEMSMathAlgorithms.hh:46-60)
-__device__ inline int grid_bin(const float* a, int size, float key) {
-  int low = 0, high = size - 1;
-  while (high - low > 1) {
-    const int mid = (high + low) / 2;
-    if (a[mid] == key) return mid;
-    if (a[mid] < key) low = mid;
-    else high = mid;
-  }
-  return low;
-}
-
-// The probability w_b of each energy bin under the source's sampling, as the
-// host builds it for ggh_drr: thread k sums bin k's share of every spectrum
-// interval in interval order (the host's order of additions, so the FP64
-// sums are identical), then one lane keeps the bins with weight, in order.
-constexpr int kWeightsBlock = 256;
-__global__ __launch_bounds__(kWeightsBlock) void drr_weights_kernel(const float* eb, int nb, const float* e, int n_e,
-                                                                   const float* f, int n_f, int is_interp,
-                                                                   uint32_t* stage) {
-  __shared__ double W[kNoAllocMaxBins];
-  for (int k = threadIdx.x; k < nb; k += kWeightsBlock) {
-    double acc = 0.0;
-    for (int idx = 0; idx + 1 < n_f && idx + 1 < n_e; ++idx) {
-      const double p = (double)f[idx + 1] - (double)f[idx];
-      if (!(p > 0.0)) continue;
-      const double a = e[idx], b = e[idx + 1];
-      if (!is_interp || !(b > a)) {
-        if (grid_bin(eb, nb, e[idx]) == k) acc += p;
-        continue;
-      }
-      if (k + 1 < nb) {
-        const double lo = k == 0 ? -INFINITY : (double)eb[k];
-        const double hi = k + 2 == nb ? INFINITY : (double)eb[k + 1];
-        const double ov = (hi < b ? hi : b) - (a < lo ? lo : a);  // std::min(b, hi) - std::max(a, lo)
-        if (ov > 0.0) acc += p * ov / (b - a);
-      }
-    }
-    W[k] = acc;
+  const int tiles_x = (box.ne[0] + kDrrTileX - 1) / kDrrTileX;
+  const int ix = (int)(blockIdx.x % tiles_x) * kDrrTileX + pixel % kDrrTileX;
+  const int iy = (int)(blockIdx.x / tiles_x) * kDrrTileY + pixel / kDrrTileX;
+  const bool inside = ix < box.ne[0] && iy < box.ne[1];
+  if (inside) {
+    const float esx = box.box_size.x / (float)box.ne[0], esy = box.box_size.y / (float)box.ne[1];
+    const f3 pc = mk(box.border.lo.x + ((float)ix + 0.5f) * esx, box.border.lo.y + ((float)iy + 0.5f) * esy,
+                     0.5f * (box.border.lo.z + box.border.hi.z));
+    const f3 ge = l2g_pos(D.box_m, pc);
+    const f3 gs = l2g_pos(D.src_m, mk(0.0f, 0.0f, 0.0f));
+    for (int k = 0; k < D.n_solids; ++k)
+      if (D.solids[k].type == kVoxel && (D.only < 0 || k == D.only)) drr_voxel_solid(D.solids[k], gs, ge, seg, L);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int32_t* bins = reinterpret_cast<int32_t*>(stage + kScratchBins);
-    float* w = reinterpret_cast<float*>(stage + kScratchWeights);
-    uint32_t n = 0;
-    for (int k = 0; k < nb; ++k)
-      if (W[k] > 0.0) {
-        bins[n] = k;
-        w[n] = (float)W[k];
-        ++n;
-      }
-    stage[0] = n;
+  // the pixel's lengths, summed in the order of its parts into part 0's place
+  for (int m = seg; m < D.n_mat; m += kDrrSegs) {
+    double* row = s_len + m * kDrrBlock + pixel;
+    double sum = row[0];
+    for (int k = 1; k < kDrrSegs; ++k) sum += row[k * kDrrTile];
+    row[0] = sum;
+  }
+  __syncthreads();
+  double t = 0.0;
+  for (int j = seg; j < D.n_w; j += kDrrSegs) {
+    double mu = 0.0;
+    for (int m = 0; m < D.n_mat; ++m) mu += D.mu[(size_t)j * D.n_mat + m] * s_len[m * kDrrBlock + pixel];
+    t += (double)D.w[j] * exp(-mu);
+  }
+  double* part = s_len + (size_t)D.n_mat * kDrrBlock;
+  part[tid] = t;
+  __syncthreads();
+  if (seg == 0 && inside) {
+    for (int k = 1; k < kDrrSegs; ++k) t += part[k * kDrrTile + pixel];
+    D.image[(size_t)iy * box.ne[0] + ix] = (float)t;
   }
 }
 
@@ -1851,8 +1842,13 @@ struct ggh_context {
   DevBuf<DevSolid> acq_solids;
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
-  // this device's address of the file-scope staging array `scratch`
-  uint32_t* scratch = nullptr;
+  // ray tracer: the spectrum's energy bins of nonzero weight (set with the
+  // physics tables and the source), and ggh_drr's image, kept between calls
+  DevBuf<float> drr_w;
+  DevBuf<double> drr_mu;  // sigma_tot [bin][material]
+  int drr_n_w = 0;
+  DevBuf<float> drr_image;
+  std::mutex drr_mu_image;  // one ggh_drr at a time uses drr_image
 };
 
 namespace {
@@ -1860,27 +1856,6 @@ namespace {
 int check_ctx(ggh_context* c) {
   if (!c) return fail(-1, "null context");
   HIP_TRY(hipSetDevice(c->device));
-  return 0;
-}
-
-// The device address of `scratch` on `device`, which must be the current
-// device: each GPU holds its own copy of the array.  Resolved once per
-// device; host code passes this address, never the array's name, to kernels.
-constexpr int kMaxDevices = 64;
-std::mutex g_scratch_mu;
-uint32_t* g_scratch[kMaxDevices] = {};
-
-int scratch_address(int device, uint32_t** out) {
-  if (device < 0 || device >= kMaxDevices) return fail(-2, "device index beyond the staging-array table");
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  if (!g_scratch[device]) {
-    void* p = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !p)
-      return fail(-100 - (int)e, std::string("staging array address: ") + hipGetErrorString(e));
-    g_scratch[device] = static_cast<uint32_t*>(p);
-  }
-  *out = g_scratch[device];
   return 0;
 }
 
@@ -2069,6 +2044,81 @@ int batch_layout(uint64_t n, uint32_t& n_batches, uint32_t& base, uint32_t& rem,
   return 0;
 }
 
+// BinarySearch over the host energy grid, as the transport does it
+int host_bin(const std::vector<float>& a, float key) {
+  int low = 0, high = (int)a.size() - 1;
+  while (high - low > 1) {
+    const int mid = (high + low) / 2;
+    if (a[mid] == key) return mid;
+    if (a[mid] < key) low = mid;
+    else high = mid;
+  }
+  return low;
+}
+
+// Probability of each energy bin of the cross-section tables under the
+// source's sampling (GetPrimariesGGEMSXRaySource.cl:103-125): line idx has
+// probability cdf[idx+1] - cdf[idx]; an interpolated spectrum spreads it
+// uniformly over [E_idx, E_idx+1), split at the bin edges.  W holds nbins
+// (<= 2048) doubles of work space; bins and w receive the bins of nonzero
+// weight, whose count is returned.  Allocates nothing.
+int drr_weights(const ggh_context* c, double* W, int32_t* bins, float* w) {
+  const std::vector<float>& eb = c->ebins_host;
+  const int nb = (int)eb.size();
+  for (int k = 0; k < nb; ++k) W[k] = 0.0;
+  const std::vector<float>& e = c->spectrum_host;
+  const std::vector<float>& f = c->cdf_host;
+  for (int idx = 0; idx + 1 < (int)f.size() && idx + 1 < (int)e.size(); ++idx) {
+    const double p = (double)f[idx + 1] - (double)f[idx];
+    if (!(p > 0.0)) continue;
+    const double a = e[idx], b = e[idx + 1];
+    if (!c->is_interp || !(b > a)) {
+      W[host_bin(eb, e[idx])] += p;
+      continue;
+    }
+    for (int k = 0; k + 1 < nb; ++k) {
+      const double lo = k == 0 ? -INFINITY : (double)eb[k];
+      const double hi = k + 2 == nb ? INFINITY : (double)eb[k + 1];
+      const double ov = std::min(b, hi) - std::max(a, lo);
+      if (ov > 0.0) W[k] += p * ov / (b - a);
+    }
+  }
+  int n = 0;
+  for (int k = 0; k < nb; ++k)
+    if (W[k] > 0.0) {
+      bins[n] = k;
+      w[n] = (float)W[k];
+      ++n;
+    }
+  return n;
+}
+
+// The ray tracer's spectrum table: the weights and the total cross sections
+// of the energy bins the source reaches.  Built when the physics tables or
+// the source are set, so that an image takes one launch and allocates nothing.
+int refresh_drr_table(ggh_context* c) {
+  c->drr_w.release();
+  c->drr_mu.release();
+  c->drr_n_w = 0;
+  if (!c->have_physics || !c->have_source || c->n_mat > kDrrMaxMat) return 0;
+  std::vector<double> W((size_t)c->nbins);
+  std::vector<int32_t> bins((size_t)c->nbins);
+  std::vector<float> w((size_t)c->nbins);
+  const int n = drr_weights(c, W.data(), bins.data(), w.data());
+  std::vector<double> mu((size_t)n * c->n_mat);
+  for (int j = 0; j < n; ++j)
+    for (int m = 0; m < c->n_mat; ++m) {
+      const float4 sg = c->sig_host[(size_t)m * c->nbins + bins[j]];
+      mu[(size_t)j * c->n_mat + m] = (double)sg.x + (double)sg.y + (double)sg.z;
+    }
+  int rc = dev_upload(c->drr_w, w.data(), (size_t)n, c->stream);
+  if (!rc) rc = dev_upload(c->drr_mu, mu.data(), mu.size(), c->stream);
+  if (rc) return rc;
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  c->drr_n_w = n;
+  return 0;
+}
+
 struct Launch {
   void (*fn)(RunParams);
   unsigned grid;
@@ -2200,8 +2250,7 @@ int ggh_context_create(int device, ggh_context** out) {
     delete c;
     return fail(-100 - (int)e, std::string("device query / stream / event creation: ") + hipGetErrorString(e));
   }
-  int rc = scratch_address(device, &c->scratch);
-  if (!rc) rc = dev_alloc(c->stats, 8);
+  int rc = dev_alloc(c->stats, 8);
   if (!rc) rc = dev_alloc(c->rng, (size_t)5 * GGH_MAX_SLOTS);
   if (!rc) rc = dev_alloc(c->queue, 1);
   if (rc) {
@@ -2229,6 +2278,7 @@ int ggh_context_destroy(ggh_context* c) {
   c->solids_dev.release();
   drop_acquisition(c);
   c->tally.release(); c->ptrack.release();
+  c->drr_w.release(); c->drr_mu.release(); c->drr_image.release();
   c->spectrum.release(); c->cdf.release(); c->rng.release(); c->queue.release(); c->stats.release();
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -2293,7 +2343,7 @@ int ggh_set_physics(ggh_context* c, const ggh_physics_desc* d) {
   if ((rc = dev_upload(c->density, d->density, (size_t)nm, c->stream))) return rc;
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->have_physics = true;
-  return 0;
+  return refresh_drr_table(c);
 }
 
 int ggh_add_voxel_solid(ggh_context* c, const ggh_voxel_solid_desc* d) {
@@ -2658,7 +2708,7 @@ int ggh_set_xray_source(ggh_context* c, const ggh_xray_source_desc* d) {
   c->cdf_host = f;
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->have_source = true;
-  return 0;
+  return refresh_drr_table(c);
 }
 
 int ggh_seed(ggh_context* c, uint32_t seed) {
@@ -2859,55 +2909,6 @@ int ggh_replay_acquisition(ggh_context* c) {
 
 namespace {
 
-// BinarySearch over the host energy grid, as the device does it
-int host_bin(const std::vector<float>& a, float key) {
-  int low = 0, high = (int)a.size() - 1;
-  while (high - low > 1) {
-    const int mid = (high + low) / 2;
-    if (a[mid] == key) return mid;
-    if (a[mid] < key) low = mid;
-    else high = mid;
-  }
-  return low;
-}
-
-// Probability of each energy bin of the cross-section tables under the
-// source's sampling (GetPrimariesGGEMSXRaySource.cl:103-125): line idx has
-// probability cdf[idx+1] - cdf[idx]; an interpolated spectrum spreads it
-// uniformly over [E_idx, E_idx+1), split at the bin edges.  W holds nbins
-// (<= 2048) doubles of work space; bins and w receive the bins of nonzero
-// weight, whose count is returned.  Allocates nothing.
-int drr_weights(const ggh_context* c, double* W, int32_t* bins, float* w) {
-  const std::vector<float>& eb = c->ebins_host;
-  const int nb = (int)eb.size();
-  for (int k = 0; k < nb; ++k) W[k] = 0.0;
-  const std::vector<float>& e = c->spectrum_host;
-  const std::vector<float>& f = c->cdf_host;
-  for (int idx = 0; idx + 1 < (int)f.size() && idx + 1 < (int)e.size(); ++idx) {
-    const double p = (double)f[idx + 1] - (double)f[idx];
-    if (!(p > 0.0)) continue;
-    const double a = e[idx], b = e[idx + 1];
-    if (!c->is_interp || !(b > a)) {
-      W[host_bin(eb, e[idx])] += p;
-      continue;
-    }
-    for (int k = 0; k + 1 < nb; ++k) {
-      const double lo = k == 0 ? -INFINITY : (double)eb[k];
-      const double hi = k + 2 == nb ? INFINITY : (double)eb[k + 1];
-      const double ov = std::min(b, hi) - std::max(a, lo);
-      if (ov > 0.0) W[k] += p * ov / (b - a);
-    }
-  }
-  int n = 0;
-  for (int k = 0; k < nb; ++k)
-    if (W[k] > 0.0) {
-      bins[n] = k;
-      w[n] = (float)W[k];
-      ++n;
-    }
-  return n;
-}
-
 // Checks shared by both ray-tracer entry points; fills the launch
 // parameters except the weights and the image.  Allocates nothing when the
 // solid table is already on the device (allow_upload false).
@@ -2943,12 +2944,22 @@ int drr_setup(ggh_context* c, int solid, int projection, const float* image, boo
   D.solids = c->solids_dev.p;
   D.n_solids = (int32_t)c->solids.size();
   D.box = solid;
-  D.sig = c->tab_sig.p;
-  D.nbins = c->nbins;
   D.n_mat = c->n_mat;
+  D.w = c->drr_w.p;
+  D.mu = c->drr_mu.p;
+  D.n_w = c->drr_n_w;
   return 0;
 }
 
+int drr_launch(const ggh_context* c, const DevSolid& box, const DrrParams& D, hipStream_t stream) {
+  const unsigned tiles = (unsigned)((box.ne[0] + kDrrTileX - 1) / kDrrTileX) *
+                         (unsigned)((box.ne[1] + kDrrTileY - 1) / kDrrTileY);
+  const size_t lds = drr_lds_bytes(D.n_mat);
+  if (lds > (size_t)c->max_lds) return fail(-3, "the ray tracer's path lengths do not fit in LDS");
+  hipLaunchKernelGGL(drr_kernel, dim3(tiles), dim3(kDrrBlock), lds, stream, D);
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
 
 }  // namespace
 
@@ -2959,28 +2970,13 @@ int ggh_drr(ggh_context* c, int solid, int projection, float* image) {
   int rc = drr_setup(c, solid, projection, image, true, D);
   if (rc) return rc;
   const DevSolid& box = c->solids[solid];
-  std::vector<double> W((size_t)c->nbins);
-  std::vector<int32_t> bins((size_t)c->nbins);
-  std::vector<float> w((size_t)c->nbins);
-  const int n_w = drr_weights(c, W.data(), bins.data(), w.data());
   const size_t npx = (size_t)box.ne[0] * box.ne[1];
-  DevBuf<int32_t> db;
-  DevBuf<float> dw, dimg;
-  if ((rc = dev_upload(db, bins.data(), (size_t)n_w, c->stream)) || (rc = dev_upload(dw, w.data(), (size_t)n_w, c->stream)) ||
-      (rc = dev_alloc(dimg, npx)))
-    return rc;
-  D.w_bin = db.p;
-  D.w = dw.p;
-  D.n_w = n_w;
-  D.image = dimg.p;
-  hipLaunchKernelGGL(drr_kernel, dim3((unsigned)((npx + kDrrBlock - 1) / kDrrBlock)), dim3(kDrrBlock), 0, c->stream, D);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(image, dimg.p, npx * sizeof(float), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  db.release();
-  dw.release();
-  dimg.release();
-  if (e != hipSuccess) return fail(-100 - (int)e, std::string("ray tracer: ") + hipGetErrorString(e));
+  std::lock_guard<std::mutex> lock(c->drr_mu_image);
+  if (c->drr_image.n < npx && (rc = dev_alloc(c->drr_image, npx))) return rc;
+  D.image = c->drr_image.p;
+  if ((rc = drr_launch(c, box, D, c->stream))) return rc;
+  HIP_TRY(hipMemcpyAsync(image, D.image, npx * sizeof(float), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
   return 0;
 }
 
@@ -2989,23 +2985,10 @@ int ggh_drr_noalloc(ggh_context* c, int solid, int projection, float* image, voi
   int rc = drr_setup(c, solid, projection, image, false, D);
   if (rc) return rc;
   if (c->nbins > kNoAllocMaxBins)
-    return fail(-2, "ggh_drr_noalloc stages the weights of at most 1024 energy bins (the physics tables have " +
+    return fail(-2, "ggh_drr_noalloc takes physics tables of at most 1024 energy bins (these have " +
                         std::to_string(c->nbins) + "); ggh_drr has no such limit");
-  if (!c->scratch) return fail(-3, "the staging array was not resolved for this device");
-  const hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c->stream;
-  uint32_t* stage = c->scratch;
-  hipLaunchKernelGGL(drr_weights_kernel, dim3(1), dim3(kWeightsBlock), 0, s, c->ebins.p, c->nbins, c->spectrum.p,
-                     (int)c->spectrum_host.size(), c->cdf.p, (int)c->cdf_host.size(), c->is_interp, stage);
-  const DevSolid& box = c->solids[solid];
-  const size_t npx = (size_t)box.ne[0] * box.ne[1];
-  D.w_bin = reinterpret_cast<const int32_t*>(stage + kScratchBins);
-  D.w = reinterpret_cast<const float*>(stage + kScratchWeights);
-  D.n_w_dev = stage;
   D.image = image;
-  hipLaunchKernelGGL(drr_kernel, dim3((unsigned)((npx + kDrrBlock - 1) / kDrrBlock)), dim3(kDrrBlock), 0, s, D);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(-100 - (int)e, std::string("ray tracer (no allocation): ") + hipGetErrorString(e));
-  return 0;
+  return drr_launch(c, c->solids[solid], D, stream ? static_cast<hipStream_t>(stream) : c->stream);
 }
 
 int ggh_get_projection(ggh_context* c, int solid, int projection, int32_t* counts, int32_t* scatter) {

@@ -250,11 +250,9 @@ int ggh_drr(ggh_context* ctx, int solid, int projection, float* image);
 /* ggh_drr without allocating: no counterpart in GGEMS.  For callers that
  * cannot allocate device memory (code under HIP graph capture, serving
  * loops).  `image` is a device buffer of the box solid's rows x cols floats
- * on the context's device; the two kernels (spectrum weights, ray tracer)
- * are queued on `stream` (a hipStream_t; null: the context's stream) and the
- * call returns without waiting.  The weights are staged in one array of
- * 8,448 bytes per GPU, shared by every call on that GPU: calls that overlap
- * on one GPU race.  Limits: at most 1,024 energy bins in the physics tables,
+ * on the context's device; the kernel is queued on `stream` (a hipStream_t;
+ * null: the context's stream) and the call returns without waiting.  Calls
+ * may overlap.  Limits: at most 1,024 energy bins in the physics tables,
  * and the solid table must already be on the device (after a ggh_run,
  * ggh_run_acquisition or ggh_drr since the last solid was added); otherwise
  * the call fails and allocates nothing.  Same image as ggh_drr, bit for bit. */
