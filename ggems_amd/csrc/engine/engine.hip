@@ -64,7 +64,8 @@ enum SolidType : int32_t { kVoxel = 0, kBoxSolid = 1, kMesh = 2 };
 // (exact division, see div_rn); in_lo/in_hi = border -/+ the geometry
 // tolerance, the bounds IsParticleInAABB compares against.  labels is the
 // MHD order (x fastest); bricks holds the same labels in 128-byte bricks of
-// 8 x 4 x 4 voxels (kBrick*), nbx bricks along x and nbxy per brick layer.
+// 8 x 4 x 4 voxels (kBrick*), nbx bricks along x and nbxy per brick layer;
+// brick_y and brick_z are brick_offset's strides.
 struct VoxGeom {
   f3 lo, vs, rvs, in_lo, in_hi;
   int32_t nx, ny, nz, nxy;
@@ -73,6 +74,7 @@ struct VoxGeom {
   int32_t mat_offset;
   int32_t solid;
   int32_t nbx, nbxy;
+  int32_t brick_y, brick_z;
 };
 
 // 128-byte label bricks: one L2 line holds an 8 x 4 x 4 neighbourhood
@@ -83,9 +85,12 @@ struct VoxGeom {
 constexpr int kBrickX = 8, kBrickY = 4, kBrickZ = 4;
 static_assert(kBrickX * kBrickY * kBrickZ == 128, "brick_offset's shifts assume 8 x 4 x 4");
 
-__host__ __device__ inline uint32_t brick_offset(int nbx, int nbxy, int vx, int vy, int vz) {
-  const uint32_t b = (uint32_t)((vz >> 2) * nbxy + (vy >> 2) * nbx + (vx >> 3));
-  return (b << 7) | ((uint32_t)(vz & 3) << 5) | ((uint32_t)(vy & 3) << 3) | (uint32_t)(vx & 7);
+// ((z / 4) nbxy + (y / 4) nbx + x / 8) * 128 + (z % 4) 32 + (y % 4) 8 + x % 8,
+// with each axis's quotient and remainder folded into one product:
+// brick_y = 128 nbx - 32, brick_z = 128 nbxy - 128
+__host__ __device__ inline uint32_t brick_offset(const VoxGeom& G, int vx, int vy, int vz) {
+  return (uint32_t)(vx + (vx >> 3) * 120) + (uint32_t)(8 * vy + (vy >> 2) * G.brick_y) +
+         (uint32_t)(32 * vz + (vz >> 2) * G.brick_z);
 }
 
 struct DevSolid {
@@ -106,7 +111,6 @@ struct DevSolid {
   const float4* tris;
   int32_t n_bvh;
   int32_t box_index;  // rank among the box solids (per-projection matrices), -1 otherwise
-  int32_t pad_[2];
 };
 
 static_assert(sizeof(DevSolid) % 16 == 0, "solids are staged in LDS after 16-byte table entries");
@@ -201,7 +205,7 @@ struct Tabs {
 // ---------------------------------------------------------------------------
 enum Mode : int32_t {
   kInVoxel = 0,    // stepping through a voxel solid (hot)
-  kInteract = 1,   // a voxel step ended on a discrete process (pend = proc | gmat << 2)
+  kInteract = 1,   // a voxel step stopped on a discrete process, or may have (see Lane)
   kCut = 2,        // a voxel step left the photon at or below the material's energy cut
   kExit = 3,       // left the voxel solid
   kNeedPrimary = 4,
@@ -211,7 +215,10 @@ enum Mode : int32_t {
 };
 
 // p and ray hold the local frame of the solid while mode is kInVoxel ..
-// kExit, the global frame otherwise.
+// kExit, the global frame otherwise.  In mode kInteract the reference
+// sampling keeps the stopped step's random sums in pend, s1 and s2, with p
+// where the step began; tau sampling keeps the material (gmat << 2) in pend,
+// and the reference step of thin voxels proc | gmat << 2.
 struct Lane {
   Rng r;
   f3 p;
@@ -222,7 +229,7 @@ struct Lane {
   int32_t solid;
   int32_t hop;
   int32_t scatter;
-  int32_t pend;
+  uint32_t pend, s1, s2;
   uint32_t todo;
   uint32_t slot;
   uint32_t proj;  // current projection of an acquisition
@@ -479,7 +486,7 @@ __device__ inline void dose_record(const RunParams& P, float edep, f3 p) {
 // ---------------------------------------------------------------------------
 // voxel solid transport (src/kernels/TrackThroughGGEMSVoxelizedSolid.cl:133-310)
 // ---------------------------------------------------------------------------
-__device__ inline bool in_bounds(f3 p, const VoxGeom& G) {
+__host__ __device__ inline bool in_bounds(f3 p, const VoxGeom& G) {
   // IsParticleInAABB with its tolerance folded into the bounds
   return !((p.x < G.in_lo.x) | (p.x > G.in_hi.x) | (p.y < G.in_lo.y) | (p.y > G.in_hi.y) | (p.z < G.in_lo.z) |
            (p.z > G.in_hi.z));
@@ -489,26 +496,170 @@ __device__ inline bool in_bounds(f3 p, const VoxGeom& G) {
 // IEEE quotient.  False when outside the label volume (the reference checks
 // the upper bound only; a negative index would read outside the volume, so
 // it ends the walk like an exit).
-__device__ inline bool voxel_of(f3 p, const VoxGeom& G, int& vx, int& vy, int& vz) {
+__host__ __device__ inline bool voxel_of(f3 p, const VoxGeom& G, int& vx, int& vy, int& vz) {
   vx = (int)div_rn(p.x - G.lo.x, G.vs.x, G.rvs.x);
   vy = (int)div_rn(p.y - G.lo.y, G.vs.y, G.rvs.y);
   vz = (int)div_rn(p.z - G.lo.z, G.vs.z, G.rvs.z);
   return ((uint32_t)vx < (uint32_t)G.nx) & ((uint32_t)vy < (uint32_t)G.ny) & ((uint32_t)vz < (uint32_t)G.nz);
 }
 
-__device__ inline Box voxel_box(const VoxGeom& G, int vx, int vy, int vz) {
+__host__ __device__ inline Box voxel_box(const VoxGeom& G, int vx, int vy, int vz) {
   Box b;
   b.lo = mk(G.lo.x + (float)vx * G.vs.x, G.lo.y + (float)vy * G.vs.y, G.lo.z + (float)vz * G.vs.z);
   b.hi = add(b.lo, G.vs);
   return b;
 }
 
-// One iteration of the reference do-while, up to the point where the step's
-// outcome is known.  Returns true when the step counts as a voxel step (the
-// voxel index was inside the volume).  The label gather is issued first and
-// the random draws of the step, which do not depend on it, cover its latency.
+// voxel_of for a point that is known to lie inside the volume (in_bounds,
+// and grid_is_quick)
+__device__ inline void voxel_inside(f3 p, const VoxGeom& G, int& vx, int& vy, int& vz) {
+  vx = (int)div_rn(p.x - G.lo.x, G.vs.x, G.rvs.x);
+  vy = (int)div_rn(p.y - G.lo.y, G.vs.y, G.rvs.y);
+  vz = (int)div_rn(p.z - G.lo.z, G.vs.z, G.rvs.z);
+}
+
+// photon fluence of a crossed voxel (dose_photon_tracking)
+__device__ inline void track_fluence(const RunParams& P, const VoxGeom& G, f3 p) {
+  if (!P.ptrack || G.solid != P.dose_solid) return;
+  const int id = dosel_index(P, p);
+  if (id >= 0) atomicAdd(&P.ptrack[id], 1);
+}
+
+// the mode a voxel step leaves: out of the phantom, at or below the
+// material's energy cut, or in the next voxel.  By selects: stores to
+// different lane fields on different paths would be merged by the compiler
+// into one store through a selected address, which keeps the lane state out
+// of registers.
+__device__ inline int32_t after_step(const VoxGeom& G, const Lane& L, float cut) {
+  return !in_bounds(L.p, G) ? kExit : (L.e <= cut ? kCut : kInVoxel);
+}
+
+// One iteration of the reference do-while.  The label gather is issued first
+// and the random draws of the step, which do not depend on it, cover its
+// latency.
+//
+// Three competing exponentials decide whether the photon interacts before
+// the voxel's boundary at distance db, and about one step in fifty does.  A
+// process with cross section sigma can only win when -log(u) < sigma db; as
+// -log(u) >= 1 - u, a draw with u < 1 - sigma db cannot.  The step therefore
+// compares (float)sum 2^-32 + 1.01 sigma db with 1 - 2^-19 (the margins cover
+// the uniform's and the logarithm's rounding: over all 2^32 sums -log(u) is
+// at least 0.998 (1 - u) above 2^-19), and only a step that this cannot rule
+// out stops, with its sums kept, to take the logarithms and quotients in
+// resolve_interaction: three logarithms, three correctly rounded quotients
+// and the second table read are gone from the step (about 170 of its 770
+// cycles of issue; the geometry gave another 200).  3*10^7 primaries through a
+// 256 x 256 x 128 body: 50.8 -> 46.6 ms with both.
 template <int NP, bool kTrack>
 __device__ inline bool hot_step(const RunParams& P, const Tabs& T, const VoxGeom& G, Lane& L) {
+  int vx, vy, vz;
+  voxel_inside(L.p, G, vx, vy, vz);
+  const uint32_t label = G.labels[vx + vy * G.nx + vz * G.nxy];
+  const int np = NP >= 0 ? NP : P.n_proc;
+  uint32_t s0 = 0, s1 = 0, s2 = 0;
+  if (np > 0) s0 = L.r.next_sum();
+  if (np > 1) s1 = L.r.next_sum();
+  if (np > 2) s2 = L.r.next_sum();
+  const Box vox = voxel_box(G, vx, vy, vz);
+  const f3 p = inside_quick(L.p, vox);
+  const float db = exit_quick(p, L.ray, vox);
+  const float4 sig = T.sig[(G.mat_offset + (int)label) * P.nbins + L.eid];
+  const float far = db * 1.01f;
+  const float most = fmaxf(fmaxf(__builtin_fmaf((float)s0, 0x1p-32f, sig.x * far),
+                                 __builtin_fmaf((float)s1, 0x1p-32f, sig.y * far)),
+                           __builtin_fmaf((float)s2, 0x1p-32f, sig.z * far));
+  if (most < 1.0f - 0x1p-19f) {
+    if (kTrack) track_fluence(P, G, p);
+    L.p = add(p, scl(L.ray.d, db + kTol));
+    safety_outside(L.p, vox);
+    L.mode = after_step(G, L, sig.w);
+  } else {
+    L.mode = kInteract;
+    L.pend = s0;
+    L.s1 = s1;
+    L.s2 = s2;
+  }
+  return true;
+}
+
+// The step that hot_step stopped, from its point and its sums: the process
+// it ends on, or kTransportation when it crosses the voxel or leaves the
+// phantom; the lane's mode then says where it went.
+template <int NP, bool kTrack>
+__device__ inline int stopped_step(const RunParams& P, const Tabs& T, const VoxGeom& G, Lane& L, int& gmat) {
+  int vx, vy, vz;
+  voxel_inside(L.p, G, vx, vy, vz);
+  gmat = G.mat_offset + (int)G.labels[vx + vy * G.nx + vz * G.nxy];
+  const float lg[3] = {neg_log_uniform(L.pend), neg_log_uniform(L.s1), neg_log_uniform(L.s2)};
+  const Box vox = voxel_box(G, vx, vy, vz);
+  const f3 p = inside_quick(L.p, vox);
+  const float db = exit_quick(p, L.ray, vox);
+  const int ti = gmat * P.nbins + L.eid;
+  const float4 sig = T.sig[ti];
+  int proc;
+  float next = next_interaction<NP>(P, sig, T.rcp[ti], lg, proc);
+  if (db <= next) {
+    next = db + kTol;
+    proc = kTransportation;
+    if (kTrack) track_fluence(P, G, p);
+  }
+  L.p = add(p, scl(L.ray.d, next));
+  safety_outside(L.p, vox);
+  if (proc == kTransportation || !in_bounds(L.p, G)) {
+    L.mode = after_step(G, L, sig.w);
+    proc = kTransportation;
+  }
+  return proc;
+}
+
+// The voxel step of tau sampling: the walk, tolerances and outcomes of
+// the reference step, with the interaction decided by the flight's tau
+// instead of three fresh exponentials.  A step whose boundary distance db
+// costs a = sigma_tot * db <= tau crosses the voxel and spends a; otherwise
+// the photon interacts at tau / sigma_tot (the IEEE quotient) and the process
+// is chosen when the interaction is resolved.  sigma_tot = (sigma_0 +
+// sigma_1) + sigma_2 in activation order, its reciprocal in the w of the
+// second table entry.
+template <bool kTrack, bool kThin>
+__device__ inline bool hot_step_tau(const RunParams& P, const Tabs& T, const VoxGeom& G, Lane& L) {
+  int vx, vy, vz;
+  if (kThin) {
+    if (!voxel_of(L.p, G, vx, vy, vz)) {
+      L.mode = kExit;
+      return false;
+    }
+  } else {
+    voxel_inside(L.p, G, vx, vy, vz);
+  }
+  const uint32_t label = G.bricks[brick_offset(G, vx, vy, vz)];
+  const Box vox = voxel_box(G, vx, vy, vz);
+  if (kThin) safety_inside(L.p, vox);
+  else L.p = inside_quick(L.p, vox);
+  const float db = kThin ? distance_to_aabb(L.p, L.ray, vox) : exit_quick(L.p, L.ray, vox);
+  const int gmat = G.mat_offset + (int)label;
+  const int ti = gmat * P.nbins + L.eid;
+  const float4 sig = T.sig[ti];
+  const float rtot = T.rcp[ti].w;
+  const float tot = (sig.x + sig.y) + sig.z;
+  const float a = tot * db;
+  const bool cross = !(L.tau < a);
+  const float next = cross ? db + kTol : div_rn(L.tau, tot, rtot);
+  L.tau = cross ? L.tau - a : L.tau;
+  if (kTrack && cross) track_fluence(P, G, L.p);
+  L.p = add(L.p, scl(L.ray.d, next));
+  safety_outside(L.p, vox);
+  const bool out = !in_bounds(L.p, G);
+  const bool inter = !out & !cross;
+  const bool cut = !out & !inter & (L.e <= sig.w);  // photon_energy_cut_[material]
+  L.mode = out ? kExit : (inter ? kInteract : (cut ? kCut : kInVoxel));
+  L.pend = inter ? (uint32_t)(gmat << 2) : L.pend;
+  return true;
+}
+
+// The reference step on any grid (thin voxels, far coordinates: see
+// quick_grid), which resolves its three exponentials at once.
+template <int NP, bool kTrack>
+__device__ inline bool hot_step_thin(const RunParams& P, const Tabs& T, const VoxGeom& G, Lane& L) {
   int vx, vy, vz;
   if (!voxel_of(L.p, G, vx, vy, vz)) {
     L.mode = kExit;
@@ -529,63 +680,15 @@ __device__ inline bool hot_step(const RunParams& P, const Tabs& T, const VoxGeom
   if (db <= next) {
     next = db + kTol;
     proc = kTransportation;
-    if (kTrack && P.ptrack && G.solid == P.dose_solid) {
-      int id = dosel_index(P, L.p);
-      if (id >= 0) atomicAdd(&P.ptrack[id], 1);
-    }
+    if (kTrack) track_fluence(P, G, L.p);
   }
   L.p = add(L.p, scl(L.ray.d, next));
   safety_outside(L.p, vox);
-  // outcome by selects: stores to different lane fields on different paths
-  // would be merged by the compiler into one store through a selected
-  // address, which keeps the lane state out of registers
   const bool out = !in_bounds(L.p, G);
   const bool inter = !out & (proc != kTransportation);
   const bool cut = !out & !inter & (L.e <= sig.w);  // photon_energy_cut_[material]
   L.mode = out ? kExit : (inter ? kInteract : (cut ? kCut : kInVoxel));
-  L.pend = inter ? (proc | (gmat << 2)) : L.pend;
-  return true;
-}
-
-// The voxel step of tau sampling: the walk, tolerances and outcomes of
-// hot_step, with the interaction decided by the flight's tau instead of
-// three fresh exponentials.  A step whose boundary distance db costs
-// a = sigma_tot * db <= tau crosses the voxel and spends a; otherwise the
-// photon interacts at tau / sigma_tot (the IEEE quotient) and the process
-// is chosen when the interaction is resolved.  sigma_tot = (sigma_0 +
-// sigma_1) + sigma_2 in activation order, its reciprocal in the w of the
-// second table entry.
-template <bool kTrack>
-__device__ inline bool hot_step_tau(const RunParams& P, const Tabs& T, const VoxGeom& G, Lane& L) {
-  int vx, vy, vz;
-  if (!voxel_of(L.p, G, vx, vy, vz)) {
-    L.mode = kExit;
-    return false;
-  }
-  const uint32_t label = G.bricks[brick_offset(G.nbx, G.nbxy, vx, vy, vz)];
-  const Box vox = voxel_box(G, vx, vy, vz);
-  safety_inside(L.p, vox);
-  const float db = distance_to_aabb(L.p, L.ray, vox);
-  const int gmat = G.mat_offset + (int)label;
-  const int ti = gmat * P.nbins + L.eid;
-  const float4 sig = T.sig[ti];
-  const float rtot = T.rcp[ti].w;
-  const float tot = (sig.x + sig.y) + sig.z;
-  const float a = tot * db;
-  const bool cross = !(L.tau < a);
-  const float next = cross ? db + kTol : div_rn(L.tau, tot, rtot);
-  L.tau = cross ? L.tau - a : L.tau;
-  if (kTrack && cross && P.ptrack && G.solid == P.dose_solid) {
-    int id = dosel_index(P, L.p);
-    if (id >= 0) atomicAdd(&P.ptrack[id], 1);
-  }
-  L.p = add(L.p, scl(L.ray.d, next));
-  safety_outside(L.p, vox);
-  const bool out = !in_bounds(L.p, G);
-  const bool inter = !out & !cross;
-  const bool cut = !out & !inter & (L.e <= sig.w);  // photon_energy_cut_[material]
-  L.mode = out ? kExit : (inter ? kInteract : (cut ? kCut : kInVoxel));
-  L.pend = inter ? (gmat << 2) : L.pend;
+  L.pend = inter ? (uint32_t)(proc | (gmat << 2)) : L.pend;
   return true;
 }
 
@@ -947,10 +1050,14 @@ __device__ inline void store_stream(const RunParams& P, uint32_t slot, const Rng
 
 // The discrete process a voxel step stopped on, then the energy cut
 // (TrackThroughGGEMSVoxelizedSolid.cl:238-310).
-template <int NP, bool kTau, class Counters>
-__device__ inline void resolve_interaction(const RunParams& P, const Tabs& T, Lane& L, Counters& c) {
-  const int gmat = L.pend >> 2;
-  int proc = L.pend & 3;
+template <int NP, bool kTau, bool kTrack, bool kThin, class Counters>
+__device__ inline void resolve_interaction(const RunParams& P, const Tabs& T, const VoxGeom& G, Lane& L, Counters& c) {
+  int gmat = (int)(L.pend >> 2);
+  int proc = (int)(L.pend & 3u);
+  if (!kTau && !kThin) {
+    proc = stopped_step<NP, kTrack>(P, T, G, L, gmat);
+    if (proc == kTransportation) return;
+  }
   if (kTau) {
     // the process, in proportion to its left-bin cross section: the first
     // whose running sum in activation order exceeds u * sigma_tot
@@ -1001,9 +1108,10 @@ __device__ inline void next_projection(const RunParams& P, Lane& L) {
 
 // the cold work of one lane, one state at a time in an order that lets a
 // lane pass through several states in one call
-template <int NP, bool kSingle, bool kAcq, bool kTau, class Counters>
+template <int NP, bool kSingle, bool kAcq, bool kTau, bool kTrack, bool kThin, class Counters>
 __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Counters& c) {
-  if (L.mode == kInteract) resolve_interaction<NP, kTau>(P, T, L, c);
+  if (L.mode == kInteract)
+    resolve_interaction<NP, kTau, kTrack, kThin>(P, T, kSingle ? P.vox0 : T.solids[L.solid].vox, L, c);
   if (L.mode == kCut) {
     if (L.solid == P.dose_solid) dose_record(P, L.e, L.p);
     L.mode = kNeedPrimary;
@@ -1075,7 +1183,10 @@ __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Cou
     if (s.type == kVoxel) {
       L.p = g2l_pos(s.m, L.p);
       L.ray.set(g2l_dir(s.m, L.ray.d));
-      L.mode = kInVoxel;
+      // hot_step takes only points inside the volume (the change of frames
+      // can round a point off its edge)
+      int vx, vy, vz;
+      L.mode = kThin || voxel_of(L.p, s.vox, vx, vy, vz) ? kInVoxel : kExit;
       if (kTau) L.tau = draw_tau(L.r);
     } else if (!kSingle && s.type == kMesh) {
       // ggh_run launches the single-voxel-solid variant only on scenes
@@ -1114,15 +1225,10 @@ __device__ inline void exchange_lane(Lane& L, uint4* s_x, uint32_t pos) {
   __syncthreads();
   dst[0] = make_uint4(__float_as_uint(L.ray.inv.y), __float_as_uint(L.ray.inv.z), __float_as_uint(L.e),
                       (uint32_t)L.eid);
-  if (kTau) {
-    // mode (3 bits), scatter (1 bit) and hop (<= GGH_MAX_HOPS) share a word to make room for tau
-    dst[1] = make_uint4((uint32_t)L.mode | ((uint32_t)L.scatter << 3) | ((uint32_t)L.hop << 4), (uint32_t)L.solid,
-                        (uint32_t)L.pend, L.todo);
-    dst[2] = make_uint4(L.slot, L.proj, __float_as_uint(L.tau), 0u);
-  } else {
-    dst[1] = make_uint4((uint32_t)L.mode, (uint32_t)L.solid, (uint32_t)L.hop, (uint32_t)L.scatter);
-    dst[2] = make_uint4((uint32_t)L.pend, L.todo, L.slot, L.proj);
-  }
+  // mode (3 bits), scatter (1 bit) and hop (<= GGH_MAX_HOPS) share a word to make room for tau or the sums
+  dst[1] = make_uint4((uint32_t)L.mode | ((uint32_t)L.scatter << 3) | ((uint32_t)L.hop << 4), (uint32_t)L.solid,
+                      L.pend, L.todo);
+  dst[2] = make_uint4(L.slot, L.proj, kTau ? __float_as_uint(L.tau) : L.s1, kTau ? 0u : L.s2);
   __syncthreads();
   a = src[0];
   b = src[1];
@@ -1131,25 +1237,19 @@ __device__ inline void exchange_lane(Lane& L, uint4* s_x, uint32_t pos) {
   L.ray.inv.z = __uint_as_float(a.y);
   L.e = __uint_as_float(a.z);
   L.eid = (int32_t)a.w;
+  L.mode = (int32_t)(b.x & 7u);
+  L.scatter = (int32_t)((b.x >> 3) & 1u);
+  L.hop = (int32_t)(b.x >> 4);
+  L.solid = (int32_t)b.y;
+  L.pend = b.z;
+  L.todo = b.w;
+  L.slot = d.x;
+  L.proj = d.y;
   if (kTau) {
-    L.mode = (int32_t)(b.x & 7u);
-    L.scatter = (int32_t)((b.x >> 3) & 1u);
-    L.hop = (int32_t)(b.x >> 4);
-    L.solid = (int32_t)b.y;
-    L.pend = (int32_t)b.z;
-    L.todo = b.w;
-    L.slot = d.x;
-    L.proj = d.y;
     L.tau = __uint_as_float(d.z);
   } else {
-    L.mode = (int32_t)b.x;
-    L.solid = (int32_t)b.y;
-    L.hop = (int32_t)b.z;
-    L.scatter = (int32_t)b.w;
-    L.pend = (int32_t)d.x;
-    L.todo = d.y;
-    L.slot = d.z;
-    L.proj = d.w;
+    L.s1 = d.z;
+    L.s2 = d.w;
   }
   __syncthreads();
 }
@@ -1176,7 +1276,9 @@ __device__ inline uint32_t lds_load_relaxed(uint32_t* p) {
 // and module placement); kRegroup: the scene has a voxel solid, and blocks
 // work in rounds with regrouping (below).  Without a voxel solid every
 // photon is navigated and tracked by its lane's state machine alone.
-template <int NP, bool kSingle, bool kLDS, bool kTrack, bool kAcq, bool kRegroup, bool kTau = false>
+// kThin: a voxel solid is outside what quick_grid allows, and every step takes
+// the general geometry.
+template <int NP, bool kSingle, bool kLDS, bool kTrack, bool kAcq, bool kRegroup, bool kTau = false, bool kThin = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWavesPerEU)))
 void transport_kernel(RunParams P) {
   extern __shared__ float4 s_tab[];
@@ -1229,7 +1331,7 @@ void transport_kernel(RunParams P) {
   L.solid = -1;
   L.hop = 0;
   L.scatter = 0;
-  L.pend = 0;
+  L.pend = L.s1 = L.s2 = 0;
   L.todo = 0;
   L.slot = 0xffffffffu;
   L.proj = 0;
@@ -1245,7 +1347,7 @@ void transport_kernel(RunParams P) {
     for (;;) {
       const bool cold = L.mode != kInVoxel && L.mode != kDone;
       if (!__any(cold)) break;
-      if (cold) cold_step<NP, kSingle, kAcq, kTau>(cold_params(), T, L, c);
+      if (cold) cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin>(cold_params(), T, L, c);
     }
   } else {
     // The block works in rounds.  In each round every wave
@@ -1278,7 +1380,7 @@ void transport_kernel(RunParams P) {
       for (int pass = 0; pass < P.cold_passes; ++pass) {
         const bool cold = L.mode != kInVoxel && L.mode != kDone;
         if (!__any(cold)) break;
-        if (cold) cold_step<NP, kSingle, kAcq, kTau>(cold_params(), T, L, c);
+        if (cold) cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin>(cold_params(), T, L, c);
       }
       if (lane == 0) atomicAdd(&s_cold_done[rb], 1u);
       bool ready = false;
@@ -1294,11 +1396,12 @@ void transport_kernel(RunParams P) {
         // solid, else the lane's solid in the (LDS-staged) solid table
         if (L.mode == kInVoxel) {
           const VoxGeom& G = kSingle ? P.vox0 : T.solids[L.solid].vox;
-          stepped = kTau ? hot_step_tau<kTrack>(P, T, G, L) : hot_step<NP, kTrack>(P, T, G, L);
+          stepped = kTau ? hot_step_tau<kTrack, kThin>(P, T, G, L)
+                         : (kThin ? hot_step_thin<NP, kTrack>(P, T, G, L) : hot_step<NP, kTrack>(P, T, G, L));
           // tau sampling makes two steps per pass: its step is short, so the
           // pass's ballots and round checks weigh more (measured faster; three
           // gained little more, four was slower)
-          if (kTau && L.mode == kInVoxel) stepped2 = hot_step_tau<kTrack>(P, T, G, L);
+          if (kTau && L.mode == kInVoxel) stepped2 = hot_step_tau<kTrack, kThin>(P, T, G, L);
         }
         steps += __popcll(__ballot(stepped)) + (kTau ? __popcll(__ballot(stepped2)) : 0);
         // pending interactions resolved in batches, so that scattered photons
@@ -1307,7 +1410,9 @@ void transport_kernel(RunParams P) {
         // without the interaction code (measured), and its steps are cheap
         // enough that the waiting lanes cost less.
         if (!kTau && __popcll(__ballot(L.mode == kInteract)) >= P.interact_batch) {
-          if (L.mode == kInteract) resolve_interaction<NP, kTau>(cold_params(), T, L, c);
+          const RunParams& Q = cold_params();
+          if (L.mode == kInteract)
+            resolve_interaction<NP, kTau, kTrack, kThin>(Q, T, kSingle ? Q.vox0 : T.solids[L.solid].vox, L, c);
         }
       }
       if constexpr (kTau) {
@@ -1560,7 +1665,7 @@ __device__ void drr_voxel_solid(const DevSolid& s, f3 gs, f3 ge, int seg, double
 #pragma unroll
     for (int b = 0; b < kDrrBatch; ++b) {
       // a finished walk repeats its last voxel with no length
-      off[b] = brick_offset(G.nbx, G.nbxy, i[0], i[1], i[2]);
+      off[b] = brick_offset(G, i[0], i[1], i[2]);
       const bool x = (tmax[0] < tmax[1]) & (tmax[0] < tmax[2]);
       const bool y = !x & (tmax[1] < tmax[2]);
       const bool z = !x & !y;
@@ -1887,9 +1992,28 @@ VoxGeom make_vox(const ggh_voxel_solid_desc* d, int solid) {
   G.nxy = d->n_voxels[0] * d->n_voxels[1];
   G.nbx = (G.nx + kBrickX - 1) / kBrickX;
   G.nbxy = G.nbx * ((G.ny + kBrickY - 1) / kBrickY);
+  G.brick_y = (int32_t)(128u * (uint32_t)G.nbx - 32u);
+  G.brick_z = (int32_t)(128u * (uint32_t)G.nbxy - 128u);
   G.mat_offset = d->material_offset;
   G.solid = solid;
   return G;
+}
+
+// Whether voxel steps may take the quick geometry (quick_grid) and, for every
+// point inside the borders' tolerance, a voxel index without a check: the
+// index grows with the coordinate, so the two ends say it for all.
+bool grid_is_quick(const DevSolid& s) {
+  const VoxGeom& G = s.vox;
+  const int n[3] = {G.nx, G.ny, G.nz};
+  if (!quick_grid(G.lo, G.vs, n)) return false;
+  const float lo[3] = {G.lo.x, G.lo.y, G.lo.z}, vs[3] = {G.vs.x, G.vs.y, G.vs.z}, rvs[3] = {G.rvs.x, G.rvs.y, G.rvs.z};
+  const float in_lo[3] = {G.in_lo.x, G.in_lo.y, G.in_lo.z}, in_hi[3] = {G.in_hi.x, G.in_hi.y, G.in_hi.z};
+  for (int a = 0; a < 3; ++a) {
+    const float first = in_lo[a] - lo[a], last = in_hi[a] - lo[a];
+    if (!(first > 0.0f) || !(last >= first)) return false;
+    if ((int)div_rn(last, vs[a], rvs[a]) >= n[a]) return false;
+  }
+  return true;
 }
 
 int n_solids_of(const ggh_context* c, int32_t type) {
@@ -2137,7 +2261,11 @@ int pick_launch(ggh_context* c, uint64_t slots, bool acq, Launch& L) {
   // exchange area of the block's regrouping
   const size_t xchg = regroup ? kXchgBytes : 0;
   const size_t lds = (tables_lds_bytes(c) + 15) & ~(size_t)15;
-  const bool use_lds = lds <= (size_t)kLdsBudget && lds + xchg <= (size_t)c->max_lds;
+  // voxels thinner than the quick geometry takes, or too far out: the general
+  // steps, built once, with the tables in memory
+  bool thin = false;
+  for (const DevSolid& s : c->solids) thin |= s.type == kVoxel && !grid_is_quick(s);
+  const bool use_lds = lds <= (size_t)kLdsBudget && lds + xchg <= (size_t)c->max_lds && !thin;
   if (xchg > (size_t)c->max_lds) return fail(-3, "the block's lane-state exchange area does not fit in LDS");
   // three activated processes, tables in LDS, no fluence tracking: the
   // specialised variant for one voxel solid, else its several-solid form
@@ -2148,7 +2276,12 @@ int pick_launch(ggh_context* c, uint64_t slots, bool acq, Launch& L) {
   // tau sampling changes only the voxel step: scenes without a voxel solid
   // run the plain variants
   const bool tau = c->tau_mode != 0 && regroup;
-  if (special && tau)
+  if (thin)
+    L.fn = acq ? (tau ? transport_kernel<-1, false, false, true, true, true, true, true>
+                      : transport_kernel<-1, false, false, true, true, true, false, true>)
+               : (tau ? transport_kernel<-1, false, false, true, false, true, true, true>
+                      : transport_kernel<-1, false, false, true, false, true, false, true>);
+  else if (special && tau)
     L.fn = acq ? transport_kernel<3, true, true, false, true, true, true>
                : transport_kernel<3, true, true, false, false, true, true>;
   else if (special)
@@ -3299,6 +3432,38 @@ void ggh_host_energy_bin(const float* e, size_t n, const float* ebins, int32_t n
   float l2min, inv;
   energy_bin_guess(eb, l2min, inv);
   for (size_t i = 0; i < n; ++i) out[i] = energy_bin(e[i], ebins, nbins, l2min, inv);
+}
+
+int ggh_host_voxel_exit(const float* p, const float* d, size_t n, const float* lo, const float* voxel,
+                        const int32_t* dims, float* general, float* quick) {
+  ggh_voxel_solid_desc desc;
+  std::memset(&desc, 0, sizeof desc);
+  for (int a = 0; a < 3; ++a) {
+    desc.obb.border_min[a] = lo[a];
+    desc.obb.border_max[a] = lo[a] + (float)dims[a] * voxel[a];
+    desc.n_voxels[a] = dims[a];
+    desc.voxel_size[a] = voxel[a];
+  }
+  DevSolid s;
+  std::memset(&s, 0, sizeof s);
+  s.vox = make_vox(&desc, 0);
+  for (size_t i = 0; i < n; ++i) {
+    Ray r;
+    r.set(mk(d[3 * i], d[3 * i + 1], d[3 * i + 2]));
+    const f3 q = mk(p[3 * i], p[3 * i + 1], p[3 * i + 2]);
+    int vx, vy, vz;
+    const bool in = in_bounds(q, s.vox) && voxel_of(q, s.vox, vx, vy, vz);
+    for (int k = 0; k < 4; ++k) general[4 * i + k] = quick[4 * i + k] = 0.0f;
+    if (!in) continue;
+    const Box b = voxel_box(s.vox, vx, vy, vz);
+    f3 a = q;
+    safety_inside(a, b);
+    const f3 c = inside_quick(q, b);
+    const float out[8] = {a.x, a.y, a.z, distance_to_aabb(a, r, b), c.x, c.y, c.z, exit_quick(c, r, b)};
+    std::memcpy(general + 4 * i, out, 4 * sizeof(float));
+    std::memcpy(quick + 4 * i, out + 4, 4 * sizeof(float));
+  }
+  return grid_is_quick(s) ? 1 : 0;
 }
 
 void ggh_host_distance_to_aabb(const float* p, const float* d, const float* box, float* out, size_t n) {

@@ -117,6 +117,7 @@ def library():
             "ggh_host_uniform_from_sum": ([vp, vp, C.c_size_t], None),
             "ggh_host_div_rn": ([vp, vp, vp, C.c_size_t], None),
             "ggh_host_distance_to_aabb": ([vp, vp, vp, vp, C.c_size_t], None),
+            "ggh_host_voxel_exit": ([vp, vp, C.c_size_t, vp, vp, vp, vp, vp], C.c_int),
             "ggh_host_energy_bin": ([vp, C.c_size_t, vp, C.c_int32, vp], None),
             "ggh_set_launch": ([vp, C.POINTER(LaunchDesc)], C.c_int),
             "ggh_last_grid": ([vp, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)], C.c_int),
@@ -184,6 +185,19 @@ def host_distance_to_aabb(p, d, box):
     out = np.empty(p.shape[0], np.float32)
     library().ggh_host_distance_to_aabb(_ptr(p), _ptr(d), _ptr(box), _ptr(out), p.shape[0])
     return out
+
+
+def host_voxel_exit(p, d, lo, voxel, dims):
+    """The voxel step's nudged point and boundary distance, host build: (general
+    [n, 4], quick [n, 4], whether the engine takes the quick form on this grid)."""
+    p = np.ascontiguousarray(p, np.float32).reshape(-1, 3)
+    d = np.ascontiguousarray(d, np.float32).reshape(-1, 3)
+    lo, voxel = np.asarray(lo, np.float32), np.asarray(voxel, np.float32)
+    dims = np.asarray(dims, np.int32)
+    general, quick = np.empty((len(p), 4), np.float32), np.empty((len(p), 4), np.float32)
+    took = library().ggh_host_voxel_exit(_ptr(p), _ptr(d), len(p), _ptr(lo), _ptr(voxel), _ptr(dims), _ptr(general),
+                                         _ptr(quick))
+    return general, quick, bool(took)
 
 
 def device_count():

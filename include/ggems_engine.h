@@ -360,6 +360,12 @@ void ggh_host_div_rn(const float* a, const float* b, float* out, size_t n);
 /* the engine's energy-bin lookup (BinarySearch on the energy grid,
  * include/GGEMS/maths/GGEMSMathAlgorithms.hh:46-60) for e[0..n-1] */
 void ggh_host_energy_bin(const float* e, size_t n, const float* ebins, int32_t nbins, int32_t* out);
+/* the voxel step's geometry at points p with directions d [n][3] in a grid of
+ * dims voxels from lo: the nudged point and the distance to the voxel's
+ * boundary [n][4], by the general functions and by the quick ones (zeros for
+ * a point outside).  Returns whether the engine takes the quick ones on it. */
+int ggh_host_voxel_exit(const float* p, const float* d, size_t n, const float* lo, const float* voxel,
+                        const int32_t* dims, float* general, float* quick);
 /* the engine's slab test: p, d [n][3], box [n][6] = {min xyz, max xyz} */
 void ggh_host_distance_to_aabb(const float* p, const float* d, const float* box, float* out, size_t n);
 
