@@ -175,7 +175,6 @@ struct RunParams {
   unsigned long long* stats;  // ggh_stats fields
   int32_t round_steps;        // voxel steps a wave makes at least per round
   int32_t cold_passes;        // navigation passes per round
-  int32_t interact_batch;
   uint32_t xchg_offset;       // byte offset of the lane-state exchange area in dynamic LDS
   VoxGeom vox0;               // the only voxel solid, when there is exactly one
   // CT acquisition: projection p places the source at acq_src[p] and box
@@ -1206,6 +1205,12 @@ __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Cou
 // not change any history: a photon carries its slot, its random stream and
 // its counters of work left.
 constexpr int kWaves = kBlock / 64;
+// Voxel steps per pass of the voxel loop: the steps are short, so the pass's
+// ballots and round checks weigh (10^6 photons through 100^3 voxels, 256 x
+// 256 x 128 body, 40-view acquisition: 0.967, 40.3 and 28.6 ms with one,
+// 0.973, 40.0 and 27.0 with two; three gained little more with tau sampling
+// and four was slower).
+constexpr int kPassSteps = 2;
 constexpr size_t kXchgBytes = (size_t)kBlock * 12 * sizeof(uint32_t);
 
 template <bool kTau>
@@ -1365,7 +1370,7 @@ void transport_kernel(RunParams P) {
     // Every wave passes the same barriers in every round, and every loop
     // above is bounded, so the block cannot deadlock.
     uint4* s_x = reinterpret_cast<uint4*>(reinterpret_cast<char*>(s_tab) + P.xchg_offset);
-    __shared__ uint32_t s_cnt[kWaves][kTau ? 3 : 2];
+    __shared__ uint32_t s_cnt[kWaves][3];
     __shared__ uint32_t s_cold_done[2];
     __shared__ uint32_t s_ready[2];
     const int wave = (int)(threadIdx.x >> 6), lane = __lane_id();
@@ -1375,6 +1380,10 @@ void transport_kernel(RunParams P) {
       s_ready[threadIdx.x] = 0;
     }
     __syncthreads();
+    auto one_step = [&](const VoxGeom& G) {
+      return kTau ? hot_step_tau<kTrack, kThin>(P, T, G, L)
+                  : (kThin ? hot_step_thin<NP, kTrack>(P, T, G, L) : hot_step<NP, kTrack>(P, T, G, L));
+    };
     for (uint32_t round = 0;; ++round) {
       const uint32_t rb = round & 1u;
       for (int pass = 0; pass < P.cold_passes; ++pass) {
@@ -1384,7 +1393,7 @@ void transport_kernel(RunParams P) {
       }
       if (lane == 0) atomicAdd(&s_cold_done[rb], 1u);
       bool ready = false;
-      for (int k = 0;; k += kTau ? 2 : 1) {  // k counts voxel steps
+      for (int k = 0;; k += kPassSteps) {  // k counts voxel steps
         const uint64_t act = __ballot(L.mode == kInVoxel);
         if (!ready && (act == 0 || (k >= P.round_steps && lds_load_relaxed(&s_cold_done[rb]) == (uint32_t)kWaves))) {
           ready = true;
@@ -1396,93 +1405,49 @@ void transport_kernel(RunParams P) {
         // solid, else the lane's solid in the (LDS-staged) solid table
         if (L.mode == kInVoxel) {
           const VoxGeom& G = kSingle ? P.vox0 : T.solids[L.solid].vox;
-          stepped = kTau ? hot_step_tau<kTrack, kThin>(P, T, G, L)
-                         : (kThin ? hot_step_thin<NP, kTrack>(P, T, G, L) : hot_step<NP, kTrack>(P, T, G, L));
-          // tau sampling makes two steps per pass: its step is short, so the
-          // pass's ballots and round checks weigh more (measured faster; three
-          // gained little more, four was slower)
-          if (kTau && L.mode == kInVoxel) stepped2 = hot_step_tau<kTrack, kThin>(P, T, G, L);
+          stepped = one_step(G);
+          if (L.mode == kInVoxel) stepped2 = one_step(G);
         }
-        steps += __popcll(__ballot(stepped)) + (kTau ? __popcll(__ballot(stepped2)) : 0);
-        // pending interactions resolved in batches, so that scattered photons
-        // keep stepping without waiting for the next round.  Tau sampling
-        // leaves them to the navigation passes: its voxel loop runs faster
-        // without the interaction code (measured), and its steps are cheap
-        // enough that the waiting lanes cost less.
-        if (!kTau && __popcll(__ballot(L.mode == kInteract)) >= P.interact_batch) {
-          const RunParams& Q = cold_params();
-          if (L.mode == kInteract)
-            resolve_interaction<NP, kTau, kTrack, kThin>(Q, T, kSingle ? Q.vox0 : T.solids[L.solid].vox, L, c);
+        steps += __popcll(__ballot(stepped)) + __popcll(__ballot(stepped2));
+      }
+      // regrouping by event: rank 0 inside a phantom, 1 a pending
+      // interaction, 2 other navigation (exit, cut, new primary or slot),
+      // 3 no work left, so that the next navigation passes run one kind of
+      // event per wave.  Interactions wait for these passes: resolved inside
+      // the voxel loop 16 lanes at a time, as the reference sampling once did,
+      // they took a third of the kernel's instructions on a quarter of the
+      // lanes (256 x 256 x 128 body: 46.6 ms, and 40.0 ms resolved here).
+      const int key = L.mode == kInVoxel ? 0 : (L.mode == kInteract ? 1 : (L.mode != kDone ? 2 : 3));
+      const uint64_t b0 = __ballot(key == 0), b1 = __ballot(key == 1), b2 = __ballot(key == 2);
+      if (lane == 0) {
+        s_cnt[wave][0] = (uint32_t)__popcll(b0);
+        s_cnt[wave][1] = (uint32_t)__popcll(b1);
+        s_cnt[wave][2] = (uint32_t)__popcll(b2);
+      }
+      __syncthreads();
+      uint32_t n0 = 0, n1 = 0, n2 = 0, before0 = 0, before1 = 0, before2 = 0, before3 = 0;
+      for (int w = 0; w < kWaves; ++w) {
+        const uint32_t c0 = s_cnt[w][0], c1 = s_cnt[w][1], c2 = s_cnt[w][2];
+        n0 += c0;
+        n1 += c1;
+        n2 += c2;
+        if (w < wave) {
+          before0 += c0;
+          before1 += c1;
+          before2 += c2;
+          before3 += 64u - c0 - c1 - c2;
         }
       }
-      if constexpr (kTau) {
-        // regrouping by event: rank 0 inside a phantom, 1 a pending
-        // interaction, 2 other navigation (exit, cut, new primary or slot),
-        // 3 no work left, so that the next navigation passes run one kind of
-        // event per wave (measured faster for tau sampling, whose
-        // interactions all wait for these passes; slower for the reference
-        // sampling, which resolves most of them inside the voxel loop)
-        const int key = L.mode == kInVoxel ? 0 : (L.mode == kInteract ? 1 : (L.mode != kDone ? 2 : 3));
-        const uint64_t b0 = __ballot(key == 0), b1 = __ballot(key == 1), b2 = __ballot(key == 2);
-        if (lane == 0) {
-          s_cnt[wave][0] = (uint32_t)__popcll(b0);
-          s_cnt[wave][1] = (uint32_t)__popcll(b1);
-          s_cnt[wave][2] = (uint32_t)__popcll(b2);
-        }
-        __syncthreads();
-        uint32_t n0 = 0, n1 = 0, n2 = 0, before0 = 0, before1 = 0, before2 = 0, before3 = 0;
-        for (int w = 0; w < kWaves; ++w) {
-          const uint32_t c0 = s_cnt[w][0], c1 = s_cnt[w][1], c2 = s_cnt[w][2];
-          n0 += c0;
-          n1 += c1;
-          n2 += c2;
-          if (w < wave) {
-            before0 += c0;
-            before1 += c1;
-            before2 += c2;
-            before3 += 64u - c0 - c1 - c2;
-          }
-        }
-        if (n0 + n1 + n2 == 0) break;  // read from LDS after a barrier: the same for the whole block
-        if (threadIdx.x == 0) {  // the next round's counters; nobody reads them before the barriers below
-          s_cold_done[rb ^ 1u] = 0;
-          s_ready[rb ^ 1u] = 0;
-        }
-        const uint64_t mine = key == 0 ? b0 : (key == 1 ? b1 : (key == 2 ? b2 : ~(b0 | b1 | b2)));
-        const uint32_t pos = (key == 0 ? before0 : (key == 1 ? n0 + before1 : (key == 2 ? n0 + n1 + before2
-                                                                                 : n0 + n1 + n2 + before3))) +
-                             (uint32_t)__popcll(mine & below);
-        exchange_lane<kTau>(L, s_x, pos);
-      } else {
-        // regrouping: rank 0 inside a phantom, 1 stopped, 2 no work left
-        const int key = L.mode == kInVoxel ? 0 : (L.mode != kDone ? 1 : 2);
-        const uint64_t b0 = __ballot(key == 0), b1 = __ballot(key == 1);
-        if (lane == 0) {
-          s_cnt[wave][0] = (uint32_t)__popcll(b0);
-          s_cnt[wave][1] = (uint32_t)__popcll(b1);
-        }
-        __syncthreads();
-        uint32_t n_hot = 0, n_cold = 0, before0 = 0, before1 = 0, before2 = 0;
-        for (int w = 0; w < kWaves; ++w) {
-          const uint32_t h = s_cnt[w][0], cl = s_cnt[w][1];
-          n_hot += h;
-          n_cold += cl;
-          if (w < wave) {
-            before0 += h;
-            before1 += cl;
-            before2 += 64u - h - cl;
-          }
-        }
-        if (n_hot + n_cold == 0) break;  // read from LDS after a barrier: the same for the whole block
-        if (threadIdx.x == 0) {  // the next round's counters; nobody reads them before the barriers below
-          s_cold_done[rb ^ 1u] = 0;
-          s_ready[rb ^ 1u] = 0;
-        }
-        const uint64_t mine = key == 0 ? b0 : (key == 1 ? b1 : ~(b0 | b1));
-        const uint32_t pos = (key == 0 ? before0 : (key == 1 ? n_hot + before1 : n_hot + n_cold + before2)) +
-                             (uint32_t)__popcll(mine & below);
-        exchange_lane<kTau>(L, s_x, pos);
+      if (n0 + n1 + n2 == 0) break;  // read from LDS after a barrier: the same for the whole block
+      if (threadIdx.x == 0) {  // the next round's counters; nobody reads them before the barriers below
+        s_cold_done[rb ^ 1u] = 0;
+        s_ready[rb ^ 1u] = 0;
       }
+      const uint64_t mine = key == 0 ? b0 : (key == 1 ? b1 : (key == 2 ? b2 : ~(b0 | b1 | b2)));
+      const uint32_t pos = (key == 0 ? before0 : (key == 1 ? n0 + before1 : (key == 2 ? n0 + n1 + before2
+                                                                               : n0 + n1 + n2 + before3))) +
+                           (uint32_t)__popcll(mine & below);
+      exchange_lane<kTau>(L, s_x, pos);
     }
   }
 
@@ -1927,8 +1892,8 @@ struct ggh_context {
   DevBuf<uint32_t> queue;
   DevBuf<unsigned long long> stats;
   // launch shape
-  int round_steps = 0;  // 0: 16 with tau sampling, 20 with the reference sampling (measured best)
-  int cold_passes = 0;  // 0: 1 with tau sampling, 2 with the reference sampling (measured best)
+  int round_steps = 0;  // 0: 16 (measured best; 12 and 20 within 2 %, 32 slower by 5 %)
+  int cold_passes = 0;  // 0: 1 (two were 2-5 % slower with the reference sampling)
   int interact_batch = 16;
   int blocks_per_cu = 0;  // 0: as many as fit
   bool force_general = false;
@@ -2075,9 +2040,8 @@ RunParams make_params(ggh_context* c) {
   P.rng_stride = GGH_MAX_SLOTS;
   P.queue = c->queue.p;
   P.stats = c->stats.p;
-  P.round_steps = c->round_steps ? c->round_steps : (c->tau_mode ? 16 : 20);
-  P.cold_passes = c->cold_passes ? c->cold_passes : (c->tau_mode ? 1 : 2);
-  P.interact_batch = c->interact_batch;
+  P.round_steps = c->round_steps ? c->round_steps : 16;
+  P.cold_passes = c->cold_passes ? c->cold_passes : 1;
   P.xchg_offset = 0;
   for (const DevSolid& s : c->solids)
     if (s.type == kVoxel) {
@@ -3150,38 +3114,29 @@ int ggh_autotune(ggh_context* c, uint64_t n_trial, ggh_launch_desc* best) {
   DevBuf<uint32_t> saved;
   if ((rc = dev_alloc(saved, c->rng.n))) return rc;
   HIP_TRY(hipMemcpyAsync(saved.p, c->rng.p, c->rng.n * sizeof(uint32_t), hipMemcpyDeviceToDevice, c->stream));
-  const int keep_round = c->round_steps, keep_cold = c->cold_passes, keep_batch = c->interact_batch,
-            keep_blocks = c->blocks_per_cu;
+  const int keep_round = c->round_steps, keep_blocks = c->blocks_per_cu;
   float best_ms = INFINITY;
   ggh_launch_desc b{};
-  // With the reference sampling the grid is round steps x interaction
-  // batch.  Tau sampling leaves its interactions to the navigation passes,
-  // so the batch does not apply, and it keeps its passes per round (one
-  // pass beat two at full size by less than a short trial's timing noise):
-  // its grid is round steps only, centred on its measured best.
-  const bool tau = c->tau_mode != 0;
+  // One navigation pass per round beat two by less than a short trial's
+  // timing noise in some scenes, so the passes stay: the grid is round steps,
+  // the lengths each sampling mode has always been offered, around their
+  // measured best.
   const int rounds[2][4] = {{12, 20, 32, 0}, {12, 16, 20, 24}};
-  const int batches[3] = {8, 16, 32};
   for (int blocks : {1, 2}) {
-    for (int round : rounds[tau]) {
+    for (int round : rounds[c->tau_mode != 0]) {
       if (round == 0) continue;
-      for (int bi = 0; bi < (tau ? 1 : 3); ++bi) {  // tau sampling: one trial per round length
-        c->blocks_per_cu = blocks;
-        c->round_steps = round;
-        c->interact_batch = tau ? keep_batch : batches[bi];
-        c->cold_passes = keep_cold;
-        HIP_TRY(hipMemcpyAsync(c->rng.p, saved.p, saved.n * sizeof(uint32_t), hipMemcpyDeviceToDevice, c->stream));
-        if ((rc = ggh_run(c, n_trial))) break;
-        if (c->last_ms < best_ms) {
-          best_ms = c->last_ms;
-          b.round_steps = round;
-          b.cold_passes = c->cold_passes;
-          b.interact_batch = c->interact_batch;
-          b.blocks_per_cu = blocks;
-          b.general_kernel = c->force_general ? 1 : 0;
-        }
+      c->blocks_per_cu = blocks;
+      c->round_steps = round;
+      HIP_TRY(hipMemcpyAsync(c->rng.p, saved.p, saved.n * sizeof(uint32_t), hipMemcpyDeviceToDevice, c->stream));
+      if ((rc = ggh_run(c, n_trial))) break;  // a failed trial ends the search with its error
+      if (c->last_ms < best_ms) {
+        best_ms = c->last_ms;
+        b.round_steps = round;
+        b.cold_passes = c->cold_passes;
+        b.interact_batch = c->interact_batch;
+        b.blocks_per_cu = blocks;
+        b.general_kernel = c->force_general ? 1 : 0;
       }
-      if (rc) break;  // a failed trial ends the search with its error
     }
     if (rc) break;
   }
@@ -3191,14 +3146,10 @@ int ggh_autotune(ggh_context* c, uint64_t n_trial, ggh_launch_desc* best) {
   saved.release();
   if (rc || e != hipSuccess) {
     c->round_steps = keep_round;
-    c->cold_passes = keep_cold;
-    c->interact_batch = keep_batch;
     c->blocks_per_cu = keep_blocks;
     return rc ? rc : fail(-100 - (int)e, "autotune: restoring the random streams failed");
   }
   c->round_steps = b.round_steps;
-  c->cold_passes = b.cold_passes;
-  c->interact_batch = b.interact_batch;
   c->blocks_per_cu = b.blocks_per_cu;
   if (best) *best = b;
   return ggh_reset_tallies(c);

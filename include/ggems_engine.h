@@ -166,14 +166,11 @@ int ggh_get_stats(ggh_context* ctx, ggh_stats* out);
  * Zero fields keep the defaults. */
 typedef struct {
   int32_t round_steps;     /* voxel steps a wave makes at least between two regroupings of its
-                              block's photons (1..1024; default 20 with the reference sampling, 16
-                              with tau sampling) */
+                              block's photons (1..1024; default 16) */
   int32_t cold_passes;     /* navigation passes per round for the photons that are not inside a
-                              phantom (1..16; default 2 with the reference sampling, 1 with tau
-                              sampling) */
-  int32_t interact_batch;  /* inside the voxel loop, resolve pending Compton/Rayleigh/photoelectric
-                              interactions once this many lanes wait for one (default 16; 64 leaves
-                              them to the navigation passes) */
+                              phantom (1..16; default 1) */
+  int32_t interact_batch;  /* accepted (0..64) and without effect: interactions are resolved in the
+                              navigation passes */
   int32_t blocks_per_cu;   /* cap on persistent blocks per compute unit (default: as many as fit) */
   int32_t general_kernel;  /* nonzero: the general kernel variant even where the specialised one applies */
 } ggh_launch_desc;
@@ -259,8 +256,7 @@ int ggh_drr(ggh_context* ctx, int solid, int projection, float* image);
 int ggh_drr_noalloc(ggh_context* ctx, int solid, int projection, float* image, void* stream);
 
 /* Launch autotuner: times ggh_run(n_trial) over a grid of launch shapes
- * (blocks per compute unit, round steps, and with the reference sampling the
- * interaction batch) and keeps the fastest.  Call after ggh_seed and before any run: it restores the seeded
+ * (blocks per compute unit, round steps) and keeps the fastest.  Call after ggh_seed and before any run: it restores the seeded
  * random streams and zeroes every tally and counter afterwards. */
 int ggh_autotune(ggh_context* ctx, uint64_t n_trial, ggh_launch_desc* best);
 int ggh_get_dose_tallies(ggh_context* ctx, double* edep, double* edep_squared, int32_t* hit,
