@@ -1389,8 +1389,12 @@ void transport_kernel(RunParams P) {
       for (int pass = 0; pass < P.cold_passes; ++pass) {
         const bool cold = L.mode != kInVoxel && L.mode != kDone;
         if (!__any(cold)) break;
+        // the block's round lasts until these passes are done: they issue first
+        // (256 x 256 x 128 body: 41.3 ms without, 39.5 with)
+        __builtin_amdgcn_s_setprio(3);
         if (cold) cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin>(cold_params(), T, L, c);
       }
+      __builtin_amdgcn_s_setprio(0);
       if (lane == 0) atomicAdd(&s_cold_done[rb], 1u);
       bool ready = false;
       for (int k = 0;; k += kPassSteps) {  // k counts voxel steps
