@@ -32,6 +32,7 @@
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 thread_local std::string g_unet_error;
@@ -220,6 +221,224 @@ __global__ __launch_bounds__(64 * kWaves) void conv_fwd_splitk_kernel(const __bf
     if (relu) v = v > 0.0f ? v : 0.0f;
     const int px = p0 + 16 * i + 4 * g + e;
     y[(size_t)px * Cout + co] = (__bf16)v;
+  }
+}
+
+// The forward convolution of the U-Net's channel counts.  A block takes a tile
+// of 8 x 16 pixels: its input with the halo (10 x 18 pixels, every channel)
+// is loaded into LDS once and serves all nine taps, and each wave multiplies
+// two rows of 16 pixels by 16 NT output channels.  The kernel above fetched
+// every tap's fragment from the caches and divided to find it, which cost
+// about 70 operations for every two fragments.  Here a fragment is one
+// 16-byte LDS read at a constant from the tap; a pixel's channels are padded
+// by 16 bytes, so that eight pixels in a row start in different banks.  The
+// weights pass through LDS in slices of three K steps, double-buffered (one
+// slice where Cin is no multiple of 32 and K is short).  The products of a
+// K step and their order are those of the other kernels, so their outputs are
+// equal bit for bit; with kSplit, the sums are the four of the split-K kernel.
+// The weights multiply from the left, so that a lane ends with four
+// neighbouring channels of one pixel: an 8-byte store.
+// Bound by LDS reads for 16 and 32 output channels and by MFMA issue and the
+// tile's load for the others.  16 x 256 x 256, 48 -> 16 channels: FWD_48_16;
+// 16 x 64 x 64, 192 -> 64: FWD_192_64.
+constexpr int kTileH = 8, kTileW = 16, kHaloW = kTileW + 2, kHaloPix = (kTileH + 2) * kHaloW;
+
+template <int CIN, bool kSplit>
+struct ConvTile {
+  static constexpr int kPixBytes = 2 * CIN + 16;
+  static constexpr int kK = 9 * CIN, kChunks = (kK + 31) / 32;
+  static constexpr int kSlice = CIN % 32 != 0 ? kChunks : (kSplit ? 4 : 3);  // K steps
+  static constexpr int kSlices = (kChunks + kSlice - 1) / kSlice;
+  static constexpr int kRow = kSlice * 32 + 8;                               // bf16 per staged weight row
+  static constexpr int kXBytes = kHaloPix * kPixBytes + 16;                  // the tile, then 16 zero bytes
+  static constexpr int lds(int nt) { return kXBytes + (kSlices > 1 ? 2 : 1) * 16 * nt * kRow * 2; }
+};
+
+// 8 weights of one row from memory, BF16 or rounded from the FP32 masters
+template <bool kF32>
+__device__ inline bf16x8 load_w8(const void* w, size_t at) {
+  if (!kF32) return *reinterpret_cast<const bf16x8*>(static_cast<const __bf16*>(w) + at);
+  const float4* f = reinterpret_cast<const float4*>(static_cast<const float*>(w) + at);
+  const float4 a = f[0], b = f[1];
+  bf16x8 v;
+  v[0] = (__bf16)a.x; v[1] = (__bf16)a.y; v[2] = (__bf16)a.z; v[3] = (__bf16)a.w;
+  v[4] = (__bf16)b.x; v[5] = (__bf16)b.y; v[6] = (__bf16)b.z; v[7] = (__bf16)b.w;
+  return v;
+}
+
+template <int CIN, int NT, bool kSplit, bool kF32>
+__global__ __launch_bounds__(64 * kWaves) void conv_tile_kernel(const __bf16* __restrict__ x,
+                                                                const void* __restrict__ w,
+                                                                const float* __restrict__ bias,
+                                                                __bf16* __restrict__ y, int N, int H, int W, int Cout,
+                                                                int relu) {
+  using T = ConvTile<CIN, kSplit>;
+  constexpr int kCh = 16 * NT, kSums = kSplit ? 4 : 1;
+  extern __shared__ __attribute__((aligned(16))) char s_mem[];
+  __bf16* s_b = reinterpret_cast<__bf16*>(s_mem + T::kXBytes);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tiles_x = W / kTileW, tiles_y = (H + kTileH - 1) / kTileH;
+  const int n_tiles = N * tiles_x * tiles_y;
+  const int bt = xcd_tile(n_tiles);
+  if (bt >= n_tiles) return;  // the whole block: no barrier is skipped
+  const int img = bt / (tiles_x * tiles_y), rest = bt % (tiles_x * tiles_y);
+  const int y0 = rest / tiles_x * kTileH, x0 = rest % tiles_x * kTileW;
+  const int ch_tiles = (Cout + kCh - 1) / kCh;
+  const int r = lane & 15, g = lane >> 4;  // fragment row / k group
+
+  // weights: slice `s` of channel tile `ct`, through registers
+  constexpr int kPieces = kCh * T::kSlice * 4, kPerThread = (kPieces + 64 * kWaves - 1) / (64 * kWaves);
+  bf16x8 next[kPerThread];
+  auto fetch = [&](int ct, int s) {
+#pragma unroll
+    for (int q = 0; q < kPerThread; ++q) {
+      const int t = threadIdx.x + q * 64 * kWaves;
+      const int row = t / (T::kSlice * 4), k = s * T::kSlice * 32 + t % (T::kSlice * 4) * 8;
+      const int co = ct * kCh + row;
+      next[q] = zero8();
+      if (t < kPieces && co < Cout && k < T::kK) next[q] = load_w8<kF32>(w, (size_t)co * T::kK + k);
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < kPerThread; ++q) {
+      const int t = threadIdx.x + q * 64 * kWaves;
+      if (t < kPieces)
+        *reinterpret_cast<bf16x8*>(s_b + (size_t)buf * kCh * T::kRow + t / (T::kSlice * 4) * T::kRow +
+                                   t % (T::kSlice * 4) * 8) = next[q];
+    }
+  };
+  fetch(blockIdx.y, 0);
+  // the input tile
+  constexpr int kXPieces = kHaloPix * (CIN / 8);
+#pragma unroll 6
+  for (int t = threadIdx.x; t < kXPieces; t += 64 * kWaves) {
+    const int p = t / (CIN / 8), c8 = t % (CIN / 8) * 8;
+    const int yy = y0 - 1 + p / kHaloW, xx = x0 - 1 + p % kHaloW;
+    bf16x8 v = zero8();
+    if (yy >= 0 && yy < H && xx >= 0 && xx < W)
+      v = *reinterpret_cast<const bf16x8*>(x + (((size_t)img * H + yy) * W + xx) * CIN + c8);
+    *reinterpret_cast<bf16x8*>(s_mem + p * T::kPixBytes + c8 * 2) = v;
+  }
+  if (threadIdx.x == 0) *reinterpret_cast<bf16x8*>(s_mem + T::kXBytes - 16) = zero8();
+  stage(0);
+  __syncthreads();
+
+  const int base = (2 * wave * kHaloW + r) * T::kPixBytes + (CIN % 32 == 0 ? 16 * g : 0);
+  const int row_y = y0 + 2 * wave;
+  int buf = 0;
+  for (int ct = blockIdx.y; ct < ch_tiles; ct += gridDim.y) {
+    f32x4 acc[kSums][2][NT];
+    for (int m = 0; m < kSums; ++m)
+      for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < NT; ++j) acc[m][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < T::kSlices; ++s) {
+      const bool last = s + 1 == T::kSlices;
+      const bool more = !last || ct + (int)gridDim.y < ch_tiles;
+      if (more && T::kSlices > 1) fetch(last ? ct + gridDim.y : ct, last ? 0 : s + 1);
+#pragma unroll
+      for (int q = 0; q < T::kSlice; ++q) {
+        const int c = s * T::kSlice + q;
+        if (T::kChunks % T::kSlice != 0 && c >= T::kChunks) break;
+        int at;
+        bool tail = false;
+        if (CIN % 32 == 0) {
+          const int tap = 32 * c / CIN;
+          at = base + (tap / 3 * kHaloW + tap % 3) * T::kPixBytes + (32 * c - tap * CIN) * 2;
+        } else {
+          const int k = 32 * c + 8 * g, tap = k / CIN;
+          tail = k >= T::kK;  // K ends inside the step: zeros
+          at = base + (tap / 3 * kHaloW + tap % 3) * T::kPixBytes + (k - tap * CIN) * 2;
+        }
+        bf16x8 a[2], b[NT];
+        for (int i = 0; i < 2; ++i)
+          a[i] = *reinterpret_cast<const bf16x8*>(
+              s_mem + (tail ? T::kXBytes - 16 : at + i * kHaloW * T::kPixBytes));
+        for (int j = 0; j < NT; ++j)
+          b[j] = *reinterpret_cast<const bf16x8*>(s_b + (size_t)buf * kCh * T::kRow + (16 * j + r) * T::kRow + 32 * q +
+                                                  8 * g);
+        for (int i = 0; i < 2; ++i)
+          for (int j = 0; j < NT; ++j)
+            acc[q % kSums][i][j] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[q % kSums][i][j], 0, 0, 0);
+      }
+      if (T::kSlices > 1) {
+        if (more) stage(buf ^ 1);  // nobody reads it during this slice
+        __syncthreads();
+        buf ^= 1;
+      } else if (more) {  // one slice: the next channel tile's weights replace it
+        fetch(ct + gridDim.y, 0);
+        __syncthreads();
+        stage(0);
+        __syncthreads();
+      }
+    }
+    // C fragment: column r (pixel), rows 4 g .. 4 g + 3 (output channels)
+    for (int j = 0; j < NT; ++j) {
+      const int co = ct * kCh + 16 * j + 4 * g;
+      if (co >= Cout) continue;
+      float bb[4];
+      for (int e = 0; e < 4; ++e) bb[e] = bias ? bias[co + e] : 0.0f;
+      for (int i = 0; i < 2; ++i) {
+        if (row_y + i >= H) continue;
+        bf16x4 o;
+        for (int e = 0; e < 4; ++e) {
+          float v = acc[0][i][j][e];
+          for (int m = 1; m < kSums; ++m) v += acc[m][i][j][e];
+          v += bb[e];
+          if (relu) v = v > 0.0f ? v : 0.0f;
+          o[e] = (__bf16)v;
+        }
+        *reinterpret_cast<bf16x4*>(y + (((size_t)img * H + row_y + i) * W + x0 + r) * Cout + co) = o;
+      }
+    }
+  }
+}
+
+template <int CIN, int NT, bool kSplit, bool kF32>
+void launch_tile_nt(const __bf16* x, const void* w, const float* bias, __bf16* y, int n, int h, int wd, int cout,
+                    int relu, hipStream_t st) {
+  const unsigned tiles = (unsigned)(n * (wd / kTileW) * ((h + kTileH - 1) / kTileH));
+  const unsigned ch_tiles = (unsigned)((cout + 16 * NT - 1) / (16 * NT));
+  // channel tiles in one block keep its input tile; a small image spreads them over blocks
+  const unsigned gy = tiles >= 1024 ? 1 : ch_tiles;
+  hipLaunchKernelGGL((conv_tile_kernel<CIN, NT, kSplit, kF32>), dim3((tiles + kXcds - 1) / kXcds * kXcds, gy),
+                     dim3(64 * kWaves), (ConvTile<CIN, kSplit>::lds(NT)), st, x, w, bias, y, n, h, wd, cout, relu);
+}
+
+template <int CIN, bool kSplit, bool kF32>
+void launch_tile_ch(const __bf16* x, const void* w, const float* bias, __bf16* y, int n, int h, int wd, int cout,
+                    int relu, hipStream_t st) {
+  const long long tiles = (long long)n * (wd / kTileW) * ((h + kTileH - 1) / kTileH);
+  int nt = cout % 64 == 0 ? 4 : (cout % 48 == 0 ? 3 : (cout % 32 == 0 ? 2 : 1));
+  // fewer blocks than compute units: fewer channels a block (two suffice for the split sums' registers)
+  while (nt % 2 == 0 && nt > 1 && (tiles * (cout / (16 * nt)) < 256 || (kSplit && nt > 2))) nt /= 2;
+  if (nt == 4) launch_tile_nt<CIN, kSplit ? 2 : 4, kSplit, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
+  else if (nt == 3) launch_tile_nt<CIN, 3, kSplit, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
+  else if (nt == 2) launch_tile_nt<CIN, 2, kSplit, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
+  else launch_tile_nt<CIN, 1, kSplit, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
+}
+
+// launches the tile kernel where there is one for cin; false: the caller takes the general kernels
+template <bool kF32>
+bool launch_tile(const __bf16* x, const void* w, const float* bias, __bf16* y, int n, int h, int wd, int cin, int cout,
+                 int relu, bool split, hipStream_t st) {
+  switch (cin) {
+    case 8: launch_tile_ch<8, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
+    case 16: launch_tile_ch<16, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
+    case 32: launch_tile_ch<32, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
+    case 48: launch_tile_ch<48, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
+    case 64: launch_tile_ch<64, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
+    case 96: launch_tile_ch<96, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
+    case 128:
+      if (split) launch_tile_ch<128, true, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
+      else launch_tile_ch<128, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
+      return true;
+    case 192:
+      if (split) launch_tile_ch<192, true, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
+      else launch_tile_ch<192, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
+      return true;
+    default: return false;
   }
 }
 
@@ -574,7 +793,11 @@ int ggh_conv3x3_forward(const void* x, const void* w, const float* bias, void* y
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const __bf16 *xb = static_cast<const __bf16*>(x), *wb = static_cast<const __bf16*>(w);
   __bf16* yb = static_cast<__bf16*>(y);
-  if (split) {
+  // the tile kernel stores 8 bytes at a time
+  const bool aligned = reinterpret_cast<uintptr_t>(y) % 8 == 0;
+  if (aligned && launch_tile<false>(xb, wb, bias, yb, n, h, wd, cin, cout, relu, split, st)) {
+    // the U-Net's channel counts
+  } else if (split) {
     const dim3 grid((unsigned)((pix_tiles * ch_tiles + kXcds - 1) / kXcds * kXcds));
     hipLaunchKernelGGL(conv_fwd_splitk_kernel, grid, dim3(64 * kWaves), 0, st, xb, wb, bias, yb, n, h, wd, cin, cout,
                        relu);
