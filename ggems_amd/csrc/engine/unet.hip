@@ -24,6 +24,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <string>
 
@@ -239,8 +240,8 @@ __global__ __launch_bounds__(64 * kWaves) void conv_fwd_splitk_kernel(const __bf
 // The weights multiply from the left, so that a lane ends with four
 // neighbouring channels of one pixel: an 8-byte store.
 // Bound by LDS reads for 16 and 32 output channels and by MFMA issue and the
-// tile's load for the others.  16 x 256 x 256, 48 -> 16 channels: FWD_48_16;
-// 16 x 64 x 64, 192 -> 64: FWD_192_64.
+// tile's load for the others.  16 x 256 x 256, 16 -> 16 channels: 43 us before,
+// 21 us; 16 x 64 x 64, 192 -> 64: 84 us before, 43 us (333 TFLOP/s).
 constexpr int kTileH = 8, kTileW = 16, kHaloW = kTileW + 2, kHaloPix = (kTileH + 2) * kHaloW;
 
 template <int CIN, bool kSplit>
@@ -563,6 +564,189 @@ __global__ __launch_bounds__(64 * kWaves) void conv_wgrad_kernel(const __bf16* _
   }
 }
 
+// The weight gradient from tiles.  The kernel above gives each 64 columns
+// (tap, ci) a block of their own, which loads its pixels' dY and one shifted
+// input per tap: dY crosses LDS once per 64 columns and the input nine times.
+// Here a block loads dY of 8 x 16 pixels and the input with its halo once for
+// all nine taps (a tap is an offset of the transposing read), for 16 MT output
+// and 16 CIT input channels; a wave takes two image rows, i.e. one K step of
+// 32 pixels, and keeps all MT x CIT x 9 <= 36 sums in registers over the
+// tiles its block walks.  The waves' sums meet in LDS, and a block adds each
+// weight to memory once.  Staged rows are an odd multiple of 32 bytes, so the
+// four rows that 16 lanes read lie in different banks.  Bound by LDS reads
+// for few output channels (one fragment feeds MT products) and by the tiles'
+// load from L2 otherwise, with the additions to memory on top.  16 x 256 x 256,
+// 48 -> 16 channels: 217 us before, 46 us; 16 x 64 x 64, 192 -> 64: 127 us
+// before, 44 us.
+template <int MT, int CIT, bool kC8>
+struct WgTile {
+  static constexpr int kDyRow = MT == 1 ? 16 : 16 * MT + 16;            // bf16 per staged pixel
+  static constexpr int kXRow = kC8 ? 8 : (CIT % 2 ? 16 * CIT : 16 * CIT + 16);
+  static constexpr int kCols = kC8 ? 5 : 9 * CIT;                        // column tiles of 16
+  static constexpr int kDyBytes = kTileH * kTileW * kDyRow * 2, kXBytes = kHaloPix * kXRow * 2;
+  static constexpr int kSumBytes = MT * kCols * 64 * 16;
+  static constexpr int lds() {
+    return kDyBytes + kXBytes > kSumBytes ? kDyBytes + kXBytes : kSumBytes;
+  }
+};
+
+template <int MT, int CIT, bool kC8>
+__global__ __launch_bounds__(64 * kWaves, 2) void conv_wgrad_tile_kernel(const __bf16* __restrict__ x,
+                                                                         const __bf16* __restrict__ dy,
+                                                                         float* __restrict__ dw, int N, int H, int W,
+                                                                         int Cin, int Cout) {
+  using T = WgTile<MT, CIT, kC8>;
+  constexpr int kCi = kC8 ? 8 : 16 * CIT, kCo = 16 * MT;
+  extern __shared__ __attribute__((aligned(16))) char s_mem[];
+  __bf16* s_dy = reinterpret_cast<__bf16*>(s_mem);
+  __bf16* s_x = reinterpret_cast<__bf16*>(s_mem + T::kDyBytes);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int j = lane & 15, g = lane >> 4;
+  const int co_groups = Cout / kCo;
+  const int co0 = (int)(blockIdx.y % co_groups) * kCo, ci0 = (int)(blockIdx.y / co_groups) * kCi;
+  const int tiles_x = W / kTileW, tiles_y = (H + kTileH - 1) / kTileH;
+  const int n_tiles = N * tiles_x * tiles_y;
+
+  constexpr int kDyPieces = kTileH * kTileW * kCo / 8, kXPieces = kHaloPix * kCi / 8;
+  constexpr int kDyPer = (kDyPieces + 64 * kWaves - 1) / (64 * kWaves);
+  constexpr int kXPer = (kXPieces + 64 * kWaves - 1) / (64 * kWaves);
+  bf16x8 vdy[kDyPer], vx[kXPer];
+  auto fetch = [&](int tile) {
+    const int img = tile / (tiles_x * tiles_y), rest = tile % (tiles_x * tiles_y);
+    const int y0 = rest / tiles_x * kTileH, x0 = rest % tiles_x * kTileW;
+#pragma unroll
+    for (int q = 0; q < kDyPer; ++q) {
+      const int t = threadIdx.x + q * 64 * kWaves;
+      const int p = t / (kCo / 8), c8 = t % (kCo / 8) * 8;
+      const int yy = y0 + p / kTileW, xx = x0 + p % kTileW;
+      vdy[q] = zero8();
+      if (t < kDyPieces && yy < H)
+        vdy[q] = *reinterpret_cast<const bf16x8*>(dy + (((size_t)img * H + yy) * W + xx) * Cout + co0 + c8);
+    }
+#pragma unroll
+    for (int q = 0; q < kXPer; ++q) {
+      const int t = threadIdx.x + q * 64 * kWaves;
+      const int p = t / (kCi / 8), c8 = t % (kCi / 8) * 8;
+      const int yy = y0 - 1 + p / kHaloW, xx = x0 - 1 + p % kHaloW;
+      vx[q] = zero8();
+      if (t < kXPieces && yy >= 0 && yy < H && xx >= 0 && xx < W)
+        vx[q] = *reinterpret_cast<const bf16x8*>(x + (((size_t)img * H + yy) * W + xx) * Cin + ci0 + c8);
+    }
+  };
+  auto store = [&]() {
+#pragma unroll
+    for (int q = 0; q < kDyPer; ++q) {
+      const int t = threadIdx.x + q * 64 * kWaves;
+      if (t < kDyPieces)
+        *reinterpret_cast<bf16x8*>(s_dy + t / (kCo / 8) * T::kDyRow + t % (kCo / 8) * 8) = vdy[q];
+    }
+#pragma unroll
+    for (int q = 0; q < kXPer; ++q) {
+      const int t = threadIdx.x + q * 64 * kWaves;
+      if (t < kXPieces) *reinterpret_cast<bf16x8*>(s_x + t / (kCi / 8) * T::kXRow + t % (kCi / 8) * 8) = vx[q];
+    }
+  };
+  // column tile c of 16 columns: tap and first channel; with 8 channels a
+  // tile holds two taps, whose columns the lanes' addresses tell apart
+  auto x_at = [&](int c) {
+    const int q = j & 3;
+    const int tap = kC8 ? (2 * c + (q >> 1) < 9 ? 2 * c + (q >> 1) : 8) : c / CIT;
+    const int ch = kC8 ? 4 * (q & 1) : 16 * (c % CIT) + 4 * q;
+    return s_x + ((2 * wave + tap / 3) * kHaloW + tap % 3 + 4 * g + (j >> 2)) * T::kXRow + ch;
+  };
+  auto frag = [](const __bf16* p0, const __bf16* p1) {
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p0);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p1);
+    return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+
+  f32x4 acc[MT][T::kCols];
+  for (int i = 0; i < MT; ++i)
+    for (int c = 0; c < T::kCols; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int tile = blockIdx.x;
+  if (tile < n_tiles) fetch(tile);
+  for (; tile < n_tiles; tile += gridDim.x) {
+    store();
+    __syncthreads();
+    if (tile + (int)gridDim.x < n_tiles) fetch(tile + gridDim.x);  // in flight during this tile's products
+    const int y0 = tile % (tiles_x * tiles_y) / tiles_x * kTileH;
+    if (y0 + 2 * wave < H) {  // H is even: both of the wave's rows or none
+      bf16x8 a[MT];
+      for (int i = 0; i < MT; ++i) {
+        const __bf16* p0 = s_dy + (32 * wave + 4 * g + (j >> 2)) * T::kDyRow + 16 * i + 4 * (j & 3);
+        a[i] = frag(p0, p0 + 16 * T::kDyRow);
+      }
+#pragma unroll
+      for (int c = 0; c < T::kCols; ++c) {
+        const __bf16* p0 = x_at(c);
+        const bf16x8 b = frag(p0, p0 + kHaloW * T::kXRow);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b, acc[i][c], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
+  // the waves' sums, one wave after the other, then one addition per weight
+  f32x4* s_sum = reinterpret_cast<f32x4*>(s_mem);
+  for (int w = 0; w < kWaves; ++w) {
+    if (wave == w) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int c = 0; c < T::kCols; ++c) {
+          f32x4* at = s_sum + (i * T::kCols + c) * 64 + lane;
+          *at = w == 0 ? acc[i][c] : *at + acc[i][c];
+        }
+    }
+    __syncthreads();
+  }
+  for (int t = threadIdx.x; t < MT * T::kCols * 64; t += 64 * kWaves) {
+    // C fragment: column j, rows 4 g + e of row tile i
+    const int l = t & 63, i = t / 64 / T::kCols, c = t / 64 % T::kCols;
+    const int col = l & 15;
+    const int tap = kC8 ? 2 * c + (col >> 3) : c / CIT, ch = kC8 ? col & 7 : 16 * (c % CIT) + col;
+    if (tap >= 9) continue;
+    const f32x4 v = s_sum[t];
+    for (int e = 0; e < 4; ++e)
+      unsafeAtomicAdd(&dw[((size_t)(co0 + 16 * i + 4 * (l >> 4) + e) * 9 + tap) * Cin + ci0 + ch], v[e]);
+  }
+}
+
+template <int MT, int CIT, bool kC8>
+void launch_wgrad_tile(const __bf16* x, const __bf16* dy, float* dw, int n, int h, int wd, int cin, int cout,
+                       hipStream_t st) {
+  const int tiles = n * (wd / kTileW) * ((h + kTileH - 1) / kTileH);
+  const int groups = (cout / (16 * MT)) * (kC8 ? 1 : cin / (16 * CIT));
+  // two blocks fit a compute unit; each walks its share of the tiles (more
+  // blocks add each weight more often: 256, 512, 768 and 1,280 blocks take 37, 31,
+  // 36 and 47 us at 16 x 256 x 256, 16 -> 16, and 33, 40, 54 and 78 us at 128 x
+  // 128, 32 -> 32)
+  const int splits = std::max(1, std::min(tiles, 512 / groups));
+  hipLaunchKernelGGL((conv_wgrad_tile_kernel<MT, CIT, kC8>), dim3(splits, groups), dim3(64 * kWaves),
+                     (WgTile<MT, CIT, kC8>::lds()), st, x, dy, dw, n, h, wd, cin, cout);
+}
+
+// false: the general kernel (a height that leaves a wave one row, channels that do not fill a tile)
+bool wgrad_tile(const __bf16* x, const __bf16* dy, float* dw, int n, int h, int wd, int cin, int cout, hipStream_t st) {
+  if (h % 2 || (cin != 8 && cin % 16)) return false;
+  if (cout % 64 == 0) {
+    if (cin == 8) launch_wgrad_tile<4, 1, true>(x, dy, dw, n, h, wd, cin, cout, st);
+    else launch_wgrad_tile<4, 1, false>(x, dy, dw, n, h, wd, cin, cout, st);
+  } else if (cout % 32 == 0) {
+    if (cin == 8) launch_wgrad_tile<2, 1, true>(x, dy, dw, n, h, wd, cin, cout, st);
+    else if (cin % 32 == 0) launch_wgrad_tile<2, 2, false>(x, dy, dw, n, h, wd, cin, cout, st);
+    else launch_wgrad_tile<2, 1, false>(x, dy, dw, n, h, wd, cin, cout, st);
+  } else {
+    if (cin == 8) launch_wgrad_tile<1, 1, true>(x, dy, dw, n, h, wd, cin, cout, st);
+    else if (cin % 64 == 0) launch_wgrad_tile<1, 4, false>(x, dy, dw, n, h, wd, cin, cout, st);
+    else if (cin % 48 == 0) launch_wgrad_tile<1, 3, false>(x, dy, dw, n, h, wd, cin, cout, st);
+    else if (cin % 32 == 0) launch_wgrad_tile<1, 2, false>(x, dy, dw, n, h, wd, cin, cout, st);
+    else launch_wgrad_tile<1, 1, false>(x, dy, dw, n, h, wd, cin, cout, st);
+  }
+  return true;
+}
+
 // The backward of a layer's ReLU and bias in one pass: dy_out = dy where
 // the layer's output y > 0 (everywhere without ReLU), as BF16, and
 // db[c] += sum over pixels of dy_out[., c] in FP32.  A thread takes 8
@@ -860,6 +1044,12 @@ int ggh_conv3x3_weight_grad(const void* x, const void* dy, float* dw, int32_t n,
                             int32_t cout, int32_t splits, void* stream) {
   if (!x || !dy || !dw) return ufail(-1, "null pointer");
   if (!shapes_ok(n, h, wd, cin, cout) || cout > kWgMaxM) return ufail(-2, "unsupported shape (Cout <= 128)");
+  const __bf16 *xb = static_cast<const __bf16*>(x), *db = static_cast<const __bf16*>(dy);
+  if (wgrad_tile(xb, db, dw, n, h, wd, cin, cout, static_cast<hipStream_t>(stream))) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return ufail(-100 - (int)e, std::string("conv weight gradient: ") + hipGetErrorString(e));
+    return 0;
+  }
   const int P = n * h * wd;
   if (splits < 1) splits = 1;
   int per = (P + splits - 1) / splits;
@@ -867,7 +1057,7 @@ int ggh_conv3x3_weight_grad(const void* x, const void* dy, float* dw, int32_t n,
   splits = (P + per - 1) / per;
   const int cols = (9 * cin + kWgN - 1) / kWgN;
   hipLaunchKernelGGL(conv_wgrad_kernel, dim3(cols, splits), dim3(64 * kWaves), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const __bf16*>(x), static_cast<const __bf16*>(dy), dw, n, h, wd, cin, cout, per);
+                     xb, db, dw, n, h, wd, cin, cout, per);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return ufail(-100 - (int)e, std::string("conv weight gradient: ") + hipGetErrorString(e));
   return 0;

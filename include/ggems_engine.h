@@ -299,7 +299,8 @@ const char* ggh_unet_last_error(void);
 int ggh_conv3x3_forward(const void* x, const void* w, const float* bias, void* y, int32_t n, int32_t h, int32_t w_px,
                         int32_t cin, int32_t cout, int32_t relu, void* stream);
 /* dw[cout][9 cin] += sum over pixels of dy (x) shifted x, FP32 (cout <= 128);
- * the pixels are split over `splits` groups of blocks that add atomically */
+ * blocks split the pixels and add atomically; `splits` is the number of pixel
+ * groups for the shapes whose kernel does not choose its own */
 int ggh_conv3x3_weight_grad(const void* x, const void* dy, float* dw, int32_t n, int32_t h, int32_t w_px, int32_t cin,
                             int32_t cout, int32_t splits, void* stream);
 
