@@ -267,12 +267,19 @@ __device__ inline bf16x8 load_w8(const void* w, size_t at) {
   return v;
 }
 
-template <int CIN, int NT, bool kSplit, bool kF32>
+// 8 channels of a gradient behind a ReLU: zero where the layer's output y is not positive
+__device__ inline bf16x8 masked8(bf16x8 v, bf16x8 y) {
+  for (int e = 0; e < 8; ++e) v[e] = (float)y[e] > 0.0f ? v[e] : (__bf16)0.0f;
+  return v;
+}
+
+// kMask: the input is a gradient, masked by the output `mask` of its layer's ReLU as it is loaded
+template <int CIN, int NT, bool kSplit, bool kF32, bool kMask>
 __global__ __launch_bounds__(64 * kWaves) void conv_tile_kernel(const __bf16* __restrict__ x,
                                                                 const void* __restrict__ w,
                                                                 const float* __restrict__ bias,
                                                                 __bf16* __restrict__ y, int N, int H, int W, int Cout,
-                                                                int relu) {
+                                                                int relu, const __bf16* __restrict__ mask) {
   using T = ConvTile<CIN, kSplit>;
   constexpr int kCh = 16 * NT, kSums = kSplit ? 4 : 1;
   extern __shared__ __attribute__((aligned(16))) char s_mem[];
@@ -317,8 +324,11 @@ __global__ __launch_bounds__(64 * kWaves) void conv_tile_kernel(const __bf16* __
     const int p = t / (CIN / 8), c8 = t % (CIN / 8) * 8;
     const int yy = y0 - 1 + p / kHaloW, xx = x0 - 1 + p % kHaloW;
     bf16x8 v = zero8();
-    if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-      v = *reinterpret_cast<const bf16x8*>(x + (((size_t)img * H + yy) * W + xx) * CIN + c8);
+    if (yy >= 0 && yy < H && xx >= 0 && xx < W) {
+      const size_t at = (((size_t)img * H + yy) * W + xx) * CIN + c8;
+      v = *reinterpret_cast<const bf16x8*>(x + at);
+      if (kMask) v = masked8(v, *reinterpret_cast<const bf16x8*>(mask + at));
+    }
     *reinterpret_cast<bf16x8*>(s_mem + p * T::kPixBytes + c8 * 2) = v;
   }
   if (threadIdx.x == 0) *reinterpret_cast<bf16x8*>(s_mem + T::kXBytes - 16) = zero8();
@@ -396,51 +406,74 @@ __global__ __launch_bounds__(64 * kWaves) void conv_tile_kernel(const __bf16* __
   }
 }
 
-template <int CIN, int NT, bool kSplit, bool kF32>
-void launch_tile_nt(const __bf16* x, const void* w, const float* bias, __bf16* y, int n, int h, int wd, int cout,
-                    int relu, hipStream_t st) {
-  const unsigned tiles = (unsigned)(n * (wd / kTileW) * ((h + kTileH - 1) / kTileH));
-  const unsigned ch_tiles = (unsigned)((cout + 16 * NT - 1) / (16 * NT));
+struct ConvArgs {
+  const __bf16* x;
+  const void* w;
+  const float* bias;
+  __bf16* y;
+  int n, h, wd, cin, cout, relu;
+  const __bf16* mask;
+  hipStream_t st;
+};
+
+template <int CIN, int NT, bool kSplit, bool kF32, bool kMask>
+void launch_tile_nt(const ConvArgs& A) {
+  const unsigned tiles = (unsigned)(A.n * (A.wd / kTileW) * ((A.h + kTileH - 1) / kTileH));
+  const unsigned ch_tiles = (unsigned)((A.cout + 16 * NT - 1) / (16 * NT));
   // channel tiles in one block keep its input tile; a small image spreads them over blocks
   const unsigned gy = tiles >= 1024 ? 1 : ch_tiles;
-  hipLaunchKernelGGL((conv_tile_kernel<CIN, NT, kSplit, kF32>), dim3((tiles + kXcds - 1) / kXcds * kXcds, gy),
-                     dim3(64 * kWaves), (ConvTile<CIN, kSplit>::lds(NT)), st, x, w, bias, y, n, h, wd, cout, relu);
+  hipLaunchKernelGGL((conv_tile_kernel<CIN, NT, kSplit, kF32, kMask>), dim3((tiles + kXcds - 1) / kXcds * kXcds, gy),
+                     dim3(64 * kWaves), (ConvTile<CIN, kSplit>::lds(NT)), A.st, A.x, A.w, A.bias, A.y, A.n, A.h, A.wd,
+                     A.cout, A.relu, A.mask);
 }
 
-template <int CIN, bool kSplit, bool kF32>
-void launch_tile_ch(const __bf16* x, const void* w, const float* bias, __bf16* y, int n, int h, int wd, int cout,
-                    int relu, hipStream_t st) {
-  const long long tiles = (long long)n * (wd / kTileW) * ((h + kTileH - 1) / kTileH);
-  int nt = cout % 64 == 0 ? 4 : (cout % 48 == 0 ? 3 : (cout % 32 == 0 ? 2 : 1));
+template <int CIN, bool kSplit, bool kF32, bool kMask>
+void launch_tile_ch(const ConvArgs& A) {
+  const long long tiles = (long long)A.n * (A.wd / kTileW) * ((A.h + kTileH - 1) / kTileH);
+  int nt = A.cout % 64 == 0 ? 4 : (A.cout % 48 == 0 ? 3 : (A.cout % 32 == 0 ? 2 : 1));
   // fewer blocks than compute units: fewer channels a block (two suffice for the split sums' registers)
-  while (nt % 2 == 0 && nt > 1 && (tiles * (cout / (16 * nt)) < 256 || (kSplit && nt > 2))) nt /= 2;
-  if (nt == 4) launch_tile_nt<CIN, kSplit ? 2 : 4, kSplit, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
-  else if (nt == 3) launch_tile_nt<CIN, 3, kSplit, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
-  else if (nt == 2) launch_tile_nt<CIN, 2, kSplit, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
-  else launch_tile_nt<CIN, 1, kSplit, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
+  while (nt % 2 == 0 && nt > 1 && (tiles * (A.cout / (16 * nt)) < 256 || (kSplit && nt > 2))) nt /= 2;
+  if (nt == 4) launch_tile_nt<CIN, kSplit ? 2 : 4, kSplit, kF32, kMask>(A);
+  else if (nt == 3) launch_tile_nt<CIN, 3, kSplit, kF32, kMask>(A);
+  else if (nt == 2) launch_tile_nt<CIN, 2, kSplit, kF32, kMask>(A);
+  else launch_tile_nt<CIN, 1, kSplit, kF32, kMask>(A);
 }
 
-// launches the tile kernel where there is one for cin; false: the caller takes the general kernels
-template <bool kF32>
-bool launch_tile(const __bf16* x, const void* w, const float* bias, __bf16* y, int n, int h, int wd, int cin, int cout,
-                 int relu, bool split, hipStream_t st) {
-  switch (cin) {
-    case 8: launch_tile_ch<8, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
-    case 16: launch_tile_ch<16, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
-    case 32: launch_tile_ch<32, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
-    case 48: launch_tile_ch<48, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
-    case 64: launch_tile_ch<64, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
-    case 96: launch_tile_ch<96, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st); return true;
+// deep layers with few output tiles take four sums over the K steps
+bool split_sums(const ConvArgs& A) {
+  const int pix_tiles = A.n * A.h * A.wd / kFwdPix, ch_tiles = (A.cout + kFwdCh - 1) / kFwdCh;
+  return 9 * A.cin >= 8 * 32 * kWaves && pix_tiles * ch_tiles < 1024;
+}
+
+// launches the tile kernel where there is one for the channel count (a
+// gradient has the count of a layer's output); false: the general kernels
+template <bool kF32, bool kMask>
+bool launch_tile(const ConvArgs& A) {
+  if (reinterpret_cast<uintptr_t>(A.y) % 8) return false;  // it stores 8 bytes at a time
+  const bool split = split_sums(A);
+  switch (A.cin) {
+    case 16: launch_tile_ch<16, false, kF32, kMask>(A); return true;
+    case 32: launch_tile_ch<32, false, kF32, kMask>(A); return true;
+    case 64: launch_tile_ch<64, false, kF32, kMask>(A); return true;
     case 128:
-      if (split) launch_tile_ch<128, true, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
-      else launch_tile_ch<128, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
+      if (split) launch_tile_ch<128, true, kF32, kMask>(A);
+      else launch_tile_ch<128, false, kF32, kMask>(A);
       return true;
-    case 192:
-      if (split) launch_tile_ch<192, true, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
-      else launch_tile_ch<192, false, kF32>(x, w, bias, y, n, h, wd, cout, relu, st);
-      return true;
-    default: return false;
+    default: break;
   }
+  if constexpr (!kMask) {
+    switch (A.cin) {
+      case 8: launch_tile_ch<8, false, kF32, false>(A); return true;
+      case 48: launch_tile_ch<48, false, kF32, false>(A); return true;
+      case 96: launch_tile_ch<96, false, kF32, false>(A); return true;
+      case 192:
+        if (split) launch_tile_ch<192, true, kF32, false>(A);
+        else launch_tile_ch<192, false, kF32, false>(A);
+        return true;
+      default: break;
+    }
+  }
+  return false;
 }
 
 constexpr int kWgPix = 32;   // pixels per K step
@@ -585,16 +618,26 @@ struct WgTile {
   static constexpr int kCols = kC8 ? 5 : 9 * CIT;                        // column tiles of 16
   static constexpr int kDyBytes = kTileH * kTileW * kDyRow * 2, kXBytes = kHaloPix * kXRow * 2;
   static constexpr int kSumBytes = MT * kCols * 64 * 16;
+  static constexpr int kPart = MT * kCols * 256 + 16 * MT;  // floats of a block's sums: weights, then bias
+  // the weight that float k of the sums belongs to, -1 for none: C fragments
+  // of (row tile, column tile), lane, then row 4 (lane / 16) + e, column lane % 16
+  static __host__ __device__ int weight(int k, int cin, int co0, int ci0) {
+    const int e = k & 3, l = k >> 2 & 63, i = k / 256 / kCols, c = k / 256 % kCols, col = l & 15;
+    const int tap = kC8 ? 2 * c + (col >> 3) : c / CIT, ch = kC8 ? col & 7 : 16 * (c % CIT) + col;
+    return tap < 9 ? ((co0 + 16 * i + 4 * (l >> 4) + e) * 9 + tap) * cin + ci0 + ch : -1;
+  }
   static constexpr int lds() {
     return kDyBytes + kXBytes > kSumBytes ? kDyBytes + kXBytes : kSumBytes;
   }
 };
 
-template <int MT, int CIT, bool kC8>
+template <int MT, int CIT, bool kC8, bool kMask>
 __global__ __launch_bounds__(64 * kWaves, 2) void conv_wgrad_tile_kernel(const __bf16* __restrict__ x,
                                                                          const __bf16* __restrict__ dy,
                                                                          float* __restrict__ dw, int N, int H, int W,
-                                                                         int Cin, int Cout) {
+                                                                         int Cin, int Cout,
+                                                                         const __bf16* __restrict__ mask,
+                                                                         float* __restrict__ part) {
   using T = WgTile<MT, CIT, kC8>;
   constexpr int kCi = kC8 ? 8 : 16 * CIT, kCo = 16 * MT;
   extern __shared__ __attribute__((aligned(16))) char s_mem[];
@@ -610,7 +653,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void conv_wgrad_tile_kernel(const _
   constexpr int kDyPieces = kTileH * kTileW * kCo / 8, kXPieces = kHaloPix * kCi / 8;
   constexpr int kDyPer = (kDyPieces + 64 * kWaves - 1) / (64 * kWaves);
   constexpr int kXPer = (kXPieces + 64 * kWaves - 1) / (64 * kWaves);
-  bf16x8 vdy[kDyPer], vx[kXPer];
+  bf16x8 vdy[kDyPer], vmask[kMask ? kDyPer : 1], vx[kXPer];
+  // the bias gradient: a thread's pieces of dY are the same 8 channels every time
+  static_assert(64 * kWaves % (kCo / 8) == 0, "a thread keeps its 8 channels");
+  float bias_sum[8];
+  for (int e = 0; e < 8; ++e) bias_sum[e] = 0.0f;
   auto fetch = [&](int tile) {
     const int img = tile / (tiles_x * tiles_y), rest = tile % (tiles_x * tiles_y);
     const int y0 = rest / tiles_x * kTileH, x0 = rest % tiles_x * kTileW;
@@ -620,8 +667,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void conv_wgrad_tile_kernel(const _
       const int p = t / (kCo / 8), c8 = t % (kCo / 8) * 8;
       const int yy = y0 + p / kTileW, xx = x0 + p % kTileW;
       vdy[q] = zero8();
-      if (t < kDyPieces && yy < H)
-        vdy[q] = *reinterpret_cast<const bf16x8*>(dy + (((size_t)img * H + yy) * W + xx) * Cout + co0 + c8);
+      if (t < kDyPieces && yy < H) {
+        const size_t at = (((size_t)img * H + yy) * W + xx) * Cout + co0 + c8;
+        vdy[q] = *reinterpret_cast<const bf16x8*>(dy + at);
+        if (kMask) vmask[q] = *reinterpret_cast<const bf16x8*>(mask + at);
+      }
     }
 #pragma unroll
     for (int q = 0; q < kXPer; ++q) {
@@ -637,8 +687,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void conv_wgrad_tile_kernel(const _
 #pragma unroll
     for (int q = 0; q < kDyPer; ++q) {
       const int t = threadIdx.x + q * 64 * kWaves;
-      if (t < kDyPieces)
+      if (t < kDyPieces) {
+        if (kMask) vdy[q] = masked8(vdy[q], vmask[q]);
         *reinterpret_cast<bf16x8*>(s_dy + t / (kCo / 8) * T::kDyRow + t % (kCo / 8) * 8) = vdy[q];
+        if (part)
+          for (int e = 0; e < 8; ++e) bias_sum[e] += (float)vdy[q][e];
+      }
     }
 #pragma unroll
     for (int q = 0; q < kXPer; ++q) {
@@ -701,48 +755,119 @@ __global__ __launch_bounds__(64 * kWaves, 2) void conv_wgrad_tile_kernel(const _
     }
     __syncthreads();
   }
+  if (part) {
+    // this block's sums, for wgrad_sum_kernel
+    float* mine = part + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * T::kPart;
+    for (int t = threadIdx.x; t < MT * T::kCols * 64; t += 64 * kWaves) reinterpret_cast<f32x4*>(mine)[t] = s_sum[t];
+    for (int off = 32; off >= kCo / 8; off >>= 1)
+      for (int e = 0; e < 8; ++e) bias_sum[e] += __shfl_xor(bias_sum[e], off, 64);
+    __syncthreads();
+    float* s_bias = reinterpret_cast<float*>(s_mem);
+    if (lane < kCo / 8)
+      for (int e = 0; e < 8; ++e) s_bias[wave * kCo + lane * 8 + e] = bias_sum[e];
+    __syncthreads();
+    if (threadIdx.x < kCo)
+      mine[MT * T::kCols * 256 + threadIdx.x] = (s_bias[threadIdx.x] + s_bias[kCo + threadIdx.x]) +
+                                                (s_bias[2 * kCo + threadIdx.x] + s_bias[3 * kCo + threadIdx.x]);
+    return;
+  }
   for (int t = threadIdx.x; t < MT * T::kCols * 64; t += 64 * kWaves) {
-    // C fragment: column j, rows 4 g + e of row tile i
-    const int l = t & 63, i = t / 64 / T::kCols, c = t / 64 % T::kCols;
-    const int col = l & 15;
-    const int tap = kC8 ? 2 * c + (col >> 3) : c / CIT, ch = kC8 ? col & 7 : 16 * (c % CIT) + col;
-    if (tap >= 9) continue;
     const f32x4 v = s_sum[t];
-    for (int e = 0; e < 4; ++e)
-      unsafeAtomicAdd(&dw[((size_t)(co0 + 16 * i + 4 * (l >> 4) + e) * 9 + tap) * Cin + ci0 + ch], v[e]);
+    for (int e = 0; e < 4; ++e) {
+      const int at = T::weight(4 * t + e, Cin, co0, ci0);
+      if (at >= 0) unsafeAtomicAdd(&dw[at], v[e]);
+    }
   }
 }
 
+// The blocks' sums into dw and db: thread k of a group's sums adds kSumRun
+// blocks in order, and one addition to memory takes the place of kSumRun.
+// (Added by the blocks themselves, the weights of a layer met up to 512 times
+// at the same addresses, and that took longer than the products.)
+constexpr int kSumBlock = 256, kSumRun = 32;
 template <int MT, int CIT, bool kC8>
-void launch_wgrad_tile(const __bf16* x, const __bf16* dy, float* dw, int n, int h, int wd, int cin, int cout,
-                       hipStream_t st) {
-  const int tiles = n * (wd / kTileW) * ((h + kTileH - 1) / kTileH);
-  const int groups = (cout / (16 * MT)) * (kC8 ? 1 : cin / (16 * CIT));
-  // two blocks fit a compute unit; each walks its share of the tiles (more
-  // blocks add each weight more often: 256, 512, 768 and 1,280 blocks take 37, 31,
-  // 36 and 47 us at 16 x 256 x 256, 16 -> 16, and 33, 40, 54 and 78 us at 128 x
-  // 128, 32 -> 32)
-  const int splits = std::max(1, std::min(tiles, 512 / groups));
-  hipLaunchKernelGGL((conv_wgrad_tile_kernel<MT, CIT, kC8>), dim3(splits, groups), dim3(64 * kWaves),
-                     (WgTile<MT, CIT, kC8>::lds()), st, x, dy, dw, n, h, wd, cin, cout);
+__global__ __launch_bounds__(kSumBlock) void wgrad_sum_kernel(const float* __restrict__ part, int splits,
+                                                              float* __restrict__ dw, float* __restrict__ db, int Cin,
+                                                              int Cout) {
+  using T = WgTile<MT, CIT, kC8>;
+  const int k = blockIdx.x * kSumBlock + threadIdx.x;
+  if (k >= T::kPart) return;
+  const int co_groups = Cout / (16 * MT), group = blockIdx.z;
+  const int co0 = group % co_groups * 16 * MT, ci0 = group / co_groups * (kC8 ? 8 : 16 * CIT);
+  const int first = blockIdx.y * kSumRun, last = min(splits, first + kSumRun);
+  const float* at = part + ((size_t)group * splits + first) * T::kPart + k;
+  float sum = 0.0f;
+#pragma unroll 8
+  for (int s = first; s < last; ++s, at += T::kPart) sum += *at;
+  constexpr int kWeights = MT * T::kCols * 256;
+  if (k >= kWeights) {
+    if (ci0 == 0) unsafeAtomicAdd(&db[co0 + k - kWeights], sum);
+  } else {
+    const int w = T::weight(k, Cin, co0, ci0);
+    if (w >= 0) unsafeAtomicAdd(&dw[w], sum);
+  }
+}
+
+struct WgradArgs {
+  const __bf16 *x, *dy;
+  float* dw;
+  int n, h, wd, cin, cout;
+  const __bf16* mask;  // the layer's output behind its ReLU, or null
+  float *db, *part;    // the bias gradient and the blocks' sums, or null: blocks add to dw
+  hipStream_t st;
+};
+
+template <int MT, int CIT, bool kC8>
+int wgrad_splits(const WgradArgs& A, int* groups) {
+  const int tiles = A.n * (A.wd / kTileW) * ((A.h + kTileH - 1) / kTileH);
+  *groups = (A.cout / (16 * MT)) * (kC8 ? 1 : A.cin / (16 * CIT));
+  // each block walks its share of the tiles.  Two blocks of the large variants
+  // fit a compute unit; one with 9 sums or fewer leaves room for four (512 and
+  // 1,024 blocks: 25.2 and 22.9 us at 16 x 256 x 256, 16 -> 16, but 20 and 30 us
+  // at 128 x 128, 32 -> 32)
+  return std::max(1, std::min(tiles, (MT * WgTile<MT, CIT, kC8>::kCols <= 9 ? 1024 : 512) / *groups));
+}
+
+// launches the kernels; with `floats`, only says how much `part` must hold
+template <int MT, int CIT, bool kC8>
+void launch_wgrad_tile(const WgradArgs& A, size_t* floats) {
+  int groups;
+  const int splits = wgrad_splits<MT, CIT, kC8>(A, &groups);
+  using T = WgTile<MT, CIT, kC8>;
+  if (floats) {
+    *floats = (size_t)groups * splits * T::kPart;
+    return;
+  }
+  const dim3 grid(splits, groups), block(64 * kWaves);
+  if (A.mask)
+    hipLaunchKernelGGL((conv_wgrad_tile_kernel<MT, CIT, kC8, true>), grid, block, T::lds(), A.st, A.x, A.dy, A.dw, A.n,
+                       A.h, A.wd, A.cin, A.cout, A.mask, A.part);
+  else
+    hipLaunchKernelGGL((conv_wgrad_tile_kernel<MT, CIT, kC8, false>), grid, block, T::lds(), A.st, A.x, A.dy, A.dw,
+                       A.n, A.h, A.wd, A.cin, A.cout, A.mask, A.part);
+  if (A.part)
+    hipLaunchKernelGGL((wgrad_sum_kernel<MT, CIT, kC8>),
+                       dim3((T::kPart + kSumBlock - 1) / kSumBlock, (splits + kSumRun - 1) / kSumRun, groups),
+                       dim3(kSumBlock), 0, A.st, A.part, splits, A.dw, A.db, A.cin, A.cout);
 }
 
 // false: the general kernel (a height that leaves a wave one row, channels that do not fill a tile)
-bool wgrad_tile(const __bf16* x, const __bf16* dy, float* dw, int n, int h, int wd, int cin, int cout, hipStream_t st) {
-  if (h % 2 || (cin != 8 && cin % 16)) return false;
+bool wgrad_tile(const WgradArgs& A, size_t* floats = nullptr) {
+  const int cin = A.cin, cout = A.cout;
+  if (A.h % 2 || (cin != 8 && cin % 16)) return false;
   if (cout % 64 == 0) {
-    if (cin == 8) launch_wgrad_tile<4, 1, true>(x, dy, dw, n, h, wd, cin, cout, st);
-    else launch_wgrad_tile<4, 1, false>(x, dy, dw, n, h, wd, cin, cout, st);
+    if (cin == 8) launch_wgrad_tile<4, 1, true>(A, floats);
+    else launch_wgrad_tile<4, 1, false>(A, floats);
   } else if (cout % 32 == 0) {
-    if (cin == 8) launch_wgrad_tile<2, 1, true>(x, dy, dw, n, h, wd, cin, cout, st);
-    else if (cin % 32 == 0) launch_wgrad_tile<2, 2, false>(x, dy, dw, n, h, wd, cin, cout, st);
-    else launch_wgrad_tile<2, 1, false>(x, dy, dw, n, h, wd, cin, cout, st);
+    if (cin == 8) launch_wgrad_tile<2, 1, true>(A, floats);
+    else if (cin % 32 == 0) launch_wgrad_tile<2, 2, false>(A, floats);
+    else launch_wgrad_tile<2, 1, false>(A, floats);
   } else {
-    if (cin == 8) launch_wgrad_tile<1, 1, true>(x, dy, dw, n, h, wd, cin, cout, st);
-    else if (cin % 64 == 0) launch_wgrad_tile<1, 4, false>(x, dy, dw, n, h, wd, cin, cout, st);
-    else if (cin % 48 == 0) launch_wgrad_tile<1, 3, false>(x, dy, dw, n, h, wd, cin, cout, st);
-    else if (cin % 32 == 0) launch_wgrad_tile<1, 2, false>(x, dy, dw, n, h, wd, cin, cout, st);
-    else launch_wgrad_tile<1, 1, false>(x, dy, dw, n, h, wd, cin, cout, st);
+    if (cin == 8) launch_wgrad_tile<1, 1, true>(A, floats);
+    else if (cin % 64 == 0) launch_wgrad_tile<1, 4, false>(A, floats);
+    else if (cin % 48 == 0) launch_wgrad_tile<1, 3, false>(A, floats);
+    else if (cin % 32 == 0) launch_wgrad_tile<1, 2, false>(A, floats);
+    else launch_wgrad_tile<1, 1, false>(A, floats);
   }
   return true;
 }
@@ -956,6 +1081,80 @@ __global__ __launch_bounds__(kPrepBlock) void weights_bf16_kernel(const float* _
   }
 }
 
+// The network's input: k <= 8 FP32 channels as BF16, zero-padded to 8.
+__global__ __launch_bounds__(kGlueBlock) void pad8_kernel(const float* __restrict__ x, __bf16* __restrict__ z,
+                                                          long long pixels, int k) {
+  for (long long p = blockIdx.x * (long long)kGlueBlock + threadIdx.x; p < pixels;
+       p += (long long)gridDim.x * kGlueBlock) {
+    bf16x8 v = zero8();
+    for (int c = 0; c < 8; ++c)
+      if (c < k) v[c] = (__bf16)x[p * k + c];
+    *reinterpret_cast<bf16x8*>(z + 8 * p) = v;
+  }
+}
+
+// The 16 -> 1 head in one pass: out = sum_c z_c head_c + bias in FP32, one
+// thread a pixel.  The sixteen products are added in the order the tensor
+// reduction was seen to take (neighbours, then neighbouring pairs), which a
+// test holds bit for bit.  As tensor operations the head wrote and read an FP32 copy of
+// its input twice: 62 us at 16 x 256 x 256, 7.5 us here.
+constexpr int kHeadCh = 16;
+__global__ __launch_bounds__(kGlueBlock) void head_kernel(const __bf16* __restrict__ z, const float* __restrict__ head,
+                                                          const float* __restrict__ bias, float* __restrict__ out,
+                                                          long long pixels) {
+  for (long long p = blockIdx.x * (long long)kGlueBlock + threadIdx.x; p < pixels;
+       p += (long long)gridDim.x * kGlueBlock) {
+    const bf16x8 a = *reinterpret_cast<const bf16x8*>(z + kHeadCh * p);
+    const bf16x8 b = *reinterpret_cast<const bf16x8*>(z + kHeadCh * p + 8);
+    float m[kHeadCh];
+    for (int c = 0; c < 8; ++c) {
+      m[c] = (float)a[c] * head[c];
+      m[8 + c] = (float)b[c] * head[8 + c];
+    }
+#pragma unroll
+    for (int left = kHeadCh / 2; left > 0; left /= 2)
+      for (int c = 0; c < left; ++c) m[c] = m[2 * c] + m[2 * c + 1];
+    out[p] = m[0] + bias[0];
+  }
+}
+
+// Its backward: dz_c = dout head_c rounded to BF16, dhead_c += sum over pixels
+// of dout z_c, dbias += sum of dout.  Four tensor kernels and a reduction
+// before, 125 us at 16 x 256 x 256; 19 us.
+__global__ __launch_bounds__(kGlueBlock) void head_backward_kernel(const float* __restrict__ dout,
+                                                                   const __bf16* __restrict__ z,
+                                                                   const float* __restrict__ head,
+                                                                   __bf16* __restrict__ dz, float* __restrict__ dhead,
+                                                                   float* __restrict__ dbias, long long pixels) {
+  __shared__ float s_sum[kHeadCh + 1][kGlueBlock / 64];
+  float acc[kHeadCh + 1];
+  for (int c = 0; c <= kHeadCh; ++c) acc[c] = 0.0f;
+  for (long long p = blockIdx.x * (long long)kGlueBlock + threadIdx.x; p < pixels;
+       p += (long long)gridDim.x * kGlueBlock) {
+    const float d = dout[p];
+    acc[kHeadCh] += d;
+    for (int h = 0; h < 2; ++h) {
+      const bf16x8 v = *reinterpret_cast<const bf16x8*>(z + kHeadCh * p + 8 * h);
+      bf16x8 o;
+      for (int c = 0; c < 8; ++c) {
+        acc[8 * h + c] += d * (float)v[c];
+        o[c] = (__bf16)(d * head[8 * h + c]);
+      }
+      *reinterpret_cast<bf16x8*>(dz + kHeadCh * p + 8 * h) = o;
+    }
+  }
+  for (int c = 0; c <= kHeadCh; ++c) {
+    for (int off = 32; off > 0; off >>= 1) acc[c] += __shfl_xor(acc[c], off, 64);
+    if ((threadIdx.x & 63) == 0) s_sum[c][threadIdx.x >> 6] = acc[c];
+  }
+  __syncthreads();
+  if (threadIdx.x <= kHeadCh) {
+    float t = 0.0f;
+    for (int w = 0; w < kGlueBlock / 64; ++w) t += s_sum[threadIdx.x][w];
+    unsafeAtomicAdd(threadIdx.x < kHeadCh ? &dhead[threadIdx.x] : dbias, t);
+  }
+}
+
 bool shapes_ok(int N, int H, int W, int Cin, int Cout) {
   return N > 0 && H > 0 && W > 0 && W % 16 == 0 && ((long long)N * H * W) % kFwdPix == 0 && Cin > 0 &&
          Cin % 8 == 0 && Cout > 0 && Cout % 16 == 0 && (long long)N * H * W * (Cin > Cout ? Cin : Cout) < (1ll << 31);
@@ -972,16 +1171,13 @@ int ggh_conv3x3_forward(const void* x, const void* w, const float* bias, void* y
   if (!x || !w || !y) return ufail(-1, "null pointer");
   if (!shapes_ok(n, h, wd, cin, cout)) return ufail(-2, "unsupported shape (W % 16, N H W % 32, Cin % 8, Cout % 16)");
   const int pix_tiles = n * h * wd / kFwdPix, ch_tiles = (cout + kFwdCh - 1) / kFwdCh;
-  // deep layers with few output tiles: split K over the block's waves
-  const bool split = 9 * cin >= 8 * 32 * kWaves && pix_tiles * ch_tiles < 1024;
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const __bf16 *xb = static_cast<const __bf16*>(x), *wb = static_cast<const __bf16*>(w);
   __bf16* yb = static_cast<__bf16*>(y);
-  // the tile kernel stores 8 bytes at a time
-  const bool aligned = reinterpret_cast<uintptr_t>(y) % 8 == 0;
-  if (aligned && launch_tile<false>(xb, wb, bias, yb, n, h, wd, cin, cout, relu, split, st)) {
+  const ConvArgs args = {xb, w, bias, yb, n, h, wd, cin, cout, relu, nullptr, st};
+  if (launch_tile<false, false>(args)) {
     // the U-Net's channel counts
-  } else if (split) {
+  } else if (split_sums(args)) {
     const dim3 grid((unsigned)((pix_tiles * ch_tiles + kXcds - 1) / kXcds * kXcds));
     hipLaunchKernelGGL(conv_fwd_splitk_kernel, grid, dim3(64 * kWaves), 0, st, xb, wb, bias, yb, n, h, wd, cin, cout,
                        relu);
@@ -1045,7 +1241,7 @@ int ggh_conv3x3_weight_grad(const void* x, const void* dy, float* dw, int32_t n,
   if (!x || !dy || !dw) return ufail(-1, "null pointer");
   if (!shapes_ok(n, h, wd, cin, cout) || cout > kWgMaxM) return ufail(-2, "unsupported shape (Cout <= 128)");
   const __bf16 *xb = static_cast<const __bf16*>(x), *db = static_cast<const __bf16*>(dy);
-  if (wgrad_tile(xb, db, dw, n, h, wd, cin, cout, static_cast<hipStream_t>(stream))) {
+  if (wgrad_tile({xb, db, dw, n, h, wd, cin, cout, nullptr, nullptr, nullptr, static_cast<hipStream_t>(stream)})) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return ufail(-100 - (int)e, std::string("conv weight gradient: ") + hipGetErrorString(e));
     return 0;
@@ -1060,6 +1256,83 @@ int ggh_conv3x3_weight_grad(const void* x, const void* dy, float* dw, int32_t n,
                      xb, db, dw, n, h, wd, cin, cout, per);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return ufail(-100 - (int)e, std::string("conv weight gradient: ") + hipGetErrorString(e));
+  return 0;
+}
+
+int ggh_conv3x3_forward_f32w(const void* x, const float* w, const float* bias, void* y, int32_t n, int32_t h,
+                             int32_t wd, int32_t cin, int32_t cout, int32_t relu, void* stream) {
+  if (!x || !w || !y) return ufail(-1, "null pointer");
+  if (!shapes_ok(n, h, wd, cin, cout)) return ufail(-2, "unsupported shape (W % 16, N H W % 32, Cin % 8, Cout % 16)");
+  if (reinterpret_cast<uintptr_t>(w) % 16) return ufail(-2, "weights not 16-byte aligned");
+  const ConvArgs args = {static_cast<const __bf16*>(x), w, bias, static_cast<__bf16*>(y), n, h, wd, cin, cout, relu,
+                         nullptr, static_cast<hipStream_t>(stream)};
+  if (!launch_tile<true, false>(args)) return ufail(-2, "unsupported channel count or output alignment");
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return ufail(-100 - (int)e, std::string("conv forward: ") + hipGetErrorString(e));
+  return 0;
+}
+
+int ggh_unet_pad(const float* x, void* z, int64_t pixels, int32_t k, void* stream) {
+  if (!x || !z) return ufail(-1, "null pointer");
+  if (pixels <= 0 || k < 1 || k > 8) return ufail(-2, "unsupported shape");
+  hipLaunchKernelGGL(pad8_kernel, dim3(glue_grid(pixels)), dim3(kGlueBlock), 0, static_cast<hipStream_t>(stream), x,
+                     static_cast<__bf16*>(z), (long long)pixels, k);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return ufail(-100 - (int)e, std::string("input padding: ") + hipGetErrorString(e));
+  return 0;
+}
+
+int ggh_unet_head(const void* z, const float* head, const float* bias, float* out, int64_t pixels, void* stream) {
+  if (!z || !head || !bias || !out) return ufail(-1, "null pointer");
+  if (pixels <= 0) return ufail(-2, "unsupported shape");
+  hipLaunchKernelGGL(head_kernel, dim3(glue_grid(pixels)), dim3(kGlueBlock), 0, static_cast<hipStream_t>(stream),
+                     static_cast<const __bf16*>(z), head, bias, out, (long long)pixels);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return ufail(-100 - (int)e, std::string("head: ") + hipGetErrorString(e));
+  return 0;
+}
+
+int ggh_unet_head_backward(const float* dout, const void* z, const float* head, void* dz, float* dhead, float* dbias,
+                           int64_t pixels, void* stream) {
+  if (!dout || !z || !head || !dz || !dhead || !dbias) return ufail(-1, "null pointer");
+  if (pixels <= 0) return ufail(-2, "unsupported shape");
+  // two blocks a compute unit: every block ends with an addition per channel to the same addresses
+  const unsigned grid = std::min(glue_grid(pixels), 512u);
+  hipLaunchKernelGGL(head_backward_kernel, dim3(grid), dim3(kGlueBlock), 0, static_cast<hipStream_t>(stream), dout,
+                     static_cast<const __bf16*>(z), head, static_cast<__bf16*>(dz), dhead, dbias, (long long)pixels);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return ufail(-100 - (int)e, std::string("head backward: ") + hipGetErrorString(e));
+  return 0;
+}
+
+size_t ggh_conv3x3_backward_work(int32_t n, int32_t h, int32_t wd, int32_t cin, int32_t cout) {
+  size_t floats = 0;
+  const bool bias = cout == 16 || cout == 32 || cout == 64 || cout == 128;  // as ggh_relu_bias_backward, here from 16
+  if (!bias || !shapes_ok(n, h, wd, cin, cout)) return 0;
+  return wgrad_tile({nullptr, nullptr, nullptr, n, h, wd, cin, cout, nullptr, nullptr, nullptr, nullptr}, &floats)
+             ? floats * sizeof(float)
+             : 0;
+}
+
+int ggh_conv3x3_backward(const void* x, const void* y, const void* dy, const void* wt, void* dx, float* dw, float* db,
+                         float* work, size_t work_bytes, int32_t n, int32_t h, int32_t wd, int32_t cin, int32_t cout,
+                         void* stream) {
+  if (!x || !dy || !dw || !db || !work || (dx && !wt)) return ufail(-1, "null pointer");
+  const size_t need = ggh_conv3x3_backward_work(n, h, wd, cin, cout);
+  if (need == 0 || (dx && cin % 16)) return ufail(-2, "unsupported shape: the layer's gradients one by one");
+  if (work_bytes < need || reinterpret_cast<uintptr_t>(work) % 16 || reinterpret_cast<uintptr_t>(dx) % 8)
+    return ufail(-2, "work space too small or a pointer not aligned");
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  const __bf16 *dyb = static_cast<const __bf16*>(dy), *yb = static_cast<const __bf16*>(y);
+  if (dx) {
+    // the data gradient: the convolution of the masked gradient with the flipped weights
+    const ConvArgs args = {dyb, wt, nullptr, static_cast<__bf16*>(dx), n, h, wd, cout, cin, 0, yb, st};
+    if (yb) launch_tile<false, true>(args);
+    else launch_tile<false, false>(args);
+  }
+  wgrad_tile({static_cast<const __bf16*>(x), dyb, dw, n, h, wd, cin, cout, yb, db, work, st});
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return ufail(-100 - (int)e, std::string("conv backward: ") + hipGetErrorString(e));
   return 0;
 }
 

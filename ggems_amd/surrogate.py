@@ -25,6 +25,7 @@ import math
 
 import numpy as np
 import torch
+import torch.autograd.forward_ad as _fwd
 
 from .engine import EngineError, library
 
@@ -36,6 +37,12 @@ _SIGS = {
     "ggh_relu_bias_backward": ([C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_int64,
                                 C.c_int32, C.c_void_p], C.c_int),
     "ggh_conv3x3_weights_bf16": ([C.c_void_p] * 5 + [C.c_int32, C.c_int32, C.c_void_p], C.c_int),
+    "ggh_conv3x3_backward_work": ([C.c_int32] * 5, C.c_size_t),
+    "ggh_conv3x3_backward": ([C.c_void_p] * 8 + [C.c_size_t] + [C.c_int32] * 5 + [C.c_void_p], C.c_int),
+    "ggh_conv3x3_forward_f32w": ([C.c_void_p] * 4 + [C.c_int32] * 6 + [C.c_void_p], C.c_int),
+    "ggh_unet_pad": ([C.c_void_p, C.c_void_p, C.c_int64, C.c_int32, C.c_void_p], C.c_int),
+    "ggh_unet_head": ([C.c_void_p] * 4 + [C.c_int64, C.c_void_p], C.c_int),
+    "ggh_unet_head_backward": ([C.c_void_p] * 6 + [C.c_int64, C.c_void_p], C.c_int),
     "ggh_pool2x2_forward": ([C.c_void_p, C.c_void_p, C.c_void_p] + [C.c_int32] * 4 + [C.c_void_p], C.c_int),
     "ggh_pool2x2_backward": ([C.c_void_p, C.c_void_p, C.c_void_p] + [C.c_int32] * 4 + [C.c_void_p], C.c_int),
     "ggh_upcat_forward": ([C.c_void_p, C.c_void_p, C.c_void_p] + [C.c_int32] * 5 + [C.c_void_p], C.c_int),
@@ -43,15 +50,19 @@ _SIGS = {
 }
 
 
+_L = None
+
+
 def _lib():
-    L = library()
-    if not getattr(L, "_unet_ready", False):
+    global _L
+    if _L is None:
+        L = library()
         for name, (args, res) in _SIGS.items():
             f = getattr(L, name)
             f.argtypes = args
             f.restype = res
-        L._unet_ready = True
-    return L
+        _L = L
+    return _L
 
 
 def _check(rc):
@@ -60,7 +71,8 @@ def _check(rc):
 
 
 def _stream(t):
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    # the current stream's handle without a Stream object, which costs as much as a launch
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def conv3x3(x, w, bias=None, relu=False):
@@ -114,6 +126,27 @@ def relu_bias_backward(dy, y, relu, db=None):
     return out, db
 
 
+def conv3x3_backward(x, y, dy, wt, want_dx, out):
+    """(dx or None, dw [cout, 9*cin], db) of a layer in one call: dy (BF16)
+    masked where the layer's output y <= 0 (y None: no ReLU), `out` = (dw, db)
+    zeroed by the caller or None; None where the shape takes the single calls"""
+    n, h, wd, cin = x.shape
+    cout = dy.shape[3]
+    size = _lib().ggh_conv3x3_backward_work(n, h, wd, cin, cout)
+    if size == 0 or (want_dx and cin % 16) or dy.dtype != torch.bfloat16:
+        return None
+    x, dy = x.contiguous(), dy.contiguous()
+    y = None if y is None else y.contiguous()
+    dw, db = out if out is not None else (torch.zeros((cout, 9 * cin), dtype=torch.float32, device=x.device),
+                                          torch.zeros(cout, dtype=torch.float32, device=x.device))
+    dx = torch.empty((n, h, wd, cin), dtype=torch.bfloat16, device=x.device) if want_dx else None
+    work = torch.empty(size, dtype=torch.uint8, device=x.device)
+    _check(_lib().ggh_conv3x3_backward(x.data_ptr(), None if y is None else y.data_ptr(), dy.data_ptr(),
+                                       wt.data_ptr(), None if dx is None else dx.data_ptr(), dw.data_ptr(),
+                                       db.data_ptr(), work.data_ptr(), size, n, h, wd, cin, cout, _stream(x)))
+    return dx, dw, db
+
+
 def flip_transpose(w):
     """weights of the data gradient: [cout][9][cin] -> [cin][9][cout], taps reversed"""
     cout, _, cin = w.shape
@@ -133,6 +166,39 @@ def weights_bf16(w, zero=None):
                                            None if dw is None else dw.data_ptr(), None if db is None else db.data_ptr(),
                                            cout, cin, _stream(w)))
     return wb, wt
+
+
+def _untraced():
+    """no forward-mode level and no tracer that would miss a call into the library"""
+    return not (_fwd._current_level >= 0 or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling())
+
+
+def _direct():
+    """whether an operation may skip its autograd function: nothing records it"""
+    return not torch.is_grad_enabled() and _untraced()
+
+
+F32W_CHANNELS = (8, 16, 32, 48, 64, 96, 128, 192)
+F32W_PIXELS = 524288
+
+
+def _conv_layer(x, w, b, relu):
+    """a layer's output without gradients, from its FP32 weights [cout][9][cin].
+    Up to F32W_PIXELS the kernel reads them as they are; for more, its many
+    blocks would each round them, and BF16 ones are made first (the network on
+    1, 8 and 16 views of 256 x 256: 232, 295 and 460 us from FP32, 399, 391 and
+    432 us from BF16)"""
+    cout, _, cin = w.shape
+    if (cin in F32W_CHANNELS and x.numel() // cin <= F32W_PIXELS and w.dtype == torch.float32 and w.is_contiguous()
+            and w.data_ptr() % 16 == 0 and x.dtype == torch.bfloat16 and x.is_cuda and x.shape[3] == cin
+            and (b is None or (b.dtype == torch.float32 and b.is_contiguous()))):
+        x = x.contiguous()
+        n, h, wd, _ = x.shape
+        y = torch.empty((n, h, wd, cout), dtype=torch.bfloat16, device=x.device)
+        _check(_lib().ggh_conv3x3_forward_f32w(x.data_ptr(), w.data_ptr(), None if b is None else b.data_ptr(),
+                                               y.data_ptr(), n, h, wd, cin, cout, int(relu), _stream(x)))
+        return y
+    return conv3x3(x, weights_bf16(w)[0].view(cout, 9 * cin), b, relu)
 
 
 class _Conv3x3(torch.autograd.Function):
@@ -156,8 +222,12 @@ class _Conv3x3(torch.autograd.Function):
     def backward(ctx, dy):
         x, wt, y = ctx.saved_tensors
         cout, cin = ctx.shape
-        dw_buf, db_buf = ctx.zero if ctx.zero is not None else (None, None)
+        out = ctx.zero
         ctx.zero = None  # a second reference would make autograd copy the gradients instead of taking them
+        grads = conv3x3_backward(x, y if ctx.relu else None, dy, wt, ctx.needs_input_grad[0], out)
+        if grads is not None:
+            return grads[0], grads[1].view(cout, 9, cin), grads[2], None
+        dw_buf, db_buf = out if out is not None else (None, None)
         dy, db = relu_bias_backward(dy, y, ctx.relu, db=db_buf)
         dx = None
         if ctx.needs_input_grad[0]:
@@ -175,6 +245,8 @@ class Conv3x3(torch.nn.Module):
         self.relu = relu
 
     def forward(self, x):
+        if _direct():
+            return _conv_layer(x, self.weight, self.bias, self.relu)
         return _Conv3x3.apply(x, self.weight, self.bias, self.relu)
 
 
@@ -248,6 +320,34 @@ class _UpCat(torch.autograd.Function):
         return upcat_backward(dout, ctx.cz)
 
 
+class _Head(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, z, head, bias):
+        ctx.save_for_backward(z, head)
+        return head16(z, head, bias)
+
+    @staticmethod
+    def backward(ctx, dout):
+        z, head = ctx.saved_tensors
+        if torch.is_grad_enabled():  # create_graph: gradients that can be differentiated again
+            d = dout.unsqueeze(3)
+            return (d * head).to(torch.bfloat16), (d * z.float()).sum((0, 1, 2)), dout.sum().reshape(1)
+        dout = dout.contiguous()
+        dz = torch.empty_like(z)
+        sums = torch.zeros(17, dtype=torch.float32, device=z.device)
+        _check(_lib().ggh_unet_head_backward(dout.data_ptr(), z.data_ptr(), head.data_ptr(), dz.data_ptr(),
+                                             sums.data_ptr(), sums.data_ptr() + 64, dout.numel(), _stream(z)))
+        return dz, sums[:16], sums[16:]
+
+
+def head16(z, head, bias):
+    """sum over the 16 channels of z [N,H,W,16] BF16 times head, plus bias -> [N,H,W] FP32"""
+    out = torch.empty(z.shape[:3], dtype=torch.float32, device=z.device)
+    _check(_lib().ggh_unet_head(z.data_ptr(), head.data_ptr(), bias.data_ptr(), out.data_ptr(), out.numel(),
+                                _stream(z)))
+    return out
+
+
 IN_CHANNELS = 8  # the two inputs, zero-padded to the kernels' channel multiple
 
 
@@ -273,20 +373,31 @@ class UNet(torch.nn.Module):
 
     def forward(self, x):
         """x [N, H, W, k <= 8] (any float type) -> [N, H, W] FP32; H, W multiples of 32"""
+        direct = _direct()
         n, h, w, k = x.shape
-        z = torch.zeros((n, h, w, IN_CHANNELS), dtype=torch.bfloat16, device=x.device)
-        z[..., :k] = x.to(torch.bfloat16)
+        if (x.dtype == torch.float32 and x.is_cuda and x.numel() > 0 and k <= IN_CHANNELS
+                and (direct or (not x.requires_grad and _untraced()))):
+            x = x.contiguous()
+            z = torch.empty((n, h, w, IN_CHANNELS), dtype=torch.bfloat16, device=x.device)
+            _check(_lib().ggh_unet_pad(x.data_ptr(), z.data_ptr(), n * h * w, k, _stream(x)))
+        else:
+            z = torch.zeros((n, h, w, IN_CHANNELS), dtype=torch.bfloat16, device=x.device)
+            z[..., :k] = x.to(torch.bfloat16)
         skips = []
         for i, (a, b) in enumerate(self.enc):
             z = b(a(z))
             if i + 1 < len(self.enc):
                 skips.append(z)
-                z = _Pool2x2.apply(z)
+                z = pool2x2(z)[0] if direct else _Pool2x2.apply(z)
         for (a, b), s in zip(self.dec, reversed(skips)):
-            z = b(a(_UpCat.apply(z, s)))
-        # the 16 -> 1 head as a multiply and a channel sum: a matrix-vector
-        # product with 16 columns runs far below HBM speed in the BLAS path
-        return (z.float() * self.head).sum(dim=3) + self.head_bias
+            z = b(a(upcat(z, s) if direct else _UpCat.apply(z, s)))
+        head, bias = self.head, self.head_bias
+        if (z.shape[3] == 16 and z.dtype == torch.bfloat16 and z.is_contiguous() and z.is_cuda
+                and head.dtype == bias.dtype == torch.float32 and head.is_contiguous()):
+            return head16(z, head, bias) if direct else _Head.apply(z, head, bias)
+        # the head as a multiply and a channel sum: a matrix-vector product
+        # with 16 columns runs far below HBM speed in the BLAS path
+        return (z.float() * head).sum(dim=3) + bias
 
 
 def reference_forward(net, x):

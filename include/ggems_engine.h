@@ -318,6 +318,31 @@ int ggh_conv3x3_weights_bf16(const float* w, void* w_bf16, void* wt_bf16, float*
 int ggh_relu_bias_backward(const void* dy, int32_t dy_is_f32, const void* y, int32_t relu, void* dy_out, float* db,
                            int64_t n_pixels, int32_t c, void* stream);
 
+/* ggh_conv3x3_forward from the FP32 weights (16-byte aligned), rounded as they
+ * are read: no ggh_conv3x3_weights_bf16 before it.  Same output bit for bit.
+ * cin one of 8, 16, 32, 48, 64, 96, 128, 192; y 8-byte aligned. */
+int ggh_conv3x3_forward_f32w(const void* x, const float* w, const float* bias, void* y, int32_t n, int32_t h,
+                             int32_t w_px, int32_t cin, int32_t cout, int32_t relu, void* stream);
+/* z [pixels][8] BF16 = x [pixels][k] FP32, zero-padded (k <= 8) */
+int ggh_unet_pad(const float* x, void* z, int64_t pixels, int32_t k, void* stream);
+/* the 16 -> 1 head: out[p] = sum_c z[p][c] head[c] + bias[0], FP32 */
+int ggh_unet_head(const void* z, const float* head, const float* bias, float* out, int64_t pixels, void* stream);
+/* dz = dout head in BF16; dhead[16] and dbias[1] += their gradients */
+int ggh_unet_head_backward(const float* dout, const void* z, const float* head, void* dz, float* dhead, float* dbias,
+                           int64_t pixels, void* stream);
+
+/* all gradients of a layer at once: dy masked by y > 0 as it is loaded (y null:
+ * no ReLU), dx = its data gradient (null: not wanted; wt as
+ * ggh_conv3x3_weights_bf16 gives it), dw and db += the weight and bias
+ * gradients.  dy is BF16.  `work` holds ggh_conv3x3_backward_work() bytes, 16-byte
+ * aligned; 0 bytes: the shape (an odd height, cin neither 8 nor a multiple of
+ * 16, cout not one of 16, 32, 64, 128) takes the calls one by one.  The
+ * data gradient equals theirs bit for bit. */
+size_t ggh_conv3x3_backward_work(int32_t n, int32_t h, int32_t w_px, int32_t cin, int32_t cout);
+int ggh_conv3x3_backward(const void* x, const void* y, const void* dy, const void* wt, void* dx, float* dw, float* db,
+                         float* work, size_t work_bytes, int32_t n, int32_t h, int32_t w_px, int32_t cin, int32_t cout,
+                         void* stream);
+
 /* 2 x 2 max pooling, NHWC BF16 x [n][h][w][c] -> y [n][h/2][w/2][c]; arg
  * (one byte per output element) keeps which input of the window (row-major,
  * 0..3) held the first maximum.  h, w even; c % 8 == 0. */
