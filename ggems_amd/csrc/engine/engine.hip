@@ -210,7 +210,8 @@ enum Mode : int32_t {
   kNeedPrimary = 4,
   kHop = 5,
   kNeedSlot = 6,
-  kDone = 7
+  kDone = 7,
+  kInMesh = 8      // in a meshed solid, looking for its surfaces (kernels without regrouping)
 };
 
 // p and ray hold the local frame of the solid while mode is kInVoxel ..
@@ -806,117 +807,149 @@ __device__ inline bool moller_trumbore(f3 pi, f3 d, const float4& v0, const floa
 // octree nodes; here a BVH in depth-first order with skip links is walked
 // without a stack.  Its boxes are widened on the host so that pruning never
 // drops a triangle the exact test would hit.
-__device__ inline int mesh_hits(const DevSolid& s, f3 p, f3 d, f3& q0, f3& q1) {
-  const f3 inv = mk(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-  int n = 0;
-  float d0 = 0.0f, d1 = 0.0f;
-  int i = 0;
-  while (i < s.n_bvh) {
-    const float4 a = s.bvh[2 * i], b = s.bvh[2 * i + 1];
-    float t1 = (a.x - p.x) * inv.x, t2 = (b.x - p.x) * inv.x;
-    float tmin = fmaxf(0.0f, fminf(t1, t2)), tmax = fmaxf(t1, t2);
-    t1 = (a.y - p.y) * inv.y;
-    t2 = (b.y - p.y) * inv.y;
-    tmin = fmaxf(tmin, fminf(t1, t2));
-    tmax = fminf(tmax, fmaxf(t1, t2));
-    t1 = (a.z - p.z) * inv.z;
-    t2 = (b.z - p.z) * inv.z;
-    tmin = fmaxf(tmin, fminf(t1, t2));
-    tmax = fminf(tmax, fmaxf(t1, t2));
-    if (tmin <= tmax) {
-      const int info = __float_as_int(b.w);
-      const int count = info & 15, first = info >> 4;
-      for (int k = 0; k < count; ++k) {
-        const int t = first + k;
-        f3 q;
-        if (!moller_trumbore(p, d, s.tris[3 * t], s.tris[3 * t + 1], s.tris[3 * t + 2], q)) continue;
-        // DistanceSquare (:101-104)
-        const float d2 = (q.x - p.x) * (q.x - p.x) + (q.y - p.y) * (q.y - p.y) + (q.z - p.z) * (q.z - p.z);
-        ++n;
-        if (n == 1) {
-          q0 = q;
-          d0 = d2;
-        } else if (d2 < d0) {
-          q1 = q0;
-          d1 = d0;
-          q0 = q;
-          d0 = d2;
-        } else if (n == 2 || d2 < d1) {
-          q1 = q;
-          d1 = d2;
-        }
-      }
-      ++i;
-    } else {
-      i = __float_as_int(a.w);
+struct MeshWalk {
+  int32_t i, n;   // next node, hits so far
+  int32_t leaf;   // a leaf whose triangles wait to be tested: first << 4 | count, or 0
+  float d0, d1;   // squared distances of the two nearest
+  f3 q0, q1;
+};
+
+// Visits node w.i and moves on.  False when the ray crosses the box of a leaf
+// while another leaf waits: the walk stands still until that one is tested.
+// (The walk itself does not depend on the hits.)
+__device__ inline bool mesh_visit(const DevSolid& s, f3 p, f3 inv, MeshWalk& w) {
+  const float4 a = s.bvh[2 * w.i], b = s.bvh[2 * w.i + 1];
+  float t1 = (a.x - p.x) * inv.x, t2 = (b.x - p.x) * inv.x;
+  float tmin = fmaxf(0.0f, fminf(t1, t2)), tmax = fmaxf(t1, t2);
+  t1 = (a.y - p.y) * inv.y;
+  t2 = (b.y - p.y) * inv.y;
+  tmin = fmaxf(tmin, fminf(t1, t2));
+  tmax = fminf(tmax, fmaxf(t1, t2));
+  t1 = (a.z - p.z) * inv.z;
+  t2 = (b.z - p.z) * inv.z;
+  tmin = fmaxf(tmin, fminf(t1, t2));
+  tmax = fminf(tmax, fmaxf(t1, t2));
+  const bool in = tmin <= tmax;
+  const int info = __float_as_int(b.w);  // 0 inside the tree
+  const bool leaf = in & (info != 0), held = leaf & (w.leaf != 0);
+  w.leaf = (leaf & !held) ? info : w.leaf;
+  w.i = held ? w.i : (in ? w.i + 1 : __float_as_int(a.w));
+  return !held;
+}
+
+// tests the triangles of the waiting leaf
+__device__ inline void mesh_test(const DevSolid& s, f3 p, f3 d, MeshWalk& w) {
+  const int count = w.leaf & 15, first = w.leaf >> 4;
+  w.leaf = 0;
+  for (int k = 0; k < count; ++k) {
+    const int t = first + k;
+    f3 q;
+    if (!moller_trumbore(p, d, s.tris[3 * t], s.tris[3 * t + 1], s.tris[3 * t + 2], q)) continue;
+    // DistanceSquare (:101-104)
+    const float d2 = (q.x - p.x) * (q.x - p.x) + (q.y - p.y) * (q.y - p.y) + (q.z - p.z) * (q.z - p.z);
+    ++w.n;
+    if (w.n == 1) {
+      w.q0 = q;
+      w.d0 = d2;
+    } else if (d2 < w.d0) {
+      w.q1 = w.q0;
+      w.d1 = w.d0;
+      w.q0 = q;
+      w.d0 = d2;
+    } else if (w.n == 2 || d2 < w.d1) {
+      w.q1 = q;
+      w.d1 = d2;
     }
   }
-  return n;
+}
+
+__device__ inline int mesh_hits(const DevSolid& s, f3 p, f3 d, f3& q0, f3& q1) {
+  const f3 inv = mk(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+  MeshWalk w = {0, 0, 0, 0.0f, 0.0f, q0, q1};
+  while (w.i < s.n_bvh) {
+    mesh_visit(s, p, inv, w);
+    if (w.leaf) mesh_test(s, p, d, w);
+  }
+  q0 = w.q0;
+  q1 = w.q1;
+  return w.n;
 }
 
 // track_through_ggems_meshed_solid (TrackThroughGGEMSMeshSolid.cl:322-534):
 // one material (the navigator's first), global coordinates.  A photon
 // outside the mesh is moved onto its first surface; when no surface is
 // ahead it is projected out of the octree box.
-__device__ void track_mesh(const RunParams& P, const Tabs& T, const DevSolid& s, Lane& L) {
+// One step with the ray's n hits, q0 and q1 the nearest.  False when the
+// photon is done with the solid: no surface ahead, or it died (alive).
+__device__ inline bool mesh_step(const RunParams& P, const Tabs& T, const DevSolid& s, int n, f3 q0, f3 q1, f3& lp,
+                                 f3& ld, Lane& L, bool& alive, unsigned long long& steps,
+                                 unsigned long long& inter) {
+  if (n == 0) return false;
   const int gmat = s.mat_offset;
   const bool dose = L.solid == P.dose_solid;
-  f3 lp = L.p, ld = L.ray.d;
-  bool alive = true;
-  uint32_t steps = 0, inter = 0;
-  for (;;) {
-    f3 q0 = lp, q1 = lp;
-    const int n = mesh_hits(s, lp, ld, q0, q1);
-    if (n == 0) break;
-    f3 next_tri = q0;
-    if ((n & 1) == 0) {
-      lp = q0;
-      next_tri = q1;
-    }
-    float lg[3];
-    draw_logs<-1>(P, L.r, lg);
-    int proc;
-    const int ti = gmat * P.nbins + L.eid;
-    float next = next_interaction<-1>(P, T.sig[ti], T.rcp[ti], lg, proc);
-    ++steps;
-    const float dx = (next_tri.x - lp.x), dy = (next_tri.y - lp.y), dz = (next_tri.z - lp.z);
-    const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
-    if (dist <= next) {
-      next = dist + kTol;
-      proc = kTransportation;
-      if (dose && P.ptrack) {  // dose_photon_tracking at the point of departure
-        const int id = dosel_index(P, lp);
-        if (id >= 0) atomicAdd(&P.ptrack[id], 1);
-      }
-    }
-    lp = add(lp, scl(ld, next));
-    if (proc != kTransportation) {
-      ++inter;
-      const float e0 = L.e;
-      f3 dir = ld;
-      if (!discrete(P, T.ebins, proc, gmat, L.e, L.eid, dir, L.r)) alive = false;
-      if (proc == kCompton || proc == kRayleigh) L.scatter = 1;
-      if (dose) dose_record(P, e0 - L.e, lp);
-      if (proc != kPhotoelectric) {
-        ld = dir;
-        if (L.e != e0) L.eid = energy_bin(L.e, T.ebins, P.nbins, P.ebin_l2min, P.ebin_inv);
-      }
-    }
-    if (L.e <= T.sig[gmat * P.nbins].w) {  // photon_energy_cut_[0]
-      if (dose) dose_record(P, L.e, lp);
-      alive = false;
-    }
-    if (!alive) break;
+  f3 next_tri = q0;
+  if ((n & 1) == 0) {
+    lp = q0;
+    next_tri = q1;
   }
-  // ComputeDistanceToOBB, then the projection out of the box
+  float lg[3];
+  draw_logs<-1>(P, L.r, lg);
+  int proc;
+  const int ti = gmat * P.nbins + L.eid;
+  float next = next_interaction<-1>(P, T.sig[ti], T.rcp[ti], lg, proc);
+  ++steps;
+  const float dx = (next_tri.x - lp.x), dy = (next_tri.y - lp.y), dz = (next_tri.z - lp.z);
+  const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
+  if (dist <= next) {
+    next = dist + kTol;
+    proc = kTransportation;
+    if (dose && P.ptrack) {  // dose_photon_tracking at the point of departure
+      const int id = dosel_index(P, lp);
+      if (id >= 0) atomicAdd(&P.ptrack[id], 1);
+    }
+  }
+  lp = add(lp, scl(ld, next));
+  if (proc != kTransportation) {
+    ++inter;
+    const float e0 = L.e;
+    f3 dir = ld;
+    if (!discrete(P, T.ebins, proc, gmat, L.e, L.eid, dir, L.r)) alive = false;
+    if (proc == kCompton || proc == kRayleigh) L.scatter = 1;
+    if (dose) dose_record(P, e0 - L.e, lp);
+    if (proc != kPhotoelectric) {
+      ld = dir;
+      if (L.e != e0) L.eid = energy_bin(L.e, T.ebins, P.nbins, P.ebin_l2min, P.ebin_inv);
+    }
+  }
+  if (L.e <= T.sig[gmat * P.nbins].w) {  // photon_energy_cut_[0]
+    if (dose) dose_record(P, L.e, lp);
+    alive = false;
+  }
+  return alive;
+}
+
+// ComputeDistanceToOBB, then the projection out of the box
+__device__ inline void leave_mesh(const DevSolid& s, f3 lp, f3 ld, bool alive, Lane& L) {
   Ray r;
   r.set(g2l_dir(s.m, ld));
   const float dist = distance_to_aabb(g2l_pos(s.m, lp), r, s.border);
   L.p = add(lp, scl(ld, dist + kTol));
   L.ray.d = ld;
   L.mode = alive ? kHop : kNeedPrimary;
-  atomicAdd(&P.stats[6], (unsigned long long)steps);
-  atomicAdd(&P.stats[7], (unsigned long long)inter);
+}
+
+__device__ void track_mesh(const RunParams& P, const Tabs& T, const DevSolid& s, Lane& L) {
+  f3 lp = L.p, ld = L.ray.d;
+  bool alive = true;
+  unsigned long long steps = 0, inter = 0;
+  for (;;) {
+    f3 q0 = lp, q1 = lp;
+    const int n = mesh_hits(s, lp, ld, q0, q1);
+    if (!mesh_step(P, T, s, n, q0, q1, lp, ld, L, alive, steps, inter)) break;
+  }
+  leave_mesh(s, lp, ld, alive, L);
+  atomicAdd(&P.stats[6], steps);
+  atomicAdd(&P.stats[7], inter);
 }
 
 // ---------------------------------------------------------------------------
@@ -1107,7 +1140,7 @@ __device__ inline void next_projection(const RunParams& P, Lane& L) {
 
 // the cold work of one lane, one state at a time in an order that lets a
 // lane pass through several states in one call
-template <int NP, bool kSingle, bool kAcq, bool kTau, bool kTrack, bool kThin, class Counters>
+template <int NP, bool kSingle, bool kAcq, bool kTau, bool kTrack, bool kThin, bool kRegroup, class Counters>
 __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Counters& c) {
   if (L.mode == kInteract)
     resolve_interaction<NP, kTau, kTrack, kThin>(P, T, kSingle ? P.vox0 : T.solids[L.solid].vox, L, c);
@@ -1191,7 +1224,8 @@ __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Cou
       // ggh_run launches the single-voxel-solid variant only on scenes
       // without meshes, which keeps the mesh loop (and even this test) out
       // of its register allocation
-      track_mesh(P, T, s, L);
+      if (kRegroup) track_mesh(P, T, s, L);
+      else L.mode = kInMesh;
     } else {
       track_box<kAcq>(P, T, s, L, c);
     }
@@ -1205,6 +1239,15 @@ __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Cou
 // not change any history: a photon carries its slot, its random stream and
 // its counters of work left.
 constexpr int kWaves = kBlock / 64;
+// The walk of meshed scenes (transport_kernel): lanes that must be looking for
+// the wave to go on visiting nodes, and lanes that must be held up by an
+// untested leaf for the wave to test.  10^7 primaries on spheres of 81,920 and
+// 5,120 triangles (ms): 55.0 with a track loop per lane; walkers 56, 48, 32 and
+// 16 with leaves tested as met 79.8, 60.8, 46.7 and 38.2; walkers 16 with 24, 16
+// and 8 leaves together 29.7, 27.5 and 26.5, walkers 8 and 24 with 16 leaves
+// 28.2 and 28.6.  Reading the next node in memory ahead was slower (29.2): the
+// scattered 16-byte reads bound the walk, not their latency.
+constexpr int kMeshWalkers = 16, kMeshLeaves = 8;
 // Voxel steps per pass of the voxel loop: the steps are short, so the pass's
 // ballots and round checks weigh (10^6 photons through 100^3 voxels, 256 x
 // 256 x 128 body, 40-view acquisition: 0.967, 40.3 and 28.6 ms with one,
@@ -1347,12 +1390,71 @@ void transport_kernel(RunParams P) {
   unsigned long long steps = 0;  // wave-uniform
 
   if (!kRegroup) {
-    // no voxel solid, so no lane ever steps voxels: the loop ends when no
-    // lane has navigation or tracking left
+    // No voxel solid, so no lane steps voxels; a lane inside a meshed solid
+    // looks for its surfaces in the BVH.  Photons take different numbers of
+    // mesh steps, and rays meet different numbers of nodes: run to its end by
+    // each lane in turn, a wave's track loop kept most lanes waiting for the
+    // slowest.  Here every lane holds its own place in the tree, the wave
+    // visits nodes while at least kMeshWalkers of its lanes are looking, and
+    // then makes the steps and the navigation of all the others.  The loop
+    // ends when no lane has work left: with no lane looking, every other lane
+    // moves on in each pass.
+    MeshWalk w = {0, 0, 0, 0.0f, 0.0f, L.p, L.p};
+    bool looking = false;
+    unsigned long long mesh_steps = 0, mesh_inter = 0;
     for (;;) {
-      const bool cold = L.mode != kInVoxel && L.mode != kDone;
-      if (!__any(cold)) break;
-      if (cold) cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin>(cold_params(), T, L, c);
+      for (;;) {
+        const uint64_t walkers = __ballot(looking);
+        if (walkers == 0 ||
+            (__popcll(walkers) < kMeshWalkers && __any(!looking && L.mode != kDone))) break;
+        // a leaf's triangle test costs several node tests and few lanes stand at
+        // a leaf at a time: they test together, once kMeshLeaves lanes can go
+        // no further without it (or all who look)
+        bool stuck = false;
+        if (looking) {
+          const DevSolid& s = T.solids[L.solid];
+          stuck = w.i >= s.n_bvh || !mesh_visit(s, L.p, L.ray.inv, w);
+          stuck |= w.i >= s.n_bvh;
+        }
+        const uint64_t held = __ballot(stuck);
+        if (held && (__popcll(held) >= kMeshLeaves || held == walkers)) {
+          if (looking && w.leaf) mesh_test(T.solids[L.solid], L.p, L.ray.d, w);
+          if (stuck) looking = w.i < T.solids[L.solid].n_bvh;
+        }
+      }
+      const RunParams& Q = cold_params();
+      bool fresh = false;
+      if (L.mode == kInMesh && !looking) {
+        const DevSolid& s = T.solids[L.solid];
+        bool alive = true;
+        f3 lp = L.p, ld = L.ray.d;
+        if (mesh_step(Q, T, s, w.n, w.q0, w.q1, lp, ld, L, alive, mesh_steps, mesh_inter)) {
+          L.p = lp;
+          L.ray.d = ld;
+          fresh = true;
+        } else {
+          leave_mesh(s, lp, ld, alive, L);
+        }
+      }
+      const bool cold = L.mode != kInMesh && L.mode != kDone;
+      if (cold) {
+        cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin, kRegroup>(Q, T, L, c);
+        fresh = L.mode == kInMesh;
+      }
+      if (fresh) {  // a new look: from the root, with no hits
+        looking = true;
+        w = MeshWalk{0, 0, 0, 0.0f, 0.0f, L.p, L.p};
+        L.ray.inv = mk(1.0f / L.ray.d.x, 1.0f / L.ray.d.y, 1.0f / L.ray.d.z);
+      }
+      if (!__any(L.mode != kDone)) break;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      mesh_steps += __shfl_xor(mesh_steps, off, 64);
+      mesh_inter += __shfl_xor(mesh_inter, off, 64);
+    }
+    if (__lane_id() == 0 && mesh_steps) {
+      atomicAdd(&P.stats[6], mesh_steps);
+      atomicAdd(&P.stats[7], mesh_inter);
     }
   } else {
     // The block works in rounds.  In each round every wave
@@ -1392,7 +1494,7 @@ void transport_kernel(RunParams P) {
         // the block's round lasts until these passes are done: they issue first
         // (256 x 256 x 128 body: 41.3 ms without, 39.5 with)
         __builtin_amdgcn_s_setprio(3);
-        if (cold) cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin>(cold_params(), T, L, c);
+        if (cold) cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin, kRegroup>(cold_params(), T, L, c);
       }
       __builtin_amdgcn_s_setprio(0);
       if (lane == 0) atomicAdd(&s_cold_done[rb], 1u);
