@@ -176,6 +176,7 @@ struct RunParams {
   int32_t round_steps;        // voxel steps a wave makes at least per round
   int32_t cold_passes;        // navigation passes per round
   uint32_t xchg_offset;       // byte offset of the lane-state exchange area in dynamic LDS
+  int mesh_loop;              // kernels without regrouping: each lane walks its mesh to the end (pick_launch)
   VoxGeom vox0;               // the only voxel solid, when there is exactly one
   // CT acquisition: projection p places the source at acq_src[p] and box
   // solid j at acq_box[p * n_box + j]; its primaries are laid out in
@@ -1224,7 +1225,7 @@ __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Cou
       // ggh_run launches the single-voxel-solid variant only on scenes
       // without meshes, which keeps the mesh loop (and even this test) out
       // of its register allocation
-      if (kRegroup) track_mesh(P, T, s, L);
+      if (kRegroup || P.mesh_loop) track_mesh(P, T, s, L);
       else L.mode = kInMesh;
     } else {
       track_box<kAcq>(P, T, s, L, c);
@@ -1242,12 +1243,19 @@ constexpr int kWaves = kBlock / 64;
 // The walk of meshed scenes (transport_kernel): lanes that must be looking for
 // the wave to go on visiting nodes, and lanes that must be held up by an
 // untested leaf for the wave to test.  10^7 primaries on spheres of 81,920 and
-// 5,120 triangles (ms): 55.0 with a track loop per lane; walkers 56, 48, 32 and
-// 16 with leaves tested as met 79.8, 60.8, 46.7 and 38.2; walkers 16 with 24, 16
-// and 8 leaves together 29.7, 27.5 and 26.5, walkers 8 and 24 with 16 leaves
-// 28.2 and 28.6.  Reading the next node in memory ahead was slower (29.2): the
-// scattered 16-byte reads bound the walk, not their latency.
-constexpr int kMeshWalkers = 16, kMeshLeaves = 8;
+// 5,120 triangles (ms): 54.7 with a track loop per lane; walkers 56, 48 and 32
+// with leaves tested as met 79.8, 60.8 and 46.7; walkers 16 with leaves as met,
+// 24, 16 and 8 together 38.2, 29.7, 27.5 and 26.7; leaves 8 with walkers 8, 6,
+// 4 and 2 25.8, 26.7, 27.5 and 29.7.  Reading the next node in memory ahead was
+// slower (29.2 for 27.5): the scattered 16-byte reads bound the walk, not their
+// latency.
+constexpr int kMeshWalkers = 8, kMeshLeaves = 8;
+// Photons per lane below which a launch takes the track loop of each lane
+// instead: with few photons a lane there is little to even out, and the walk's
+// passes only add to each photon's time.  2 x 10^5, 7 x 10^5, 10^6, 1.5 x 10^6
+// and 2 x 10^6 primaries over 262,144 lanes (ms): loop 0.75, 1.50, 3.57, 4.16
+// and 7.43, walk 1.27, 1.72, 3.12, 4.07 and 5.67.
+constexpr uint64_t kMeshLoopBelow = 4;
 // Voxel steps per pass of the voxel loop: the steps are short, so the pass's
 // ballots and round checks weigh (10^6 photons through 100^3 voxels, 256 x
 // 256 x 128 body, 40-view acquisition: 0.967, 40.3 and 28.6 ms with one,
@@ -1393,7 +1401,8 @@ void transport_kernel(RunParams P) {
     // No voxel solid, so no lane steps voxels; a lane inside a meshed solid
     // looks for its surfaces in the BVH.  Photons take different numbers of
     // mesh steps, and rays meet different numbers of nodes: run to its end by
-    // each lane in turn, a wave's track loop kept most lanes waiting for the
+    // each lane in turn (track_mesh, which launches of few photons a lane still
+    // take: P.mesh_loop), a wave's track loop kept most lanes waiting for the
     // slowest.  Here every lane holds its own place in the tree, the wave
     // visits nodes while at least kMeshWalkers of its lanes are looking, and
     // then makes the steps and the navigation of all the others.  The loop
@@ -2009,6 +2018,7 @@ struct ggh_context {
   // CT acquisition
   int acq_n_proj = 0;
   uint32_t acq_slots = 0;
+  uint64_t acq_primaries = 0;  // of all projections
   DevBuf<Mat34> acq_src, acq_box;
   DevBuf<uint4> acq_layout;
   DevBuf<int32_t> acq_phantom;                      // per projection: the one non-box solid present, or -1
@@ -2149,6 +2159,7 @@ RunParams make_params(ggh_context* c) {
   P.round_steps = c->round_steps ? c->round_steps : 16;
   P.cold_passes = c->cold_passes ? c->cold_passes : 1;
   P.xchg_offset = 0;
+  P.mesh_loop = 0;
   for (const DevSolid& s : c->solids)
     if (s.type == kVoxel) {
       P.vox0 = s.vox;
@@ -2188,6 +2199,7 @@ void drop_acquisition(ggh_context* c) {
   c->acq_scat.clear();
   c->acq_n_proj = 0;
   c->acq_slots = 0;
+  c->acq_primaries = 0;
   c->acq_src_host.clear();
   c->acq_box_host.clear();
 }
@@ -2318,13 +2330,14 @@ struct Launch {
   unsigned grid;
   size_t shmem;
   uint32_t xchg_offset;  // RunParams::xchg_offset of this launch
+  int mesh_loop;         // RunParams::mesh_loop of this launch
 };
 
 // kernel variant and persistent grid: the specialised variant (three
 // activated processes, one voxel solid and no mesh, tables in LDS, no fluence
 // tracking) or the general one, each with or without acquisition placement;
 // block regrouping whenever the scene has a voxel solid to step through
-int pick_launch(ggh_context* c, uint64_t slots, bool acq, Launch& L) {
+int pick_launch(ggh_context* c, uint64_t slots, uint64_t primaries, bool acq, Launch& L) {
   const bool single = n_solids_of(c, kVoxel) == 1 && n_solids_of(c, kMesh) == 0;
   const bool regroup = n_solids_of(c, kVoxel) > 0;
   // dynamic LDS: the staged tables (when they fit), then the lane-state
@@ -2384,6 +2397,7 @@ int pick_launch(ggh_context* c, uint64_t slots, bool acq, Launch& L) {
                                                        L.shmem));
   if (per_cu < 1) return fail(-3, "transport kernel does not fit on a compute unit");
   if (c->blocks_per_cu > 0) per_cu = std::min(per_cu, c->blocks_per_cu);
+  L.mesh_loop = primaries < kMeshLoopBelow * (uint64_t)per_cu * c->n_cu * kBlock;
   // persistent blocks: no more than the slots can keep busy
   const uint64_t max_blocks = (slots + kBlock - 1) / kBlock;
   L.grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)per_cu * c->n_cu, max_blocks));
@@ -2418,8 +2432,9 @@ int acquisition_launch(ggh_context* c, RunParams& P, Launch& L) {
   P.n_proj = c->acq_n_proj;
   P.n_box = n_solids_of(c, kBoxSolid);
   P.n_slots = c->acq_slots;
-  if ((rc = pick_launch(c, c->acq_slots, true, L))) return rc;
+  if ((rc = pick_launch(c, c->acq_slots, c->acq_primaries, true, L))) return rc;
   P.xchg_offset = L.xchg_offset;
+  P.mesh_loop = L.mesh_loop;
   return 0;
 }
 
@@ -2987,8 +3002,9 @@ int ggh_run(ggh_context* c, uint64_t n) {
   P.rem = rem;
   P.n_slots = slots;
   Launch L;
-  if ((rc = pick_launch(c, slots, false, L))) return rc;
+  if ((rc = pick_launch(c, slots, n, false, L))) return rc;
   P.xchg_offset = L.xchg_offset;
+  P.mesh_loop = L.mesh_loop;
   HIP_TRY(hipMemsetAsync(c->queue.p, 0, sizeof(uint32_t), c->stream));
   HIP_TRY(hipEventRecord(c->ev0, c->stream));
   hipLaunchKernelGGL(L.fn, dim3(L.grid), dim3(kBlock), L.shmem, c->stream, P);
@@ -3009,11 +3025,13 @@ int ggh_set_acquisition(ggh_context* c, const ggh_acquisition_desc* d) {
   const int np = d->n_projections;
   std::vector<uint4> lay((size_t)np);
   uint32_t max_slots = 0;
+  uint64_t total = 0;
   for (int p = 0; p < np; ++p) {
     uint32_t nb, base, rem, slots;
     if ((rc = batch_layout(d->n_particles[p], nb, base, rem, slots))) return rc;
     lay[p] = make_uint4(nb, base, rem, 0u);
     max_slots = std::max(max_slots, slots);
+    total += d->n_particles[p];
   }
   std::vector<int32_t> only;
   if (d->phantoms) {
@@ -3049,6 +3067,7 @@ int ggh_set_acquisition(ggh_context* c, const ggh_acquisition_desc* d) {
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->acq_n_proj = np;
   c->acq_slots = max_slots;
+  c->acq_primaries = total;
   return 0;
 }
 

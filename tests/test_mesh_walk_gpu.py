@@ -6,6 +6,7 @@ against the oracle."""
 import numpy as np
 import pytest
 
+import plain_scene
 from ggems_amd import authoring
 from scene import Scene
 
@@ -50,4 +51,34 @@ def test_acquisition_equals_single_runs():
     assert got["stats"]["primaries"] == sum(n)
     for a, b in zip(ref["hist"], got["hist"]):
         assert int(np.abs(a.astype(np.int64) - b).sum()) <= 20 + 0.02 * int(a.sum())
+    eng.close()
+
+
+@pytest.mark.parametrize("meshes", [[(40.0, 0)], [(40.0, 4), (12.0, 2)]])
+def test_few_and_many_photons_a_lane_take_the_same_histories(meshes):
+    """600,000 photons are fewer than four for each lane of the whole card and
+    more than four for each lane of one block per compute unit: the first launch
+    runs each lane's track loop, the second the shared walk."""
+    eng = plain_scene.engine(3)
+    for k, (radius, level) in enumerate(meshes):
+        tri = authoring.icosphere(radius, level).astype(np.float32)
+        half = np.abs(tri).reshape(-1, 3).max(0) + np.float32(1e-3)
+        eng.add_mesh_solid(tri, -half, half, k)
+    panel = plain_scene.add_panel(eng, 32, 32, 4.0, 2)
+    eng.set_dosimetry(0, (4.0, 4.0, 4.0), (20, 20, 20), (-40.0,) * 3, (40.0,) * 3, photon_tracking=True)
+    plain_scene.add_source(eng)
+    got = []
+    for blocks in (0, 1):
+        eng.set_launch(blocks_per_cu=blocks)
+        eng.reset_tallies()
+        eng.seed(77)
+        eng.run(600_000)
+        edep, _, hit, track = eng.dose_tallies()
+        got.append((eng.stats(), eng.histogram(panel)[0], hit, track, edep))
+    a, b = got
+    assert a[0] == b[0] and a[0]["primaries"] == 600_000 and a[0]["mesh_interactions"] > 0
+    for x, y in zip(a[1:4], b[1:4]):
+        assert np.array_equal(x, y)
+    # FP64 sums whose order follows the atomics
+    np.testing.assert_allclose(a[4], b[4], rtol=1e-12, atol=1e-18)
     eng.close()
