@@ -381,19 +381,19 @@ class Engine:
         return counts, scatter
 
     def dose_tallies(self):
-        nx, ny, nz = self.n_dosels
+        nx, ny, nz = self.n_dosels  # arrays unwritten before: the readback is their first touch
         e2, hit, pt = self.dose_flags
-        edep = np.zeros((nz, ny, nx), np.float64)
-        edep2 = np.zeros_like(edep) if e2 else None
-        hits = np.zeros((nz, ny, nx), np.int32) if hit else None
-        ptrack = np.zeros((nz, ny, nx), np.int32) if pt else None
+        edep = np.empty((nz, ny, nx), np.float64)
+        edep2 = np.empty_like(edep) if e2 else None
+        hits = np.empty((nz, ny, nx), np.int32) if hit else None
+        ptrack = np.empty((nz, ny, nx), np.int32) if pt else None
         _check(library().ggh_get_dose_tallies(self.h, _ptr(edep), _ptr(edep2), _ptr(hits), _ptr(ptrack)))
         return edep, edep2, hits, ptrack
 
     def compute_dose(self, scale=1.0, water_reference=False, minimum_density=0.0, uncertainty=True):
         nx, ny, nz = self.n_dosels
-        dose = np.zeros((nz, ny, nx), np.float32)
-        unc = np.zeros_like(dose) if uncertainty else None
+        dose = np.empty((nz, ny, nx), np.float32)
+        unc = np.empty_like(dose) if uncertainty else None
         _check(library().ggh_compute_dose(self.h, float(scale), int(bool(water_reference)), float(minimum_density),
                                           _ptr(dose), _ptr(unc)))
         return dose, unc
