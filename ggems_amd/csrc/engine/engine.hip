@@ -175,7 +175,7 @@ struct RunParams {
   uint32_t n_batches, base, rem;
   uint32_t* queue;            // next slot to hand out
   unsigned long long* stats;  // ggh_stats fields
-  int32_t round_steps;        // voxel steps a wave makes at least per round
+  int32_t round_steps;        // voxel steps a wave makes at least per round; 0: as its photons stop
   int32_t cold_passes;        // navigation passes per round
   uint32_t xchg_offset;       // byte offset of the lane-state exchange area in dynamic LDS
   int mesh_loop;              // kernels without regrouping: each lane walks its mesh to the end (pick_launch)
@@ -218,10 +218,11 @@ enum Mode : int32_t {
 };
 
 // p and ray hold the local frame of the solid while mode is kInVoxel ..
-// kExit, the global frame otherwise.  In mode kInteract the reference
-// sampling keeps the stopped step's random sums in pend, s1 and s2, with p
-// where the step began; tau sampling keeps the material (gmat << 2) in pend,
-// and the reference step of thin voxels proc | gmat << 2.
+// kExit, the global frame otherwise.  In mode kInteract, up to the end of the
+// voxel loop, the reference sampling keeps the stopped step's random sums in
+// pend, s1 and s2, with p where the step began, and tau sampling the material
+// (gmat << 2) in pend; then (choose_process), and from the start in the
+// reference step of thin voxels, pend holds proc | gmat << 2.
 struct Lane {
   Rng r;
   f3 p;
@@ -1083,29 +1084,38 @@ __device__ inline void store_stream(const RunParams& P, uint32_t slot, const Rng
   P.rng[4 * (size_t)P.rng_stride + slot] = r.c;
 }
 
-// The discrete process a voxel step stopped on, then the energy cut
-// (TrackThroughGGEMSVoxelizedSolid.cl:238-310).
-template <int NP, bool kTau, bool kTrack, bool kThin, class Counters>
-__device__ inline void resolve_interaction(const RunParams& P, const Tabs& T, const VoxGeom& G, Lane& L, Counters& c) {
-  int gmat = (int)(L.pend >> 2);
-  int proc = (int)(L.pend & 3u);
-  if (!kTau && !kThin) {
-    proc = stopped_step<NP, kTrack>(P, T, G, L, gmat);
-    if (proc == kTransportation) return;
-  }
+// Which process a stopped step ends on, into pend beside the material: before
+// the regrouping, which gathers the photons by it.  The reference sampling's
+// quick step may turn out to cross its voxel after all (stopped_step then says
+// where it went); its general step knows the process already.
+template <int NP, bool kTau, bool kTrack, bool kThin>
+__device__ inline void choose_process(const RunParams& P, const Tabs& T, const VoxGeom& G, Lane& L) {
   if (kTau) {
-    // the process, in proportion to its left-bin cross section: the first
-    // whose running sum in activation order exceeds u * sigma_tot
+    // in proportion to its left-bin cross section: the first whose running
+    // sum in activation order exceeds u * sigma_tot
     const int np = NP >= 0 ? NP : P.n_proc;
-    const float4 s = T.sig[gmat * P.nbins + L.eid];
+    const float4 s = T.sig[(int)(L.pend >> 2) * P.nbins + L.eid];
     const float x = L.r.uniform() * ((s.x + s.y) + s.z);
-    proc = P.proc[np > 0 ? np - 1 : 0];
+    int proc = P.proc[np > 0 ? np - 1 : 0];
     if (np > 1) {
       const float c0 = s.x;
       if (x < c0) proc = P.proc[0];
       else if (np > 2 && x < c0 + s.y) proc = P.proc[1];
     }
+    L.pend |= (uint32_t)proc;
+  } else if (!kThin) {
+    int gmat;
+    const int proc = stopped_step<NP, kTrack>(P, T, G, L, gmat);
+    L.pend = ((uint32_t)gmat << 2) | (uint32_t)(proc & 3);  // read only where the mode is still kInteract
   }
+}
+
+// The chosen discrete process, then the energy cut
+// (TrackThroughGGEMSVoxelizedSolid.cl:238-310).
+template <bool kTau, class Counters>
+__device__ inline void resolve_interaction(const RunParams& P, const Tabs& T, Lane& L, Counters& c) {
+  const int gmat = (int)(L.pend >> 2);
+  const int proc = (int)(L.pend & 3u);
   c.add(kCntInteractions);
   const float e0 = L.e;
   f3 dir = L.ray.d;
@@ -1146,7 +1156,7 @@ __device__ inline void next_projection(const RunParams& P, Lane& L) {
 template <int NP, bool kSingle, bool kAcq, bool kTau, bool kTrack, bool kThin, bool kRegroup, class Counters>
 __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Counters& c) {
   if (L.mode == kInteract)
-    resolve_interaction<NP, kTau, kTrack, kThin>(P, T, kSingle ? P.vox0 : T.solids[L.solid].vox, L, c);
+    resolve_interaction<kTau>(P, T, L, c);
   if (L.mode == kCut) {
     if (L.solid == P.dose_solid) dose_record(P, L.e, L.p);
     L.mode = kNeedPrimary;
@@ -1264,6 +1274,19 @@ constexpr uint64_t kMeshLoopBelow = 4;
 // 0.973, 40.0 and 27.0 with two; three gained little more with tau sampling
 // and four was slower).
 constexpr int kPassSteps = 2;
+// Steps of a round when the caller states none: short rounds while more than a
+// third of a full block's photons stop in one, long ones again below a quarter
+// and in blocks that run out of photons.  Photons that stop early wait for the
+// round's end, and every round costs its barriers and partial waves of stopped
+// photons.  Fixed rounds of 8, 12, 16 and 20 steps (kernel ms): 256 x 256 x 128
+// body of 1.6 mm voxels 35.3, 35.5, 36.1 and 37; 40-view acquisition, 2 mm,
+// 23.9, 24.5, 25.3 and 26.0; 512 x 512 x 256 body of 0.8 mm with tau sampling,
+// where half as many stop, 183.2, 177.4, 172.5 and 171.6; 50,000 photons, a
+// fifth of the lanes, 0.53, 0.50, 0.44 and 0.46.  By this rule 35.0, 23.7,
+// 172.4 and 0.44 (switching to 10 steps, or at a quarter and a sixth: 35.2,
+// 23.9).
+constexpr int kShortRound = 8, kLongRound = 20;
+
 constexpr size_t kXchgBytes = (size_t)kBlock * 12 * sizeof(uint32_t);
 
 template <bool kTau>
@@ -1283,10 +1306,10 @@ __device__ inline void exchange_lane(Lane& L, uint4* s_x, uint32_t pos) {
   __syncthreads();
   dst[0] = make_uint4(__float_as_uint(L.ray.inv.y), __float_as_uint(L.ray.inv.z), __float_as_uint(L.e),
                       (uint32_t)L.eid);
-  // mode (3 bits), scatter (1 bit) and hop (<= GGH_MAX_HOPS) share a word to make room for tau or the sums
+  // mode (3 bits), scatter (1 bit) and hop (<= GGH_MAX_HOPS) share a word to make room for tau
   dst[1] = make_uint4((uint32_t)L.mode | ((uint32_t)L.scatter << 3) | ((uint32_t)L.hop << 4), (uint32_t)L.solid,
                       L.pend, L.todo);
-  dst[2] = make_uint4(L.slot, L.proj, kTau ? __float_as_uint(L.tau) : L.s1, kTau ? 0u : L.s2);
+  dst[2] = make_uint4(L.slot, L.proj, kTau ? __float_as_uint(L.tau) : 0u, 0u);
   __syncthreads();
   a = src[0];
   b = src[1];
@@ -1303,12 +1326,7 @@ __device__ inline void exchange_lane(Lane& L, uint4* s_x, uint32_t pos) {
   L.todo = b.w;
   L.slot = d.x;
   L.proj = d.y;
-  if (kTau) {
-    L.tau = __uint_as_float(d.z);
-  } else {
-    L.s1 = d.z;
-    L.s2 = d.w;
-  }
+  if (kTau) L.tau = __uint_as_float(d.z);
   __syncthreads();
 }
 
@@ -1473,7 +1491,7 @@ void transport_kernel(RunParams P) {
     //      primary or slot) by at most cold_passes navigation passes;
     //   2. makes voxel steps until every wave of the block is ready to stop:
     //      a wave is ready once all waves have finished step 1 and it has made
-    //      round_steps steps (or has no lane inside a phantom); ready waves
+    //      its round's steps (or has no lane inside a phantom); ready waves
     //      keep stepping until all are, so no wave idles at the barrier
     //      longer than about one step;
     //   3. regroups the block's photons: those inside a phantom first, then
@@ -1483,7 +1501,8 @@ void transport_kernel(RunParams P) {
     // Every wave passes the same barriers in every round, and every loop
     // above is bounded, so the block cannot deadlock.
     uint4* s_x = reinterpret_cast<uint4*>(reinterpret_cast<char*>(s_tab) + P.xchg_offset);
-    __shared__ uint32_t s_cnt[kWaves][3];
+    constexpr int kRanks = 5;
+    __shared__ uint32_t s_cnt[kWaves][kRanks - 1];
     __shared__ uint32_t s_cold_done[2];
     __shared__ uint32_t s_ready[2];
     const int wave = (int)(threadIdx.x >> 6), lane = __lane_id();
@@ -1497,6 +1516,7 @@ void transport_kernel(RunParams P) {
       return kTau ? hot_step_tau<kTrack, kThin>(P, T, G, L)
                   : (kThin ? hot_step_thin<NP, kTrack>(P, T, G, L) : hot_step<NP, kTrack>(P, T, G, L));
     };
+    int target = P.round_steps ? P.round_steps : kLongRound;  // the same in every wave
     for (uint32_t round = 0;; ++round) {
       const uint32_t rb = round & 1u;
       for (int pass = 0; pass < P.cold_passes; ++pass) {
@@ -1512,7 +1532,7 @@ void transport_kernel(RunParams P) {
       bool ready = false;
       for (int k = 0;; k += kPassSteps) {  // k counts voxel steps
         const uint64_t act = __ballot(L.mode == kInVoxel);
-        if (!ready && (act == 0 || (k >= P.round_steps && lds_load_relaxed(&s_cold_done[rb]) == (uint32_t)kWaves))) {
+        if (!ready && (act == 0 || (k >= target && lds_load_relaxed(&s_cold_done[rb]) == (uint32_t)kWaves))) {
           ready = true;
           if (lane == 0) atomicAdd(&s_ready[rb], 1u);
         }
@@ -1527,43 +1547,63 @@ void transport_kernel(RunParams P) {
         }
         steps += __popcll(__ballot(stepped)) + __popcll(__ballot(stepped2));
       }
-      // regrouping by event: rank 0 inside a phantom, 1 a pending
-      // interaction, 2 other navigation (exit, cut, new primary or slot),
-      // 3 no work left, so that the next navigation passes run one kind of
-      // event per wave.  Interactions wait for these passes: resolved inside
-      // the voxel loop 16 lanes at a time, as the reference sampling once did,
-      // they took a third of the kernel's instructions on a quarter of the
-      // lanes (256 x 256 x 128 body: 46.6 ms, and 40.0 ms resolved here).
-      const int key = L.mode == kInVoxel ? 0 : (L.mode == kInteract ? 1 : (L.mode != kDone ? 2 : 3));
-      const uint64_t b0 = __ballot(key == 0), b1 = __ballot(key == 1), b2 = __ballot(key == 2);
-      if (lane == 0) {
-        s_cnt[wave][0] = (uint32_t)__popcll(b0);
-        s_cnt[wave][1] = (uint32_t)__popcll(b1);
-        s_cnt[wave][2] = (uint32_t)__popcll(b2);
-      }
+      if (L.mode == kInteract)
+        choose_process<NP, kTau, kTrack, kThin>(cold_params(), T, kSingle ? P.vox0 : T.solids[L.solid].vox, L);
+      // regrouping by event: rank 0 inside a phantom, 1 Compton scattering, 2
+      // Rayleigh scattering, 3 other navigation (absorption, exit, cut, new
+      // primary or slot), 4 no work left, so that the next navigation passes
+      // run one kind of event per wave.  Interactions wait for these passes:
+      // resolved inside the voxel loop 16 lanes at a time, as the reference
+      // sampling once did, they took a third of the kernel's instructions on a
+      // quarter of the lanes (256 x 256 x 128 body: 46.6 ms, and 40.0 ms
+      // resolved here).  The process is chosen before the regrouping: with all
+      // interactions in one rank nearly every stopped wave ran Compton's and
+      // Rayleigh's loops and the source, on 30, 5 and 14 lanes; apart they run
+      // on 43, 12 and 33 (39.6 to 36.1 ms, 40-view acquisition 26.3 to 25.2).
+      const int event = (int)(L.pend & 3u);
+      const int key = L.mode == kInVoxel ? 0
+                      : L.mode == kInteract && event != kPhotoelectric
+                          ? (event == kCompton ? 1 : 2)
+                          : (L.mode != kDone ? 3 : 4);
+      uint64_t votes[kRanks];
+      for (int q = 0; q < kRanks; ++q) votes[q] = __ballot(key == q);
+      if (lane == 0)
+        for (int q = 0; q + 1 < kRanks; ++q) s_cnt[wave][q] = (uint32_t)__popcll(votes[q]);
       __syncthreads();
-      uint32_t n0 = 0, n1 = 0, n2 = 0, before0 = 0, before1 = 0, before2 = 0, before3 = 0;
-      for (int w = 0; w < kWaves; ++w) {
-        const uint32_t c0 = s_cnt[w][0], c1 = s_cnt[w][1], c2 = s_cnt[w][2];
-        n0 += c0;
-        n1 += c1;
-        n2 += c2;
-        if (w < wave) {
-          before0 += c0;
-          before1 += c1;
-          before2 += c2;
-          before3 += 64u - c0 - c1 - c2;
+      // the block's photons of smaller rank, then those of earlier waves of the same
+      uint32_t first = 0, inside = 0, total = 0, before = 0, others = 0;
+      uint64_t mine = 0;
+      for (int q = 0; q + 1 < kRanks; ++q) {
+        uint32_t n = 0, b = 0;
+        for (int w = 0; w < kWaves; ++w) {
+          const uint32_t m = s_cnt[w][q];
+          n += m;
+          b += w < wave ? m : 0u;
         }
+        if (q < key) first += n;
+        if (q == key) {
+          before = b;
+          mine = votes[q];
+        }
+        if (q == 0) inside = n;
+        total += n;
+        others += b;
       }
-      if (n0 + n1 + n2 == 0) break;  // read from LDS after a barrier: the same for the whole block
+      if (total == 0) break;  // read from LDS after a barrier: the same for the whole block
+      if (P.round_steps == 0) {
+        const uint32_t stopped = total - inside;
+        if (total < kBlock / 8 * 7 || 4 * stopped < total) target = kLongRound;
+        else if (3 * stopped > total) target = kShortRound;
+      }
+      if (key == kRanks - 1) {
+        before = 64u * (uint32_t)wave - others;
+        mine = votes[kRanks - 1];
+      }
       if (threadIdx.x == 0) {  // the next round's counters; nobody reads them before the barriers below
         s_cold_done[rb ^ 1u] = 0;
         s_ready[rb ^ 1u] = 0;
       }
-      const uint64_t mine = key == 0 ? b0 : (key == 1 ? b1 : (key == 2 ? b2 : ~(b0 | b1 | b2)));
-      const uint32_t pos = (key == 0 ? before0 : (key == 1 ? n0 + before1 : (key == 2 ? n0 + n1 + before2
-                                                                               : n0 + n1 + n2 + before3))) +
-                           (uint32_t)__popcll(mine & below);
+      const uint32_t pos = first + before + (uint32_t)__popcll(mine & below);
       exchange_lane<kTau>(L, s_x, pos);
     }
   }
@@ -2038,7 +2078,7 @@ struct ggh_context {
   DevBuf<uint32_t> queue;
   DevBuf<unsigned long long> stats;
   // launch shape
-  int round_steps = 0;  // 0: 16 (measured best; 12 and 20 within 2 %, 32 slower by 5 %)
+  int round_steps = 0;  // 0: kShortRound or kLongRound, as the block's photons stop
   int cold_passes = 0;  // 0: 1 (two were 2-5 % slower with the reference sampling)
   int interact_batch = 16;
   int blocks_per_cu = 0;  // 0: as many as fit
@@ -2278,7 +2318,7 @@ RunParams make_params(ggh_context* c) {
   P.rng_stride = GGH_MAX_SLOTS;
   P.queue = c->queue.p;
   P.stats = c->stats.p;
-  P.round_steps = c->round_steps ? c->round_steps : 16;
+  P.round_steps = c->round_steps;
   P.cold_passes = c->cold_passes ? c->cold_passes : 1;
   P.xchg_offset = 0;
   P.mesh_loop = 0;

@@ -415,7 +415,7 @@ class Engine:
         return pos, dir, e
 
     def set_launch(self, round_steps=0, interact_batch=0, blocks_per_cu=0, general_kernel=False, cold_passes=0):
-        """launch shape of run(); zero keeps a default (round_steps 16, cold_passes 1);
+        """launch shape of run(); zero keeps a default (round_steps: 8 or 20 as photons stop, cold_passes 1);
         interact_batch is accepted and has no effect"""
         d = LaunchDesc(int(round_steps), int(cold_passes), int(interact_batch), int(blocks_per_cu),
                        int(bool(general_kernel)))

@@ -166,7 +166,7 @@ int ggh_get_stats(ggh_context* ctx, ggh_stats* out);
  * Zero fields keep the defaults. */
 typedef struct {
   int32_t round_steps;     /* voxel steps a wave makes at least between two regroupings of its
-                              block's photons (1..1024; default 16) */
+                              block's photons (1..1024; default 8 or 20, as the block's photons stop) */
   int32_t cold_passes;     /* navigation passes per round for the photons that are not inside a
                               phantom (1..16; default 1) */
   int32_t interact_batch;  /* accepted (0..64) and without effect: interactions are resolved in the
