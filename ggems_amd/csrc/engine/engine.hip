@@ -2106,7 +2106,7 @@ struct ggh_context {
   int drr_n_w = 0;
   DevBuf<float> drr_image;
   std::mutex drr_mu_image;  // one ggh_drr at a time uses drr_image
-  // pinned slots of the readbacks (through_slots), made by the first and kept
+  // pinned slots of the readbacks (through_slots), kept
   char* slots = nullptr;
   hipEvent_t slot_ev[kCopiers] = {};
   std::mutex slots_mu;  // one readback at a time uses the slots
@@ -2637,6 +2637,8 @@ int ggh_context_create(int device, ggh_context** out) {
     ggh_context_destroy(c);
     return rc;
   }
+  // 1.5 ms that the first readback would pay; one that finds no slots tries again
+  if (make_slots(c) != hipSuccess) (void)hipGetLastError();
   (void)hipMemsetAsync(c->stats.p, 0, 8 * sizeof(unsigned long long), c->stream);
   *out = c;
   return 0;
