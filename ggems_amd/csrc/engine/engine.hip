@@ -1538,6 +1538,14 @@ void transport_kernel(RunParams P) {
         if (cold) cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin, kRegroup>(cold_params(), T, L, c);
       }
       __builtin_amdgcn_s_setprio(0);
+      // The reference step draws its random numbers while its label is on the
+      // way.  Where the lane's stream may itself still be on the way (a new
+      // slot's), the compiler waits for both before the first draw, in every
+      // first step of a pass: wait for the stream here instead (256 x 256 x 128
+      // body 34.5 to 33.9 ms, 5 x 10^4 photons 0.49 to 0.48).  Tau steps draw
+      // nothing and the acquisition's order its loads otherwise: there it cost
+      // up to 1 %.
+      if (!kTau && !kAcq) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       if (lane == 0) atomicAdd(&s_cold_done[rb], 1u);
       bool ready = false;
       for (int k = 0;; k += kPassSteps) {  // k counts voxel steps
