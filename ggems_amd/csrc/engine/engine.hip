@@ -20,10 +20,11 @@
 //   * navigation for a stopped lane: it resolves its interaction, leaves the
 //     phantom, starts its next primary, crosses to the next solid or tracks
 //     through a detector module, until it is back inside a phantom.
-// A block works in rounds: a few navigation passes, voxel steps, then the
-// block regroups its photons through LDS so that the photons inside a
-// phantom fill whole waves and the stopped ones gather in a few others
-// (transport_kernel).  Regrouping and the state machine only reorder work
+// A block works in rounds: a navigation pass, voxel steps, then the block
+// regroups its photons through LDS so that the photons inside a phantom fill
+// whole waves and the stopped ones gather by their event in a few others
+// (transport_kernel).  Scenes without a voxel solid share the walk through
+// their meshes instead.  Regrouping and the state machine only reorder work
 // between lanes; each photon consumes its slot's stream in exactly the
 // reference order.
 #include <hip/hip_runtime.h>
@@ -36,7 +37,9 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <random>
 #include <string>
 #include <thread>
@@ -2171,8 +2174,24 @@ hipError_t make_slots(ggh_context* c) {
 template <class Fill, class Take>
 hipError_t through_slots(ggh_context* c, int64_t items, size_t item_bytes, Fill fill, Take take) {
   std::lock_guard<std::mutex> lock(c->slots_mu);
-  const hipError_t made = make_slots(c);
-  if (made != hipSuccess) return made;
+  if (make_slots(c) != hipSuccess) {
+    // no pinned memory left: one small chunk at a time over device memory
+    (void)hipGetLastError();
+    const int64_t few = (int64_t)(kChunkBytes / item_bytes / 64 * 64);
+    std::unique_ptr<char[]> host(new (std::nothrow) char[kChunkBytes]);
+    char* dev = nullptr;
+    hipError_t e = host ? hipMalloc(reinterpret_cast<void**>(&dev), kChunkBytes) : hipErrorOutOfMemory;
+    for (int64_t at = 0; e == hipSuccess && at < items; at += few) {
+      const int64_t n = std::min(few, items - at);
+      fill(dev, few, at, n);
+      e = hipGetLastError();
+      if (e == hipSuccess) e = hipMemcpyAsync(host.get(), dev, kChunkBytes, hipMemcpyDeviceToHost, c->stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+      if (e == hipSuccess) take(host.get(), few, at, n);
+    }
+    if (dev) (void)hipFree(dev);
+    return e;
+  }
   const size_t share = ((size_t)items * item_bytes + kCopiers - 1) / kCopiers;
   const int64_t per = (int64_t)(std::min(std::max(share, kChunkBytes), kSlotBytes) / item_bytes / 64 * 64);
   std::atomic<int64_t> next{0};

@@ -7,8 +7,14 @@
 // Cout are multiples of 8 and 16 (the first layer pads its two input
 // channels); W is a multiple of 16 and N H W of 32.
 //
+// Two sets of kernels.  The channel counts of the U-Net with aligned tensors
+// take the tile kernels (conv_tile_kernel, conv_wgrad_tile_kernel): an input
+// tile with its halo goes to LDS once and serves all nine taps.  Everything
+// else takes the general ones, whose order of additions the tile kernels keep
+// in the forward pass and the data gradient:
+//
 // Forward (implicit GEMM, M = pixels, N = Cout, K = 9 Cin): a wave owns
-// 32 consecutive pixels (two runs of 16 within image rows) and 64 output
+// 32 consecutive pixels (two runs of 16 within image rows) and up to 64 output
 // channels, i.e. 2 x 4 accumulator tiles of 16 x 16; each K step of 32 loads
 // one 16-byte A fragment per pixel tile from memory and one B fragment per
 // channel tile from the block's LDS copy of the weights, and issues 8 MFMAs.
@@ -20,7 +26,7 @@
 // shifted input in LDS as they lie in memory (channels contiguous, 16-byte
 // stores) and the waves read MFMA fragments with gfx950's transposing LDS
 // read; blocks split the pixels and add their partial sums atomically in
-// FP32.
+// FP32 (the tile kernel in a work space, summed in order).
 
 #include <hip/hip_runtime.h>
 

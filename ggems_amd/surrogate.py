@@ -2,10 +2,10 @@
 projection and the ray-traced primary image to the scatter image.
 
 Its 3x3 convolutions run on the matrix cores through the engine library
-(ggh_conv3x3_forward / ggh_conv3x3_weight_grad: BF16 operands, FP32
+(ggh_conv3x3_forward / ggh_conv3x3_backward: BF16 operands, FP32
 accumulation); PyTorch holds the tensors, streams and optimiser state.
 Activations are NHWC BF16; master weights are FP32 [cout][9][cin] and are
-cast to BF16 for every call.
+rounded to BF16 in every call.
 
 Architecture (4 levels, 16-32-64-128 channels): two 3x3 conv + ReLU per
 level, 2x2 max-pooling down, nearest-neighbour 2x upsampling, concatenation
