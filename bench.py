@@ -295,7 +295,7 @@ def main():
     ap.add_argument("--round-steps", type=int, default=0,
                     help="voxel steps a wave makes at least between regroupings (0: engine default)")
     ap.add_argument("--interact-batch", type=int, default=0,
-                    help="resolve interactions inside the voxel loop once this many lanes wait (0: engine default)")
+                    help="accepted and without effect: interactions are resolved in the navigation passes")
     ap.add_argument("--cold-passes", type=int, default=0,
                     help="navigation passes per round for stopped photons (0: engine default)")
     ap.add_argument("--blocks-per-cu", type=int, default=0)
