@@ -1281,12 +1281,6 @@ constexpr int kMeshWalkers = 8, kMeshLeaves = 8;
 // and 2 x 10^6 primaries over 262,144 lanes (ms): loop 0.75, 1.50, 3.57, 4.16
 // and 7.43, walk 1.27, 1.72, 3.12, 4.07 and 5.67.
 constexpr uint64_t kMeshLoopBelow = 4;
-// Voxel steps per pass of the voxel loop: the steps are short, so the pass's
-// ballots and round checks weigh (10^6 photons through 100^3 voxels, 256 x
-// 256 x 128 body, 40-view acquisition: 0.967, 40.3 and 28.6 ms with one,
-// 0.973, 40.0 and 27.0 with two; three gained little more with tau sampling
-// and four was slower).
-constexpr int kPassSteps = 2;
 // Steps of a round when the caller states none: short rounds while more than a
 // third of a full block's photons stop in one, long ones again below a quarter
 // and in blocks that run out of photons.  Photons that stop early wait for the
@@ -1530,6 +1524,14 @@ void transport_kernel(RunParams P) {
                   : (kThin ? hot_step_thin<NP, kTrack>(P, T, G, L) : hot_step<NP, kTrack>(P, T, G, L));
     };
     int target = P.round_steps ? P.round_steps : kLongRound;  // the same in every wave
+    // Voxel steps per pass of the loop below: the steps are short, so the
+    // pass's ballots and round checks weigh (10^6 photons through 100^3 voxels,
+    // 256 x 256 x 128 body, 40-view acquisition: 0.967, 40.3 and 28.6 ms with
+    // one, 0.973, 40.0 and 27.0 with two).  Three pay for the shorter tau steps
+    // (512 x 512 x 256 body, 4 x 10^7 photons, 71.3 to 70.3 ms; 256 x 256 x 128
+    // body 29.9 to 29.3), and cost the reference steps up to 2 % (2 x 10^7
+    // photons through 100^3 voxels, 7.22 to 7.32).
+    constexpr int kPassSteps = kTau ? 3 : 2;
     for (uint32_t round = 0;; ++round) {
       const uint32_t rb = round & 1u;
       for (int pass = 0; pass < P.cold_passes; ++pass) {
@@ -1558,15 +1560,17 @@ void transport_kernel(RunParams P) {
           if (lane == 0) atomicAdd(&s_ready[rb], 1u);
         }
         if (act == 0 || (ready && lds_load_relaxed(&s_ready[rb]) == (uint32_t)kWaves)) break;
-        bool stepped = false, stepped2 = false;
+        bool stepped = false, stepped2 = false, stepped3 = false;
         // the phantom's geometry: kernel arguments for the only voxel
         // solid, else the lane's solid in the (LDS-staged) solid table
         if (L.mode == kInVoxel) {
           const VoxGeom& G = kSingle ? P.vox0 : T.solids[L.solid].vox;
           stepped = one_step(G);
           if (L.mode == kInVoxel) stepped2 = one_step(G);
+          if (kPassSteps > 2 && L.mode == kInVoxel) stepped3 = one_step(G);
         }
         steps += __popcll(__ballot(stepped)) + __popcll(__ballot(stepped2));
+        if (kPassSteps > 2) steps += __popcll(__ballot(stepped3));
       }
       if (L.mode == kInteract)
         choose_process<NP, kTau, kTrack, kThin>(cold_params(), T, kSingle ? P.vox0 : T.solids[L.solid].vox, L);
