@@ -72,13 +72,24 @@ def _check(rc):
 
 def _stream(t):
     # the current stream's handle without a Stream object, which costs as much as a launch
-    return torch._C._cuda_getCurrentRawStream(t.device.index)
+    index = t.device.index
+    if index is None:
+        raise ValueError("expected a tensor on the GPU, not on %s" % t.device)
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
+def _on_device(device, **tensors):
+    """refuses tensors (or None) that a kernel on `device` could not read"""
+    for name, t in tensors.items():
+        if t is not None and t.device != device:
+            raise EngineError("%s is on %s, the input on %s" % (name, t.device, device))
 
 
 def conv3x3(x, w, bias=None, relu=False):
     """x [N,H,W,Cin] BF16, w [Cout, 9*Cin] BF16, bias [Cout] FP32 -> [N,H,W,Cout] BF16"""
     if x.device.type != "cuda" or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise EngineError("conv3x3 takes BF16 tensors on the GPU")
+    _on_device(x.device, weights=w, bias=bias)
     x, w = x.contiguous(), w.contiguous()
     n, h, wd, cin = x.shape
     cout = w.shape[0]
@@ -189,6 +200,7 @@ def _conv_layer(x, w, b, relu):
     1, 8 and 16 views of 256 x 256: 232, 295 and 460 us from FP32, 399, 391 and
     432 us from BF16)"""
     cout, _, cin = w.shape
+    _on_device(x.device, weights=w, bias=b)
     if (cin in F32W_CHANNELS and x.numel() // cin <= F32W_PIXELS and w.dtype == torch.float32 and w.is_contiguous()
             and w.data_ptr() % 16 == 0 and x.dtype == torch.bfloat16 and x.is_cuda and x.shape[3] == cin
             and (b is None or (b.dtype == torch.float32 and b.is_contiguous()))):
@@ -342,6 +354,7 @@ class _Head(torch.autograd.Function):
 
 def head16(z, head, bias):
     """sum over the 16 channels of z [N,H,W,16] BF16 times head, plus bias -> [N,H,W] FP32"""
+    _on_device(z.device, head=head, bias=bias)
     out = torch.empty(z.shape[:3], dtype=torch.float32, device=z.device)
     _check(_lib().ggh_unet_head(z.data_ptr(), head.data_ptr(), bias.data_ptr(), out.data_ptr(), out.numel(),
                                 _stream(z)))
