@@ -95,6 +95,8 @@ def conv3x3(x, w, bias=None, relu=False):
     cout = w.shape[0]
     if w.shape[1] != 9 * cin:
         raise EngineError("weights must be [cout, 9*cin]")
+    if bias is not None and bias.numel() < cout:
+        raise EngineError("bias must hold %d channels" % cout)
     y = torch.empty((n, h, wd, cout), dtype=torch.bfloat16, device=x.device)
     b = None if bias is None else bias.contiguous().float()
     _check(_lib().ggh_conv3x3_forward(x.data_ptr(), w.data_ptr(), None if b is None else b.data_ptr(), y.data_ptr(),
@@ -168,7 +170,9 @@ def weights_bf16(w, zero=None):
     """(w as BF16 [cout][9][cin], flip_transpose of it [cin][9][cout]) from the
     FP32 weights in one kernel, which also sets the FP32 buffers `zero` =
     (dw [cout, 9 cin], db [cout]) to zero when given"""
-    cout, _, cin = w.shape
+    cout, taps, cin = w.shape
+    if taps != 9:
+        raise EngineError("weights must be [cout, 9, cin]")
     w = w.detach().contiguous().float()
     wb = torch.empty((cout, 9, cin), dtype=torch.bfloat16, device=w.device)
     wt = torch.empty((cin, 9, cout), dtype=torch.bfloat16, device=w.device)
@@ -199,11 +203,12 @@ def _conv_layer(x, w, b, relu):
     blocks would each round them, and BF16 ones are made first (the network on
     1, 8 and 16 views of 256 x 256: 232, 295 and 460 us from FP32, 399, 391 and
     432 us from BF16)"""
-    cout, _, cin = w.shape
+    cout, taps, cin = w.shape
     _on_device(x.device, weights=w, bias=b)
-    if (cin in F32W_CHANNELS and x.numel() // cin <= F32W_PIXELS and w.dtype == torch.float32 and w.is_contiguous()
-            and w.data_ptr() % 16 == 0 and x.dtype == torch.bfloat16 and x.is_cuda and x.shape[3] == cin
-            and (b is None or (b.dtype == torch.float32 and b.is_contiguous()))):
+    if (taps == 9 and cin in F32W_CHANNELS and x.numel() // cin <= F32W_PIXELS and w.dtype == torch.float32
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 and x.dtype == torch.bfloat16 and x.is_cuda
+            and x.shape[3] == cin
+            and (b is None or (b.dtype == torch.float32 and b.is_contiguous() and b.shape == (cout,)))):
         x = x.contiguous()
         n, h, wd, _ = x.shape
         y = torch.empty((n, h, wd, cout), dtype=torch.bfloat16, device=x.device)
@@ -352,9 +357,19 @@ class _Head(torch.autograd.Function):
         return dz, sums[:16], sums[16:]
 
 
+def _fits_head16(z, head, bias):
+    """whether the kernel reads these as (z * head).sum(3) + bias does: one weight
+    a channel and one bias on z's device (other shapes broadcast)"""
+    return (z.ndim == 4 and z.shape[3] == 16 and z.dtype == torch.bfloat16 and z.is_contiguous() and z.is_cuda
+            and head.dtype == bias.dtype == torch.float32 and head.is_contiguous() and head.shape == (16,)
+            and bias.shape == (1,) and head.device == bias.device == z.device)
+
+
 def head16(z, head, bias):
-    """sum over the 16 channels of z [N,H,W,16] BF16 times head, plus bias -> [N,H,W] FP32"""
+    """sum over the 16 channels of z [N,H,W,16] BF16 times head [16], plus bias [1] -> [N,H,W] FP32"""
     _on_device(z.device, head=head, bias=bias)
+    if not _fits_head16(z, head, bias):
+        raise EngineError("the head takes BF16 z [N, H, W, 16] and FP32 head [16] and bias [1] on the GPU")
     out = torch.empty(z.shape[:3], dtype=torch.float32, device=z.device)
     _check(_lib().ggh_unet_head(z.data_ptr(), head.data_ptr(), bias.data_ptr(), out.data_ptr(), out.numel(),
                                 _stream(z)))
@@ -405,8 +420,7 @@ class UNet(torch.nn.Module):
         for (a, b), s in zip(self.dec, reversed(skips)):
             z = b(a(upcat(z, s) if direct else _UpCat.apply(z, s)))
         head, bias = self.head, self.head_bias
-        if (z.shape[3] == 16 and z.dtype == torch.bfloat16 and z.is_contiguous() and z.is_cuda
-                and head.dtype == bias.dtype == torch.float32 and head.is_contiguous()):
+        if _fits_head16(z, head, bias):
             return head16(z, head, bias) if direct else _Head.apply(z, head, bias)
         # the head as a multiply and a channel sum: a matrix-vector product
         # with 16 columns runs far below HBM speed in the BLAS path

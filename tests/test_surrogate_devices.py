@@ -1,5 +1,7 @@
 """A network and an input on different devices are refused before any kernel
-is launched: a host pointer would fault the GPU.  The library is a recorder
+is launched: a host pointer would fault the GPU.  So are parameters of another
+shape than the kernels read, where tensor operations broadcast or refused
+them.  The library is a recorder
 and the GPU tensors are stand-ins, so nothing runs on a GPU here."""
 
 import pytest
@@ -15,7 +17,7 @@ class OnGpu:
 
     def __init__(self, t):
         self.t, self.device, self.is_cuda = t, GPU, True
-        self.shape, self.dtype = t.shape, t.dtype
+        self.shape, self.dtype, self.ndim = t.shape, t.dtype, t.ndim
 
     def contiguous(self):
         return self
@@ -92,3 +94,25 @@ def test_host_parameters_are_refused_before_a_launch(launches, call, here):
 def test_a_host_tensor_has_no_stream():
     with pytest.raises(ValueError):
         S._stream(torch.zeros(1))
+
+
+@pytest.mark.parametrize("w,b", [((16, 7, 16), 16), ((16, 9, 16), 12), ((16, 1, 16), 16)])
+def test_layers_of_other_shapes_do_not_reach_the_kernel(launches, w, b):
+    x = OnGpu(torch.zeros(1, 16, 16, 16, dtype=torch.bfloat16))
+    with pytest.raises((S.EngineError, RuntimeError)):
+        S._conv_layer(x, OnGpu(torch.zeros(w)), OnGpu(torch.zeros(b)), True)
+    assert not [c for c in launches if c.startswith("ggh_conv3x3_forward")]
+
+
+@pytest.mark.parametrize("head,bias,fits", [((16,), (1,), True), ((1,), (1,), False), ((16,), (), False),
+                                            ((16,), (16,), False), ((1, 16), (1,), False)])
+def test_head_shapes_that_broadcast_take_the_tensor_operations(launches, head, bias, fits):
+    z = OnGpu(torch.zeros(1, 16, 16, 16, dtype=torch.bfloat16))
+    head, bias = OnGpu(torch.zeros(head)), OnGpu(torch.zeros(bias))
+    assert S._fits_head16(z, head, bias) == fits
+    if fits:
+        S.head16(z, head, bias)
+        return
+    with pytest.raises(S.EngineError):
+        S.head16(z, head, bias)
+    assert launches == []
