@@ -346,7 +346,9 @@ class _Head(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         z, head = ctx.saved_tensors
-        if torch.is_grad_enabled():  # create_graph: gradients that can be differentiated again
+        # create_graph: gradients that can be differentiated again; a batch of
+        # gradients (is_grads_batched) has no memory that a kernel could read
+        if torch.is_grad_enabled() or not torch._C._has_storage(dout):
             d = dout.unsqueeze(3)
             return (d * head).to(torch.bfloat16), (d * z.float()).sum((0, 1, 2)), dout.sum().reshape(1)
         dout = dout.contiguous()
@@ -420,7 +422,7 @@ class UNet(torch.nn.Module):
         for (a, b), s in zip(self.dec, reversed(skips)):
             z = b(a(upcat(z, s) if direct else _UpCat.apply(z, s)))
         head, bias = self.head, self.head_bias
-        if _fits_head16(z, head, bias):
+        if _fits_head16(z, head, bias) and _untraced():
             return head16(z, head, bias) if direct else _Head.apply(z, head, bias)
         # the head as a multiply and a channel sum: a matrix-vector product
         # with 16 columns runs far below HBM speed in the BLAS path
