@@ -875,9 +875,11 @@ void GGEMS::autotune(uint64_t n_trial) {
   auto& sources = GGEMSSourceManager::get().sources;
   if (sources.empty()) raise("GGEMS", "No source registered!!!");
   upload_source(*sources.front());
-  ggh_launch_desc best;
-  engine_check(ggh_autotune(ctx, n_trial, &best), "autotune");
-  log(1, "GGEMS", "autotuned launch: round steps " + std::to_string(best.round_steps) + ", interaction batch " +
-                      std::to_string(best.interact_batch) + ", navigation passes " +
-                      std::to_string(best.cold_passes) + ", blocks per CU " + std::to_string(best.blocks_per_cu));
+  ggh_launch_desc kept;
+  engine_check(ggh_autotune(ctx, n_trial, nullptr), "autotune");
+  engine_check(ggh_get_launch(ctx, &kept), "autotune");
+  log(1, "GGEMS", "autotuned launch: round steps " +
+                      (kept.round_steps ? std::to_string(kept.round_steps) : std::string("as the photons stop")) +
+                      ", navigation passes " + std::to_string(kept.cold_passes) + ", blocks per CU " +
+                      std::to_string(kept.blocks_per_cu));
 }

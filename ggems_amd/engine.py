@@ -120,6 +120,7 @@ def library():
             "ggh_host_voxel_exit": ([vp, vp, C.c_size_t, vp, vp, vp, vp, vp], C.c_int),
             "ggh_host_energy_bin": ([vp, C.c_size_t, vp, C.c_int32, vp], None),
             "ggh_set_launch": ([vp, C.POINTER(LaunchDesc)], C.c_int),
+            "ggh_get_launch": ([vp, C.POINTER(LaunchDesc)], C.c_int),
             "ggh_last_grid": ([vp, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)], C.c_int),
             "ggh_debug_neg_log": ([vp, C.c_int, vp, vp, vp], C.c_int),
             "ggh_add_mesh_solid": ([vp, C.POINTER(MeshSolidDesc)], C.c_int),
@@ -500,8 +501,15 @@ class Engine:
         _check(library().ggh_drr_noalloc(self.h, solid, int(projection), C.c_void_p(image_ptr),
                                          None if stream is None else C.c_void_p(stream)))
 
+    def launch(self):
+        """the launch shape in force (set_launch's arguments)"""
+        d = LaunchDesc()
+        _check(library().ggh_get_launch(self.h, C.byref(d)))
+        return {k: int(getattr(d, k)) for k, _ in LaunchDesc._fields_}
+
     def autotune(self, n_trial):
-        """fastest launch shape over a trial run; call after seed() and before any run"""
+        """times launch shapes over a trial run and keeps the fastest (launch()); returns the
+        fastest with a stated round length; call after seed() and before any run"""
         d = LaunchDesc()
         _check(library().ggh_autotune(self.h, int(n_trial), C.byref(d)))
         return {k: int(getattr(d, k)) for k, _ in LaunchDesc._fields_}

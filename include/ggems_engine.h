@@ -175,6 +175,8 @@ typedef struct {
   int32_t general_kernel;  /* nonzero: the general kernel variant even where the specialised one applies */
 } ggh_launch_desc;
 int ggh_set_launch(ggh_context* ctx, const ggh_launch_desc* desc);
+/* the launch shape in force, as set or as the autotuner left it */
+int ggh_get_launch(ggh_context* ctx, ggh_launch_desc* out);
 
 /* How a voxel step samples its interaction (no counterpart in GGEMS).
  * GGH_SAMPLING_REFERENCE (the default) draws the three competing
@@ -256,8 +258,11 @@ int ggh_drr(ggh_context* ctx, int solid, int projection, float* image);
 int ggh_drr_noalloc(ggh_context* ctx, int solid, int projection, float* image, void* stream);
 
 /* Launch autotuner: times ggh_run(n_trial) over a grid of launch shapes
- * (blocks per compute unit, round steps) and keeps the fastest.  Call after ggh_seed and before any run: it restores the seeded
- * random streams and zeroes every tally and counter afterwards. */
+ * (blocks per compute unit, round steps) and keeps the fastest.  *best (may be
+ * null) is the fastest with a stated round length; where the default rule
+ * (round_steps 0) is as fast the context keeps that instead, which
+ * ggh_get_launch shows.  Call after ggh_seed and before any run: it restores
+ * the seeded random streams and zeroes every tally and counter afterwards. */
 int ggh_autotune(ggh_context* ctx, uint64_t n_trial, ggh_launch_desc* best);
 int ggh_get_dose_tallies(ggh_context* ctx, double* edep, double* edep_squared, int32_t* hit,
                          int32_t* photon_tracking);
