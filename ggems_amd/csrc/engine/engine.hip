@@ -181,6 +181,7 @@ struct RunParams {
   int32_t round_steps;        // voxel steps a wave makes at least per round; 0: as its photons stop
   int32_t cold_passes;        // navigation passes per round
   uint32_t xchg_offset;       // byte offset of the lane-state exchange area in dynamic LDS
+  int look_ahead;             // a leaving photon looks for its next solid at once (kAheadSolids)
   int mesh_loop;              // kernels without regrouping: each lane walks its mesh to the end (pick_launch)
   VoxGeom vox0;               // the only voxel solid, when there is exactly one
   // CT acquisition: projection p places the source at acq_src[p] and box
@@ -1164,17 +1165,17 @@ __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Cou
     if (L.solid == P.dose_solid) dose_record(P, L.e, L.p);
     L.mode = kNeedPrimary;
   }
+  int ahead = -1;  // the solid a leaving photon goes on to
   if (L.mode == kExit) {
     const DevSolid& s = T.solids[L.solid];
     L.p = l2g_pos(s.m, L.p);
     L.ray.d = l2g_dir(s.m, L.ray.d);
     L.mode = kHop;
-    if (kRegroup) {
+    if (kRegroup && P.look_ahead && L.hop < GGH_MAX_HOPS) {
       // a photon that meets nothing more is done: its successor starts in this
-      // pass, not a round later (256 x 256 x 128 body 35.5 to 34.7 ms, 2 x 10^7
-      // photons through 100^3 voxels 7.42 to 7.22)
-      f3 q = L.p;
-      if (L.hop < GGH_MAX_HOPS && find_and_project<kAcq>(P, T, q, L.ray.d, L.proj) < 0) {
+      // pass, not a round later (kAheadSolids)
+      ahead = find_and_project<kAcq>(P, T, L.p, L.ray.d, L.proj);
+      if (ahead < 0) {
         c.add(kCntHops);
         L.mode = kNeedPrimary;
       }
@@ -1231,7 +1232,7 @@ __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Cou
     }
     ++L.hop;
     c.add(kCntHops);
-    const int k = find_and_project<kAcq>(P, T, L.p, L.ray.d, L.proj);
+    const int k = ahead >= 0 ? ahead : find_and_project<kAcq>(P, T, L.p, L.ray.d, L.proj);
     if (k < 0) {
       L.mode = kNeedPrimary;
       return;
@@ -1281,6 +1282,16 @@ constexpr int kMeshWalkers = 8, kMeshLeaves = 8;
 // and 2 x 10^6 primaries over 262,144 lanes (ms): loop 0.75, 1.50, 3.57, 4.16
 // and 7.43, walk 1.27, 1.72, 3.12, 4.07 and 5.67.
 constexpr uint64_t kMeshLoopBelow = 4;
+// Solids up to which a photon that leaves a phantom looks for its next solid at
+// once, so that the successor of one that meets nothing more starts in the same
+// navigation pass.  The pass then searches the solids twice, for the leaving
+// photons and for the new ones, each time on a part of the lanes; with many
+// solids that costs more than the round it saves.  100^3 voxels before 1, 2, 4,
+// 8, 37 and 200 modules, 10^7 photons (ms): with it 5.08, 4.64, 4.97, 5.82, 10.5
+// and 49.4, without 5.17, 4.70, 4.92, 5.42, 8.25 and 34.7; with tau sampling
+// 4.46, 4.04, 4.36, 5.11, 9.61 and 44.7, without 4.68, 4.26, 4.53, 4.96, 7.88
+// and 31.5.
+constexpr int kAheadSolids = 5;
 // Steps of a round when the caller states none: short rounds while more than a
 // third of a full block's photons stop in one, long ones again below a quarter
 // and in blocks that run out of photons.  Photons that stop early wait for the
@@ -2362,6 +2373,7 @@ RunParams make_params(ggh_context* c) {
   P.round_steps = c->round_steps;
   P.cold_passes = c->cold_passes ? c->cold_passes : 1;
   P.xchg_offset = 0;
+  P.look_ahead = (int)c->solids.size() <= kAheadSolids;
   P.mesh_loop = 0;
   for (const DevSolid& s : c->solids)
     if (s.type == kVoxel) {
@@ -2642,6 +2654,8 @@ int acquisition_launch(ggh_context* c, RunParams& P, Launch& L) {
   P.acq_phantom = c->acq_phantom.p;
   P.n_proj = c->acq_n_proj;
   P.n_box = n_solids_of(c, kBoxSolid);
+  // a projection of one phantom sees that one and the modules
+  if (P.acq_phantom) P.look_ahead = P.n_box + 1 <= kAheadSolids;
   P.n_slots = c->acq_slots;
   if ((rc = pick_launch(c, c->acq_slots, c->acq_primaries, true, L))) return rc;
   P.xchg_offset = L.xchg_offset;
