@@ -2246,7 +2246,7 @@ hipError_t through_slots(ggh_context* c, int64_t items, size_t item_bytes, Fill 
 hipError_t words_out(ggh_context* c, const void* a, void* a_out, const void* b, void* b_out, int64_t n) {
   const void* src[2] = {a_out ? a : nullptr, b_out ? b : nullptr};
   char* out[2] = {static_cast<char*>(a_out), static_cast<char*>(b_out)};
-  if (!src[0] && !src[1]) return hipSuccess;
+  if (!src[0] && !src[1]) return hipStreamSynchronize(c->stream);  // the wait that every readback is
   return through_slots(
       c, n, 8,
       [&](char* slot, int64_t per, int64_t at, int64_t m) {
