@@ -2146,6 +2146,7 @@ struct ggh_context {
   // pinned slots of the readbacks (through_slots), kept
   char* slots = nullptr;
   hipEvent_t slot_ev[kCopiers] = {};
+  bool no_slots = false;  // ggh_debug_no_pinned
   std::mutex slots_mu;  // one readback at a time uses the slots
 };
 
@@ -2190,7 +2191,7 @@ hipError_t make_slots(ggh_context* c) {
 template <class Fill, class Take>
 hipError_t through_slots(ggh_context* c, int64_t items, size_t item_bytes, Fill fill, Take take) {
   std::lock_guard<std::mutex> lock(c->slots_mu);
-  if (make_slots(c) != hipSuccess) {
+  if (c->no_slots || make_slots(c) != hipSuccess) {
     // no pinned memory left: one small chunk at a time over device memory
     (void)hipGetLastError();
     const int64_t few = (int64_t)(kChunkBytes / item_bytes / 64 * 64);
@@ -3688,6 +3689,15 @@ int ggh_debug_primaries(ggh_context* c, int n, float* pos, float* dir, float* en
   HIP_TRY(hipMemcpyAsync(energy, de.p, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   dp.release(); dd.release(); de.release();
+  return 0;
+}
+
+int ggh_debug_no_pinned(ggh_context* c, int32_t on) {
+  int rc = check_ctx(c);
+  if (rc) return rc;
+  std::lock_guard<std::mutex> lock(c->slots_mu);
+  c->no_slots = on != 0;
+  if (c->no_slots) drop_slots(c);
   return 0;
 }
 

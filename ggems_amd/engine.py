@@ -119,6 +119,7 @@ def library():
             "ggh_host_distance_to_aabb": ([vp, vp, vp, vp, C.c_size_t], None),
             "ggh_host_voxel_exit": ([vp, vp, C.c_size_t, vp, vp, vp, vp, vp], C.c_int),
             "ggh_host_energy_bin": ([vp, C.c_size_t, vp, C.c_int32, vp], None),
+            "ggh_debug_no_pinned": ([vp, i32], C.c_int),
             "ggh_set_launch": ([vp, C.POINTER(LaunchDesc)], C.c_int),
             "ggh_get_launch": ([vp, C.POINTER(LaunchDesc)], C.c_int),
             "ggh_last_grid": ([vp, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)], C.c_int),
@@ -513,6 +514,10 @@ class Engine:
         d = LaunchDesc()
         _check(library().ggh_autotune(self.h, int(n_trial), C.byref(d)))
         return {k: int(getattr(d, k)) for k, _ in LaunchDesc._fields_}
+
+    def debug_no_pinned(self, on=True):
+        """readbacks as where no pinned host memory is to be had"""
+        _check(library().ggh_debug_no_pinned(self.h, int(on)))
 
     def debug_uniforms(self, n_slots, n):
         out = np.zeros((n_slots, n), np.float32)

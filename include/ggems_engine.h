@@ -378,6 +378,8 @@ int ggh_debug_mesh_hits(ggh_context* ctx, int solid, int n_rays, const float* po
 int ggh_debug_primaries(ggh_context* ctx, int n, float* pos, float* dir, float* energy);
 /* n draws from slot 0..n_slots-1 streams: out[s*n + k] */
 int ggh_debug_uniforms(ggh_context* ctx, int n_slots, int n, float* out);
+/* on != 0: readbacks go as they do where no pinned memory is to be had */
+int ggh_debug_no_pinned(ggh_context* ctx, int32_t on);
 /* -log(u) of the voxel step (fast[i]) and -logf(u) (ref[i]) on the device for RNG sums */
 int ggh_debug_neg_log(ggh_context* ctx, int n, const uint32_t* sums, float* fast, float* ref);
 /* host builds of the engine's arithmetic (exact-equivalence checks against the oracle) */
