@@ -1278,9 +1278,14 @@ constexpr int kWaves = kBlock / 64;
 constexpr int kMeshWalkers = 8, kMeshLeaves = 8;
 // Photons per lane below which a launch takes the track loop of each lane
 // instead: with few photons a lane there is little to even out, and the walk's
-// passes only add to each photon's time.  2 x 10^5, 7 x 10^5, 10^6, 1.5 x 10^6
-// and 2 x 10^6 primaries over 262,144 lanes (ms): loop 0.75, 1.50, 3.57, 4.16
-// and 7.43, walk 1.27, 1.72, 3.12, 4.07 and 5.67.
+// passes only add to each photon's time.  Where the two meet depends on the
+// scene: spheres of 81,920 and 5,120 triangles over 262,144 lanes, 4 x 10^5, 7 x
+// 10^5, 10^6, 1.3 x 10^6 and 2 x 10^6 primaries (ms): loop 1.67, 2.62, 3.61, 5.28
+// and 7.58, walk 1.81, 2.53, 3.19, 4.33 and 5.88, equal at 2.3 photons a lane;
+// spheres of 5,120 and 1,280 triangles: loop 1.15, 1.73, 2.41, 3.36 and 5.00, walk
+// 1.52, 2.04, 2.58, 3.46 and 4.73, equal at 5.5.  Five scenes lie between 2.3 and
+// 5.5; a line at 4 costs 15 % at most below it and 8 % above, one at 3 12 % on
+// either side.
 constexpr uint64_t kMeshLoopBelow = 4;
 // Solids up to which a photon that leaves a phantom looks for its next solid at
 // once, so that the successor of one that meets nothing more starts in the same
