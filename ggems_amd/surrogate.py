@@ -194,18 +194,23 @@ def _direct():
 
 
 F32W_CHANNELS = (8, 16, 32, 48, 64, 96, 128, 192)
-F32W_PIXELS = 524288
+F32W_PRODUCTS = 24 * 10 ** 7
 
 
 def _conv_layer(x, w, b, relu):
     """a layer's output without gradients, from its FP32 weights [cout][9][cin].
-    Up to F32W_PIXELS the kernel reads them as they are; for more, its many
-    blocks would each round them, and BF16 ones are made first (the network on
-    1, 8 and 16 views of 256 x 256: 232, 295 and 460 us from FP32, 399, 391 and
-    432 us from BF16)"""
+    Up to F32W_PRODUCTS of pixels, input and output channels the kernel reads
+    them as they are; for more, its many blocks would each round many of them,
+    and BF16 ones are made first, in a launch of 1.6 us.  Layers of 192 -> 64
+    channels on 4 and 8 views of 256 x 256 (2 and 4 x 10^8): 16.0 and 25.1 us
+    from FP32, 16.4 and 22.5 from BF16; 48 -> 16: 14.1 and 28.9, 15.5 and 27.7.
+    The network on 1, 4, 8, 12 and 16 views: 215, 219, 295, 381 and 493 us with
+    all from FP32, 365, 368, 377, 366 and 430 with none, 215, 219, 278, 355 and
+    434 by this rule (at 3 x 10^8 the last is 453, at 1.2 x 10^8 the second 254).
+    """
     cout, taps, cin = w.shape
     _on_device(x.device, weights=w, bias=b)
-    if (taps == 9 and cin in F32W_CHANNELS and x.numel() // cin <= F32W_PIXELS and w.dtype == torch.float32
+    if (taps == 9 and cin in F32W_CHANNELS and x.numel() * cout <= F32W_PRODUCTS and w.dtype == torch.float32
             and w.is_contiguous() and w.data_ptr() % 16 == 0 and x.dtype == torch.bfloat16 and x.is_cuda
             and x.shape[3] == cin
             and (b is None or (b.dtype == torch.float32 and b.is_contiguous() and b.shape == (cout,)))):
