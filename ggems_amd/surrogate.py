@@ -72,24 +72,25 @@ def _check(rc):
 
 def _stream(t):
     # the current stream's handle without a Stream object, which costs as much as a launch
-    index = t.device.index
-    if index is None:
+    index = t.get_device()
+    if index < 0:
         raise ValueError("expected a tensor on the GPU, not on %s" % t.device)
     return torch._C._cuda_getCurrentRawStream(index)
 
 
-def _on_device(device, **tensors):
-    """refuses tensors (or None) that a kernel on `device` could not read"""
-    for name, t in tensors.items():
-        if t is not None and t.device != device:
-            raise EngineError("%s is on %s, the input on %s" % (name, t.device, device))
+def _on_device(x, w, b):
+    """refuses weights and a bias (or None) that a kernel on x's device could not read"""
+    index = x.get_device()  # cheaper than comparing devices
+    if w.get_device() != index or (b is not None and b.get_device() != index):
+        raise EngineError("weights on %s, bias on %s, input on %s"
+                          % (w.device, None if b is None else b.device, x.device))
 
 
 def conv3x3(x, w, bias=None, relu=False):
     """x [N,H,W,Cin] BF16, w [Cout, 9*Cin] BF16, bias [Cout] FP32 -> [N,H,W,Cout] BF16"""
     if x.device.type != "cuda" or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise EngineError("conv3x3 takes BF16 tensors on the GPU")
-    _on_device(x.device, weights=w, bias=bias)
+    _on_device(x, w, bias)
     x, w = x.contiguous(), w.contiguous()
     n, h, wd, cin = x.shape
     cout = w.shape[0]
@@ -209,7 +210,7 @@ def _conv_layer(x, w, b, relu):
     434 by this rule (at 3 x 10^8 the last is 453, at 1.2 x 10^8 the second 254).
     """
     cout, taps, cin = w.shape
-    _on_device(x.device, weights=w, bias=b)
+    _on_device(x, w, b)
     if (taps == 9 and cin in F32W_CHANNELS and x.numel() * cout <= F32W_PRODUCTS and w.dtype == torch.float32
             and w.is_contiguous() and w.data_ptr() % 16 == 0 and x.dtype == torch.bfloat16 and x.is_cuda
             and x.shape[3] == cin
@@ -346,7 +347,7 @@ class _Head(torch.autograd.Function):
     @staticmethod
     def forward(ctx, z, head, bias):
         ctx.save_for_backward(z, head)
-        return head16(z, head, bias)
+        return _head16(z, head, bias)
 
     @staticmethod
     def backward(ctx, dout):
@@ -369,14 +370,17 @@ def _fits_head16(z, head, bias):
     a channel and one bias on z's device (other shapes broadcast)"""
     return (z.ndim == 4 and z.shape[3] == 16 and z.dtype == torch.bfloat16 and z.is_contiguous() and z.is_cuda
             and head.dtype == bias.dtype == torch.float32 and head.is_contiguous() and head.shape == (16,)
-            and bias.shape == (1,) and head.device == bias.device == z.device)
+            and bias.shape == (1,) and head.get_device() == bias.get_device() == z.get_device())
 
 
 def head16(z, head, bias):
     """sum over the 16 channels of z [N,H,W,16] BF16 times head [16], plus bias [1] -> [N,H,W] FP32"""
-    _on_device(z.device, head=head, bias=bias)
     if not _fits_head16(z, head, bias):
-        raise EngineError("the head takes BF16 z [N, H, W, 16] and FP32 head [16] and bias [1] on the GPU")
+        raise EngineError("the head takes BF16 z [N, H, W, 16] and FP32 head [16] and bias [1] on one GPU")
+    return _head16(z, head, bias)
+
+
+def _head16(z, head, bias):
     out = torch.empty(z.shape[:3], dtype=torch.float32, device=z.device)
     _check(_lib().ggh_unet_head(z.data_ptr(), head.data_ptr(), bias.data_ptr(), out.data_ptr(), out.numel(),
                                 _stream(z)))
@@ -428,7 +432,7 @@ class UNet(torch.nn.Module):
             z = b(a(upcat(z, s) if direct else _UpCat.apply(z, s)))
         head, bias = self.head, self.head_bias
         if _fits_head16(z, head, bias) and _untraced():
-            return head16(z, head, bias) if direct else _Head.apply(z, head, bias)
+            return _head16(z, head, bias) if direct else _Head.apply(z, head, bias)
         # the head as a multiply and a channel sum: a matrix-vector product
         # with 16 columns runs far below HBM speed in the BLAS path
         return (z.float() * head).sum(dim=3) + bias
