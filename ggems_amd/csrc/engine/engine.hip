@@ -554,7 +554,7 @@ __device__ inline int32_t after_step(const VoxGeom& G, const Lane& L, float cut)
 // the uniform's and the logarithm's rounding: over all 2^32 sums -log(u) is
 // at least 0.998 (1 - u) above 2^-19), and only a step that this cannot rule
 // out stops, with its sums kept, to take the logarithms and quotients in
-// resolve_interaction: three logarithms, three correctly rounded quotients
+// choose_process (stopped_step), before the regrouping: three logarithms, three correctly rounded quotients
 // and the second table read are gone from the step (about 170 of its 770
 // cycles of issue; the geometry gave another 200).  3*10^7 primaries through a
 // 256 x 256 x 128 body: 50.8 -> 46.6 ms with both.
@@ -1770,9 +1770,10 @@ __global__ __launch_bounds__(kDoseBlock) void dose_kernel(DoseParams D) {
 // share the chain.  A block holds 8 x 4 pixels, whose rays read the same
 // label bricks at a time.  What bounds it now is the FP64 issue of the walk.
 // A 512 x 384 panel behind 512 x 512 x 256 voxels: 800 us before, 229 us; a
-// 256 x 256 panel behind 96 x 96 x 64 voxels: 88 us before, 33 us, and the
-// spectrum table that a second kernel made for each such image (46 us) is now
-// made once, with the source.
+// 256 x 256 panel behind 96 x 96 x 64 voxels: 88 us before, 33 us (images of
+// several engines, each on its own stream, overlap: 23 to 25 us an image), and
+// the spectrum table that a second kernel made for each such image (46 us) is
+// now made once, with the source.
 constexpr int kDrrSegs = 8, kDrrTileX = 8, kDrrTileY = 4, kDrrTile = kDrrTileX * kDrrTileY;
 constexpr int kDrrBlock = kDrrSegs * kDrrTile;
 constexpr int kDrrBatch = 8;
@@ -2121,7 +2122,7 @@ struct ggh_context {
   // launch shape
   int round_steps = 0;  // 0: kShortRound or kLongRound, as the block's photons stop
   int cold_passes = 0;  // 0: 1 (two were 2-5 % slower with the reference sampling)
-  int interact_batch = 16;
+  int interact_batch = 16;  // as set, for ggh_get_launch and the autotuner's answer; no kernel reads it
   int blocks_per_cu = 0;  // 0: as many as fit
   bool force_general = false;
   int tau_mode = 0;  // voxel steps sample interactions by tau (one exponential per flight)

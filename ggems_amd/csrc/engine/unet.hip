@@ -7,11 +7,13 @@
 // Cout are multiples of 8 and 16 (the first layer pads its two input
 // channels); W is a multiple of 16 and N H W of 32.
 //
-// Two sets of kernels.  The channel counts of the U-Net with aligned tensors
-// take the tile kernels (conv_tile_kernel, conv_wgrad_tile_kernel): an input
-// tile with its halo goes to LDS once and serves all nine taps.  Everything
-// else takes the general ones, whose order of additions the tile kernels keep
-// in the forward pass and the data gradient:
+// Every kernel reads 8 channels of a tensor, or 8 weights, in one 16-byte load.
+// Two sets of kernels.  The channel counts of the U-Net take the tile kernels
+// (conv_tile_kernel, conv_wgrad_tile_kernel): an input tile with its halo goes
+// to LDS once and serves all nine taps.  Other counts, and in the forward pass
+// and the data gradient an output that is not 8-byte aligned (the tile kernel
+// stores four channels at a time), take the general ones, whose order of
+// additions the tile kernels keep there:
 //
 // Forward (implicit GEMM, M = pixels, N = Cout, K = 9 Cin): a wave owns
 // 32 consecutive pixels (two runs of 16 within image rows) and up to 64 output
@@ -426,7 +428,11 @@ template <int CIN, int NT, bool kSplit, bool kF32, bool kMask>
 void launch_tile_nt(const ConvArgs& A) {
   const unsigned tiles = (unsigned)(A.n * (A.wd / kTileW) * ((A.h + kTileH - 1) / kTileH));
   const unsigned ch_tiles = (unsigned)((A.cout + 16 * NT - 1) / (16 * NT));
-  // channel tiles in one block keep its input tile; a small image spreads them over blocks
+  // channel tiles in one block keep its input tile; a small image spreads them
+  // over blocks.  128 x 128 images, 32 -> 96 channels at 256, 768, 1,024 and 4,096
+  // tiles: 10.0, 14.3, 16.4 and 55.4 us in one block, 7.7, 15.3, 18.1 and 61.8
+  // spread; 64 -> 128: 15.8, 24.3, 34.2 and 107, spread 12.1, 24.8, 33.6 and 116;
+  // 128 -> 128: 22.8, 49.4, 56.2 and 204, spread 17.3, 49.0, 65.3 and 237.
   const unsigned gy = tiles >= 1024 ? 1 : ch_tiles;
   hipLaunchKernelGGL((conv_tile_kernel<CIN, NT, kSplit, kF32, kMask>), dim3((tiles + kXcds - 1) / kXcds * kXcds, gy),
                      dim3(64 * kWaves), (ConvTile<CIN, kSplit>::lds(NT)), A.st, A.x, A.w, A.bias, A.y, A.n, A.h, A.wd,
