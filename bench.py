@@ -9,7 +9,10 @@ Rayleigh, FP64 dose + uncertainty tallies.  Set up through the GGEMS API
 (ggems_amd.configs.voxel_ct), then timed on the engine with every input
 resident in HBM: one step is the workload's run of 1e9 primaries
 (--photons-per-step), one launch laid out in batches of 1,048,576 particle
-slots as GGEMS lays them out.
+slots as GGEMS lays them out.  Where the build found no GGEMS source tree, and
+so no physics data, the same scene runs on the closed-form cross sections,
+materials and spectrum of perf/cases.py, and "data" says so; there is no
+cpu_baseline then, since the oracle's tables come from the same data.
 
 Prints one JSON line (metric, value, roofline, cpu_baseline, ...).
 
@@ -106,6 +109,33 @@ def profile_record(sampling):
         return rec if ok else None
     except (OSError, ValueError, KeyError):
         return None
+
+
+def closed_form_scene():
+    """configs.voxel_ct's phantom, geometry and tallies on perf/cases.py's closed-form physics, as an engine"""
+    import math
+
+    import numpy as np
+
+    from ggems_amd import authoring
+    from ggems_amd.engine import Engine
+    sys.path.insert(0, os.path.join(REPO, "perf"))
+    import cases
+
+    shape, voxel = (256, 512, 512), 0.8
+    eng = Engine(0)
+    eng.set_physics(**cases.physics(cases.BODY + ["gos"]))
+    half = np.array(shape[::-1]) * voxel / 2
+    eng.add_voxel_solid(np.eye(4), -half, half, authoring.ellipsoid_body_phantom(20240, shape, voxel), (voxel,) * 3, 0)
+    eng.set_dosimetry(0, (voxel,) * 3, shape[::-1], -half, half, True, True)
+    panel = np.eye(4)
+    panel[:3, :3] = [[0, 0, 1], [0, 1, 0], [-1, 0, 0]]
+    panel[0, 3] = cases.SDD - cases.SID
+    size = np.array([256.0, 256.0, 1.0])
+    eng.add_box_solid(panel, -size / 2, size / 2, (256, 256, 1), size, 10e-3, len(cases.BODY), True)
+    aperture = math.atan(128 * math.sqrt(2.0) / cases.SDD)
+    eng.set_xray_source(cases.SOURCE_AT, aperture, (0.0, 0.0, 0.0), *cases.source_spectrum(True))
+    return eng
 
 
 def bench_mesh_ct(args):
@@ -339,6 +369,7 @@ def main():
     import torch
 
     from ggems_amd import configs
+    from ggems_amd.data.extract_physics_data import BLOB
     from ggems_amd.ggems import GGEMS
 
     if args.copy_calibration_mb:
@@ -348,10 +379,15 @@ def main():
         b.copy_(a)
         torch.cuda.synchronize()
         del a, b
-    keep = configs.voxel_ct(args.workdir, n_particles=args.photons_per_step, seed=20240, dosimetry=True)
-    g = GGEMS()
-    g.initialize(args.seed)
-    eng = g.engine()
+    g = keep = None
+    if os.path.exists(BLOB):
+        keep = configs.voxel_ct(args.workdir, n_particles=args.photons_per_step, seed=20240, dosimetry=True)
+        g = GGEMS()
+        g.initialize(args.seed)
+        eng = g.engine()
+    else:
+        eng = closed_form_scene()
+        eng.seed(args.seed)
     eng.set_launch(args.round_steps, args.interact_batch, args.blocks_per_cu, args.general_kernel,
                    args.cold_passes)
     eng.set_sampling(args.sampling)
@@ -408,7 +444,7 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f32",
-        "data": "synthetic",
+        "data": "synthetic" if g else "synthetic, on closed-form cross sections and materials",
         "config": {
             "workload": "voxel CT: 512x512x256 body phantom (0.8 mm, 5 materials, 40 seeded ellipsoids), "
                         "120 kVp Kramers + 2.5 mm Al point cone beam at SID 600 mm, flat 256x256 GOS detector "
@@ -447,10 +483,13 @@ def main():
             "frac": valu / VALU_PEAK_INSTR_PER_S,
             "instr_per_voxel_step": prof["valu_instr_per_step"],
         }
-    if not args.no_cpu_baseline:
+    if g and not args.no_cpu_baseline:
         out["cpu_baseline"] = cpu_baseline(args.workdir, args.photons_per_step, args.seed, args.cpu_seconds,
                                            args.cpu_threads)
-    g.delete()
+    if g:
+        g.delete()
+    else:
+        eng.close()
     del keep
     print(json.dumps(out), flush=True)
 
