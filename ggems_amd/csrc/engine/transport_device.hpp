@@ -223,16 +223,23 @@ __host__ __device__ inline bool in_aabb(f3 p, const Box& b) {
 }
 
 // Direction with its per-axis reciprocals (1.0f/d, the value the reference
-// recomputes on every call) cached until the direction changes.  An axis the
-// ray is parallel to (|d| < EPSILON6) has the reciprocal +inf: no general
-// test uses it, and exit_quick then never finds the exit there.
+// recomputes on every call) cached until the direction changes.  No general
+// test uses that of an axis the ray is parallel to (|d| < EPSILON6).
 struct Ray {
   f3 d, inv;
   __host__ __device__ inline void set(f3 dir) {
     d = dir;
-    inv.x = fabsf(dir.x) < kEps6 ? __builtin_inff() : 1.0f / dir.x;
-    inv.y = fabsf(dir.y) < kEps6 ? __builtin_inff() : 1.0f / dir.y;
-    inv.z = fabsf(dir.z) < kEps6 ? __builtin_inff() : 1.0f / dir.z;
+    inv.x = 1.0f / dir.x;
+    inv.y = 1.0f / dir.y;
+    inv.z = 1.0f / dir.z;
+  }
+  // for exit_quick too, which with +inf there never finds the exit on a
+  // parallel axis
+  __host__ __device__ inline void set_quick(f3 dir) {
+    set(dir);
+    inv.x = fabsf(dir.x) < kEps6 ? __builtin_inff() : inv.x;
+    inv.y = fabsf(dir.y) < kEps6 ? __builtin_inff() : inv.y;
+    inv.z = fabsf(dir.z) < kEps6 ? __builtin_inff() : inv.z;
   }
 };
 
