@@ -33,6 +33,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <string>
 
@@ -829,22 +830,34 @@ struct WgradArgs {
   hipStream_t st;
 };
 
+int wgrad_tiles(const WgradArgs& A) { return A.n * (A.wd / kTileW) * ((A.h + kTileH - 1) / kTileH); }
+
+// work: the blocks' sums go to a work space
 template <int MT, int CIT, bool kC8>
-int wgrad_splits(const WgradArgs& A, int* groups) {
-  const int tiles = A.n * (A.wd / kTileW) * ((A.h + kTileH - 1) / kTileH);
+int wgrad_splits(const WgradArgs& A, bool work, int* groups) {
+  const int tiles = wgrad_tiles(A);
   *groups = (A.cout / (16 * MT)) * (kC8 ? 1 : A.cin / (16 * CIT));
   // each block walks its share of the tiles.  Two blocks of the large variants
   // fit a compute unit; one with 9 sums or fewer leaves room for four (512 and
   // 1,024 blocks: 25.2 and 22.9 us at 16 x 256 x 256, 16 -> 16, but 20 and 30 us
   // at 128 x 128, 32 -> 32)
-  return std::max(1, std::min(tiles, (MT * WgTile<MT, CIT, kC8>::kCols <= 9 ? 1024 : 512) / *groups));
+  int blocks = MT * WgTile<MT, CIT, kC8>::kCols <= 9 ? 1024 : 512;
+  // Blocks that add to dw themselves: each adds its group's weights once, at the
+  // addresses of every other block of the group, so their number weighs against
+  // the tiles a block walks.  The best of 32 to 1,024 blocks over 19 layer shapes
+  // at batch 1, 4 and 16 grows with the root of the tiles, and less than the
+  // groups do (128 x 128, 32 -> 32 channels, batch 4: 18.6 us, 37 with 512 blocks;
+  // 64 x 64, 64 -> 16, batch 16: 21 and 44; 256 x 256, 16 -> 16, batch 16: 29 and
+  // 42 with 1,024).
+  if (!work) blocks = std::min(blocks, (int)(4.5f * std::sqrt((float)tiles) * std::pow((float)*groups, 2.0f / 3.0f)));
+  return std::max(1, std::min(tiles, blocks / *groups));
 }
 
 // launches the kernels; with `floats`, only says how much `part` must hold
 template <int MT, int CIT, bool kC8>
 void launch_wgrad_tile(const WgradArgs& A, size_t* floats) {
   int groups;
-  const int splits = wgrad_splits<MT, CIT, kC8>(A, &groups);
+  const int splits = wgrad_splits<MT, CIT, kC8>(A, A.part || floats, &groups);
   using T = WgTile<MT, CIT, kC8>;
   if (floats) {
     *floats = (size_t)groups * splits * T::kPart;
@@ -1253,7 +1266,13 @@ int ggh_conv3x3_weight_grad(const void* x, const void* dy, float* dw, int32_t n,
   if (!x || !dy || !dw) return ufail(-1, "null pointer");
   if (!shapes_ok(n, h, wd, cin, cout) || cout > kWgMaxM) return ufail(-2, "unsupported shape (Cout <= 128)");
   const __bf16 *xb = static_cast<const __bf16*>(x), *db = static_cast<const __bf16*>(dy);
-  if (wgrad_tile({xb, db, dw, n, h, wd, cin, cout, nullptr, nullptr, nullptr, static_cast<hipStream_t>(stream)})) {
+  const WgradArgs args = {xb, db, dw, n, h, wd, cin, cout, nullptr, nullptr, nullptr, static_cast<hipStream_t>(stream)};
+  // few tiles and few output channels: the tile kernel's additions to dw take
+  // longer than the general kernel's repeated loads (64 x 64, 64 -> 16, batch 1
+  // and 4: 10.8 and 14.5 us against 6.5 and 10.3; 128 x 128, 96 -> 32: 15.5 against
+  // 13.9; from 64 channels on the tile kernel is the faster one at any size)
+  const bool few = cout < 64 && wgrad_tiles(args) <= 128;
+  if (!few && wgrad_tile(args)) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return ufail(-100 - (int)e, std::string("conv weight gradient: ") + hipGetErrorString(e));
     return 0;
