@@ -182,7 +182,6 @@ struct RunParams {
   int32_t cold_passes;        // navigation passes per round
   uint32_t xchg_offset;       // byte offset of the lane-state exchange area in dynamic LDS
   int look_ahead;             // a leaving photon looks for its next solid at once (kAheadSolids)
-  int mesh_loop;              // kernels without regrouping: each lane walks its mesh to the end (pick_launch)
   VoxGeom vox0;               // the only voxel solid, when there is exactly one
   // CT acquisition: projection p places the source at acq_src[p] and box
   // solid j at acq_box[p * n_box + j]; its primaries are laid out in
@@ -890,8 +889,8 @@ __device__ inline int mesh_hits(const DevSolid& s, f3 p, f3 d, f3& q0, f3& q1) {
 // One step with the ray's n hits, q0 and q1 the nearest.  False when the
 // photon is done with the solid: no surface ahead, or it died (alive).
 __device__ inline bool mesh_step(const RunParams& P, const Tabs& T, const DevSolid& s, int n, f3 q0, f3 q1, f3& lp,
-                                 f3& ld, Lane& L, bool& alive, unsigned long long& steps,
-                                 unsigned long long& inter) {
+                                 f3& ld, Lane& L, bool& alive, uint32_t& steps,
+                                 uint32_t& inter) {
   if (n == 0) return false;
   const int gmat = s.mat_offset;
   const bool dose = L.solid == P.dose_solid;
@@ -949,15 +948,15 @@ __device__ inline void leave_mesh(const DevSolid& s, f3 lp, f3 ld, bool alive, L
 __device__ void track_mesh(const RunParams& P, const Tabs& T, const DevSolid& s, Lane& L) {
   f3 lp = L.p, ld = L.ray.d;
   bool alive = true;
-  unsigned long long steps = 0, inter = 0;
+  uint32_t steps = 0, inter = 0;
   for (;;) {
     f3 q0 = lp, q1 = lp;
     const int n = mesh_hits(s, lp, ld, q0, q1);
     if (!mesh_step(P, T, s, n, q0, q1, lp, ld, L, alive, steps, inter)) break;
   }
   leave_mesh(s, lp, ld, alive, L);
-  atomicAdd(&P.stats[6], steps);
-  atomicAdd(&P.stats[7], inter);
+  atomicAdd(&P.stats[6], (unsigned long long)steps);
+  atomicAdd(&P.stats[7], (unsigned long long)inter);
 }
 
 // ---------------------------------------------------------------------------
@@ -1157,7 +1156,7 @@ __device__ inline void next_projection(const RunParams& P, Lane& L) {
 
 // the cold work of one lane, one state at a time in an order that lets a
 // lane pass through several states in one call
-template <int NP, bool kSingle, bool kAcq, bool kTau, bool kTrack, bool kThin, bool kRegroup, class Counters>
+template <int NP, bool kSingle, bool kAcq, bool kTau, bool kTrack, bool kThin, bool kRegroup, bool kLoop, class Counters>
 __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Counters& c) {
   constexpr bool kBoxes = kSingle && !kRegroup;  // no photon is ever inside a phantom
   if (!kBoxes && L.mode == kInteract)
@@ -1252,7 +1251,7 @@ __device__ inline void cold_step(const RunParams& P, const Tabs& T, Lane& L, Cou
       // ggh_run launches the single-voxel-solid variant only on scenes
       // without meshes, which keeps the mesh loop (and even this test) out
       // of its register allocation
-      if (kRegroup || P.mesh_loop) track_mesh(P, T, s, L);
+      if (kRegroup || kLoop) track_mesh(P, T, s, L);
       else L.mode = kInMesh;
     } else {
       track_box<kAcq>(P, T, s, L, c);
@@ -1288,6 +1287,18 @@ constexpr int kMeshWalkers = 8, kMeshLeaves = 8;
 // 5.5; a line at 4 costs 15 % at most below it and 8 % above, one at 3 12 % on
 // either side.
 constexpr uint64_t kMeshLoopBelow = 4;
+// And the share of the source's rays that meet a mesh below which it does so
+// too: where few photons enter one, the lanes that do wait for kMeshWalkers of
+// their wave, and the walk's passes and registers weigh on all the others.
+// Spheres of 1,280 triangles in a beam of 60 mm at their place, 2 x 10^7 photons,
+// radius 2, 4, 8 and 12 mm (0.14, 0.6, 2.3 and 5 % of the rays; ms): loop 2.1,
+// 3.0, 6.8 and 8.8, walk 2.9, 3.7, 4.7 and 5.3.
+constexpr double kMeshShare = 0.01;
+// Primaries beyond which a launch takes the loop, which counts its steps in 64
+// bits: in the walk's registers 64-bit counts cost spills (81,920 and 5,120
+// triangles, 10^7 photons: 26.15 ms for 25.74), and a lane's share of 2^40
+// primaries, 2^22 with 2^18 lanes, fills 32 bits only at 1,024 steps for each.
+constexpr uint64_t kWalkMost = 1ull << 40;
 // Solids up to which a photon that leaves a phantom looks for its next solid at
 // once, so that the successor of one that meets nothing more starts in the same
 // navigation pass.  The pass then searches the solids twice, for the leaving
@@ -1310,6 +1321,16 @@ constexpr int kAheadSolids = 5;
 // 172.4 and 0.44 (switching to 10 steps, or at a quarter and a sixth: 35.2,
 // 23.9).
 constexpr int kShortRound = 8, kLongRound = 20;
+
+// a wave's sum of 32-bit counts, in 32-bit halves
+__device__ inline unsigned long long wave_sum(uint32_t v) {
+  uint32_t lo = v & 0xffffu, hi = v >> 16;
+  for (int off = 32; off > 0; off >>= 1) {
+    lo += __shfl_xor(lo, off, 64);
+    hi += __shfl_xor(hi, off, 64);
+  }
+  return ((unsigned long long)hi << 16) + lo;
+}
 
 constexpr size_t kXchgBytes = (size_t)kBlock * 12 * sizeof(uint32_t);
 
@@ -1378,8 +1399,10 @@ __device__ inline uint32_t lds_load_relaxed(uint32_t* p) {
 // work in rounds with regrouping (below).  Without a voxel solid every
 // photon is navigated and tracked by its lane's state machine alone.
 // kThin: a voxel solid is outside what quick_grid allows, and every step takes
-// the general geometry.
-template <int NP, bool kSingle, bool kLDS, bool kTrack, bool kAcq, bool kRegroup, bool kTau = false, bool kThin = false>
+// the general geometry; kLoop: a meshed scene without a voxel solid whose lanes
+// track their photons through a mesh to the end (kMeshLoopBelow, kMeshShare).
+template <int NP, bool kSingle, bool kLDS, bool kTrack, bool kAcq, bool kRegroup, bool kTau = false, bool kThin = false,
+          bool kLoop = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWavesPerEU)))
 void transport_kernel(RunParams P) {
   extern __shared__ float4 s_tab[];
@@ -1442,20 +1465,21 @@ void transport_kernel(RunParams P) {
   else for (int k = 0; k < kNumCounters; ++k) c.v[k] = 0u;
   unsigned long long steps = 0;  // wave-uniform
 
-  if (!kRegroup && kSingle) {
-    // Boxes only: navigation and tracking by each lane's state machine alone.
+  if (!kRegroup && (kSingle || kLoop)) {
+    // Boxes only, or the track loop: each lane's state machine alone.
     // With the walk of meshed scenes in the same kernel, an open field of 4 x
     // 10^6 and 4 x 10^7 photons on one panel took 0.715 and 3.52 ms, on 37
     // modules 1.02 and 8.07; 0.68 and 3.18, 0.98 and 7.81 without it (and with
     // the plain reciprocals of Ray::set in find_and_project).
     while (__any(L.mode != kDone))
-      if (L.mode != kDone) cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin, kRegroup>(cold_params(), T, L, c);
+      if (L.mode != kDone)
+        cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin, kRegroup, kLoop>(cold_params(), T, L, c);
   } else if (!kRegroup) {
     // No voxel solid, so no lane steps voxels; a lane inside a meshed solid
     // looks for its surfaces in the BVH.  Photons take different numbers of
     // mesh steps, and rays meet different numbers of nodes: run to its end by
-    // each lane in turn (track_mesh, which launches of few photons a lane still
-    // take: P.mesh_loop), a wave's track loop kept most lanes waiting for the
+    // each lane in turn (track_mesh, which some launches still take: kLoop), a
+    // wave's track loop kept most lanes waiting for the
     // slowest.  Here every lane holds its own place in the tree, the wave
     // visits nodes while at least kMeshWalkers of its lanes are looking, and
     // then makes the steps and the navigation of all the others.  The loop
@@ -1463,7 +1487,7 @@ void transport_kernel(RunParams P) {
     // moves on in each pass.
     MeshWalk w = {0, 0, 0, 0.0f, 0.0f, L.p, L.p};
     bool looking = false;
-    unsigned long long mesh_steps = 0, mesh_inter = 0;
+    uint32_t mesh_steps = 0, mesh_inter = 0;  // of this lane (kWalkMost)
     for (;;) {
       for (;;) {
         const uint64_t walkers = __ballot(looking);
@@ -1500,7 +1524,7 @@ void transport_kernel(RunParams P) {
       }
       const bool cold = L.mode != kInMesh && L.mode != kDone;
       if (cold) {
-        cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin, kRegroup>(Q, T, L, c);
+        cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin, kRegroup, kLoop>(Q, T, L, c);
         fresh = L.mode == kInMesh;
       }
       if (fresh) {  // a new look: from the root, with no hits
@@ -1510,13 +1534,10 @@ void transport_kernel(RunParams P) {
       }
       if (!__any(L.mode != kDone)) break;
     }
-    for (int off = 32; off > 0; off >>= 1) {
-      mesh_steps += __shfl_xor(mesh_steps, off, 64);
-      mesh_inter += __shfl_xor(mesh_inter, off, 64);
-    }
-    if (__lane_id() == 0 && mesh_steps) {
-      atomicAdd(&P.stats[6], mesh_steps);
-      atomicAdd(&P.stats[7], mesh_inter);
+    const unsigned long long all_steps = wave_sum(mesh_steps), all_inter = wave_sum(mesh_inter);
+    if (__lane_id() == 0 && all_steps) {
+      atomicAdd(&P.stats[6], all_steps);
+      atomicAdd(&P.stats[7], all_inter);
     }
   } else {
     // The block works in rounds.  In each round every wave
@@ -1566,7 +1587,7 @@ void transport_kernel(RunParams P) {
         // the block's round lasts until these passes are done: they issue first
         // (256 x 256 x 128 body: 41.3 ms without, 39.5 with)
         __builtin_amdgcn_s_setprio(3);
-        if (cold) cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin, kRegroup>(cold_params(), T, L, c);
+        if (cold) cold_step<NP, kSingle, kAcq, kTau, kTrack, kThin, kRegroup, kLoop>(cold_params(), T, L, c);
       }
       __builtin_amdgcn_s_setprio(0);
       // The reference step draws its random numbers while its label is on the
@@ -2392,7 +2413,6 @@ RunParams make_params(ggh_context* c) {
   P.cold_passes = c->cold_passes ? c->cold_passes : 1;
   P.xchg_offset = 0;
   P.look_ahead = (int)c->solids.size() <= kAheadSolids;
-  P.mesh_loop = 0;
   for (const DevSolid& s : c->solids)
     if (s.type == kVoxel) {
       P.vox0 = s.vox;
@@ -2565,8 +2585,62 @@ struct Launch {
   unsigned grid;
   size_t shmem;
   uint32_t xchg_offset;  // RunParams::xchg_offset of this launch
-  int mesh_loop;         // RunParams::mesh_loop of this launch
 };
+
+// Share of the source's rays that meet the box of a meshed solid: a spiral of
+// directions over the cone, from up to eight of an acquisition's placements.
+double mesh_share(const ggh_context* c, bool acq) {
+  constexpr int kRays = 1024, kPlaces = 8;
+  const int places = acq ? std::min(c->acq_n_proj, kPlaces) : 1, rays = kRays / places;
+  int hits = 0;
+  for (int k = 0; k < places; ++k) {
+    const size_t at = acq ? (size_t)k * c->acq_n_proj / places : 0;
+    const Mat34& m = acq ? c->acq_src_host[at] : c->src_m;
+    const int only = acq && !c->acq_phantom_host.empty() ? c->acq_phantom_host[at] : -1;
+    // the beam's axis points from the source to the origin (sample_primary)
+    const double o[3] = {m.m[3], m.m[7], m.m[11]};
+    const double r = std::sqrt(o[0] * o[0] + o[1] * o[1] + o[2] * o[2]);
+    if (!(r > 0.0)) return 1.0;
+    const double w[3] = {-o[0] / r, -o[1] / r, -o[2] / r};
+    const double s = w[2] < 0.0 ? -1.0 : 1.0, a = -1.0 / (s + w[2]), b = w[0] * w[1] * a;
+    const double u[3] = {1.0 + s * w[0] * w[0] * a, s * b, -s * w[0]}, v[3] = {b, s + w[1] * w[1] * a, -w[1]};
+    for (int i = 0; i < rays; ++i) {
+      const double ct = 1.0 - (i + 0.5) / rays * (1.0 - std::cos((double)c->aperture));
+      const double st = std::sqrt(std::max(0.0, 1.0 - ct * ct)), phi = 2.399963229728653 * i;  // the golden angle
+      const double p = st * std::cos(phi), q = st * std::sin(phi);
+      bool hit = false;
+      for (size_t j = 0; j < c->solids.size() && !hit; ++j) {
+        const DevSolid& g = c->solids[j];
+        if (g.type != kMesh || (only >= 0 && (int)j != only)) continue;
+        double t0 = 0.0, t1 = INFINITY;
+        const float lo[3] = {g.border.lo.x, g.border.lo.y, g.border.lo.z};
+        const float hi[3] = {g.border.hi.x, g.border.hi.y, g.border.hi.z};
+        for (int e = 0; e < 3; ++e) {  // axis e of the solid's frame: column e of its matrix
+          double pos = 0.0, dir = 0.0;
+          for (int x = 0; x < 3; ++x) {
+            pos += g.m.m[4 * x + e] * (o[x] - g.m.m[4 * x + 3]);
+            dir += g.m.m[4 * x + e] * (ct * w[x] + p * u[x] + q * v[x]);
+          }
+          const double ta = (lo[e] - pos) / dir, tb = (hi[e] - pos) / dir;
+          t0 = std::max(t0, std::min(ta, tb));
+          t1 = std::min(t1, std::max(ta, tb));
+        }
+        hit = t0 < t1;
+      }
+      hits += hit;
+    }
+  }
+  return (double)hits / (rays * places);
+}
+
+// whether the lanes of a meshed scene without a voxel solid track their photons
+// one by one
+bool mesh_loop(const ggh_context* c, uint64_t primaries, bool acq) {
+  // two blocks fit a compute unit
+  const uint64_t blocks = c->blocks_per_cu > 0 ? std::min(c->blocks_per_cu, 2) : 2;
+  return primaries < kMeshLoopBelow * blocks * c->n_cu * kBlock || primaries > kWalkMost ||
+         mesh_share(c, acq) < kMeshShare;
+}
 
 // The instantiation of a scene with a voxel solid.  special: three activated
 // processes over one voxel solid and no mesh, tables in LDS, no fluence
@@ -2628,6 +2702,11 @@ int pick_launch(ggh_context* c, uint64_t slots, uint64_t primaries, bool acq, La
   if (regroup)
     L.fn = thin ? voxel_kernel<true>(special, three, use_lds, acq, tau)
                 : voxel_kernel<false>(special, three, use_lds, acq, tau);
+  else if (n_solids_of(c, kMesh) > 0 && mesh_loop(c, primaries, acq))
+    L.fn = acq ? (use_lds ? transport_kernel<-1, false, true, true, true, false, false, false, true>
+                          : transport_kernel<-1, false, false, true, true, false, false, false, true>)
+               : (use_lds ? transport_kernel<-1, false, true, true, false, false, false, false, true>
+                          : transport_kernel<-1, false, false, true, false, false, false, false, true>);
   else if (n_solids_of(c, kMesh) > 0)
     L.fn = acq ? (use_lds ? transport_kernel<-1, false, true, true, true, false>
                           : transport_kernel<-1, false, false, true, true, false>)
@@ -2644,7 +2723,6 @@ int pick_launch(ggh_context* c, uint64_t slots, uint64_t primaries, bool acq, La
                                                        L.shmem));
   if (per_cu < 1) return fail(-3, "transport kernel does not fit on a compute unit");
   if (c->blocks_per_cu > 0) per_cu = std::min(per_cu, c->blocks_per_cu);
-  L.mesh_loop = primaries < kMeshLoopBelow * (uint64_t)per_cu * c->n_cu * kBlock;
   // persistent blocks: no more than the slots can keep busy
   const uint64_t max_blocks = (slots + kBlock - 1) / kBlock;
   L.grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)per_cu * c->n_cu, max_blocks));
@@ -2683,7 +2761,6 @@ int acquisition_launch(ggh_context* c, RunParams& P, Launch& L) {
   P.n_slots = c->acq_slots;
   if ((rc = pick_launch(c, c->acq_slots, c->acq_primaries, true, L))) return rc;
   P.xchg_offset = L.xchg_offset;
-  P.mesh_loop = L.mesh_loop;
   return 0;
 }
 
@@ -3269,7 +3346,6 @@ int ggh_run(ggh_context* c, uint64_t n) {
   Launch L;
   if ((rc = pick_launch(c, slots, n, false, L))) return rc;
   P.xchg_offset = L.xchg_offset;
-  P.mesh_loop = L.mesh_loop;
   HIP_TRY(hipMemsetAsync(c->queue.p, 0, sizeof(uint32_t), c->stream));
   HIP_TRY(hipEventRecord(c->ev0, c->stream));
   hipLaunchKernelGGL(L.fn, dim3(L.grid), dim3(kBlock), L.shmem, c->stream, P);
